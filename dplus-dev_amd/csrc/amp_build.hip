@@ -6,7 +6,9 @@
 // which is PDBAmplitude::calcAmplitude (Backend/Backend/PDBAmplitude.cpp:243-317)
 // evaluated on the grid (Backend/Backend/Grid.cpp:760-826), the work the
 // reference GPU path splits over CombinedPDBandDummyAtomJacobForSingleIonKernel
-// and CalcPDBVoxelSolventKernelJacobSphr (PDBAmplitudeCUDA.cu:15-186).
+// and CalcPDBVoxelSolventKernelJacobSphr (PDBAmplitudeCUDA.cu:15-186).  These kernels sum
+// every source at every node, for small builds; larger ones go through a frequency mesh
+// (amp_mesh.hip, mesh_pays).
 //
 // Design (MI355X):
 //  * Friedel symmetry: for real form factors A(-q) = conj(A(q)); every shell is

@@ -379,6 +379,164 @@ void form_factor_table(const dplus_pdb_desc *d, const std::vector<int> &counts, 
     }
 }
 
+namespace {
+struct BoxSet {
+    int n;
+    const int *dims;
+    const double *com;
+    double contrast;
+};
+
+// Host side of MeshSources: the cell grid over every atom and box piece (cells of
+// 0.4 nm, larger where more than kMeshCells of them would be needed along an axis),
+// the atoms' order by (ion, cell) and the box pieces by cell.
+struct MeshHost {
+    bool ok = false;
+    double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, cell0[3] = {0, 0, 0}, cell_inv = 0.0, half[3] = {0, 0, 0};
+    int ncell[3] = {1, 1, 1}, cells = 1;
+    std::vector<double4> pieces, lens;
+    long long npieces = 0;
+    std::vector<int> fion, start;
+
+    int cell(const double *p) const {
+        int c[3];
+        for (int a = 0; a < 3; a++)
+            c[a] = std::min(ncell[a] - 1, std::max(0, (int)((p[a] - cell0[a]) * cell_inv)));
+        return (c[0] * ncell[1] + c[1]) * ncell[2] + c[2];
+    }
+
+    // measure: extents, classes and the number of pieces alone
+    MeshHost(const dplus_pdb_desc *d, bool atoms_on, const BoxSet *sets, bool measure = false) {
+        double c_lo[3], c_hi[3];  // of the centres
+        for (int a = 0; a < 3; a++) {
+            c_lo[a] = 1e300;
+            c_hi[a] = -1e300;
+        }
+        auto see = [&](const double *p) {
+            for (int a = 0; a < 3; a++) {
+                c_lo[a] = std::min(c_lo[a], p[a]);
+                c_hi[a] = std::max(c_hi[a], p[a]);
+            }
+            return std::isfinite(p[0]) && std::isfinite(p[1]) && std::isfinite(p[2]);
+        };
+        if (atoms_on)
+            for (int a = 0; a < d->natoms; a++)
+                if (!see(d->xyz + 3 * a)) return;
+        size_t boxes = 0;
+        for (int si = 0; si < 2; si++) boxes += sets[si].n;
+        const size_t most = 4 * boxes + (1u << 20);
+        for (int si = 0; si < 2; si++)
+            for (int b = 0; b < sets[si].n; b++) {
+                const int *n = sets[si].dims + 3 * b;
+                const double *com = sets[si].com + 3 * b;
+                if (n[0] < 0 || n[1] < 0 || n[2] < 0) return;
+                if (n[0] == 0 || n[1] == 0 || n[2] == 0) continue;  // no volume
+                double cut[3], k = 1.0, len[3];
+                for (int a = 0; a < 3; a++) {
+                    len[a] = n[a] * d->vox_step;
+                    cut[a] = std::max(1.0, std::ceil(len[a] / kMeshPiece - 1e-9));
+                    k *= cut[a];
+                }
+                if (!(k + (double)npieces <= (double)most)) return;
+                npieces += (long long)k;
+                for (int a = 0; a < 3; a++) {
+                    len[a] /= cut[a];
+                    half[a] = std::max(half[a], 0.5 * len[a]);
+                }
+                for (int x = 0; x < (int)cut[0]; x++)
+                    for (int y = 0; y < (int)cut[1]; y++)
+                        for (int z = 0; z < (int)cut[2]; z++) {
+                            const double p[3] = {com[0] + (x - 0.5 * (cut[0] - 1.0)) * len[0],
+                                                 com[1] + (y - 0.5 * (cut[1] - 1.0)) * len[1],
+                                                 com[2] + (z - 0.5 * (cut[2] - 1.0)) * len[2]};
+                            if (!see(p)) return;
+                            if (measure) continue;
+                            pieces.push_back(make_double4(p[0], p[1], p[2], sets[si].contrast));
+                            lens.push_back(make_double4(len[0], len[1], len[2], 0.0));
+                        }
+            }
+        if (!(atoms_on && d->natoms > 0) && npieces == 0) return;
+        double size = 0.4;
+        for (int a = 0; a < 3; a++) size = std::max(size, (c_hi[a] - c_lo[a]) / kMeshCells * (1.0 + 1e-9));
+        if (!std::isfinite(size)) return;
+        cell_inv = 1.0 / size;
+        for (int a = 0; a < 3; a++) {
+            cell0[a] = c_lo[a];
+            ncell[a] = std::min(kMeshCells, (int)((c_hi[a] - c_lo[a]) * cell_inv) + 1);
+            lo[a] = c_lo[a] - half[a];
+            hi[a] = c_hi[a] + half[a];
+        }
+        cells = ncell[0] * ncell[1] * ncell[2];
+        if (atoms_on) {
+            std::vector<char> used(d->nion, 0);
+            for (int a = 0; a < d->natoms; a++) {
+                if (d->ion[a] < 0 || d->ion[a] >= d->nion) return;
+                used[d->ion[a]] = 1;
+            }
+            for (int i = 0; i < d->nion; i++)
+                if (used[i]) fion.push_back(i);
+        }
+        if (npieces > 0) fion.push_back(-1);
+        ok = true;
+        if (measure) return;
+        start.assign(fion.size() * (cells + 1), 0);
+        if (!pieces.empty()) {
+            int *st = &start[(fion.size() - 1) * (cells + 1)];
+            std::vector<int> key(pieces.size());
+            for (size_t i = 0; i < pieces.size(); i++) st[(key[i] = cell(&pieces[i].x)) + 1]++;
+            for (int c = 0; c < cells; c++) st[c + 1] += st[c];
+            std::vector<int> at(st, st + cells);
+            std::vector<double4> p2(pieces.size()), l2(pieces.size());
+            for (size_t i = 0; i < pieces.size(); i++) {
+                const int k = at[key[i]]++;
+                p2[k] = pieces[i];
+                l2[k] = lens[i];
+            }
+            pieces.swap(p2);
+            lens.swap(l2);
+        }
+    }
+
+    MeshSources sources(long long natoms) const {
+        MeshSources m;
+        m.ok = ok;
+        m.nfield = (int)fion.size();
+        m.natoms = natoms;
+        m.npieces = npieces;
+        for (int a = 0; a < 3; a++) {
+            m.lo[a] = lo[a];
+            m.hi[a] = hi[a];
+            m.cell0[a] = cell0[a];
+            m.ncell[a] = ncell[a];
+            m.piece_half[a] = half[a];
+        }
+        m.cell_inv = cell_inv;
+        return m;
+    }
+
+    // order: atoms by (ion, cell), stable; start: every used ion's cells
+    void sort_atoms(const dplus_pdb_desc *d, std::vector<int> &order) {
+        std::vector<int> field(d->nion, 0), key(d->natoms);
+        for (size_t f = 0; f < fion.size(); f++)
+            if (fion[f] >= 0) field[fion[f]] = (int)f;
+        const int n = cells + 1;
+        for (int a = 0; a < d->natoms; a++) {
+            key[a] = field[d->ion[a]] * n + cell(d->xyz + 3 * a);
+            start[key[a] + 1]++;
+        }
+        int sum = 0;
+        for (size_t f = 0; f < fion.size() && fion[f] >= 0; f++) {
+            int *st = &start[f * n];
+            st[0] = sum;
+            for (int c = 0; c < cells; c++) st[c + 1] += st[c];
+            sum = st[cells];
+        }
+        std::vector<int> at(start);
+        for (int a = 0; a < d->natoms; a++) order[at[key[a]]++] = a;
+    }
+};
+}  // namespace
+
 Structure::Structure(const dplus_pdb_desc *d, hipStream_t s) {
     if (d->natoms < 0 || d->nion <= 0 || d->nion > 255) throw Error(kErrInvalidArgs, "bad atom/ion counts");
     if (d->nbox < 0 || (d->nbox > 0 && (!d->box_dims || !d->box_com || !(d->vox_step > 0))))
@@ -390,24 +548,22 @@ Structure::Structure(const dplus_pdb_desc *d, hipStream_t s) {
     const bool atoms_on = (d->flags & (DPLUS_CALC_ATOMIC_FORMFACTORS | DPLUS_CALC_DUMMY_SOLVENT)) && d->natoms > 0;
     // box sets: the outer-solvent (hydration) layer added with box_contrast and the
     // excluded volume added with excl_contrast (PDBAmplitude.cpp:277-314)
-    struct BoxSet {
-        int n;
-        const int *dims;
-        const double *com;
-        double contrast;
-    };
     const BoxSet sets[2] = {{d->box_contrast != 0.0 ? d->nbox : 0, d->box_dims, d->box_com, d->box_contrast},
                             {d->excl_contrast != 0.0 ? d->nexcl : 0, d->excl_dims, d->excl_com, d->excl_contrast}};
     const bool boxes_on = sets[0].n > 0 || sets[1].n > 0;
     // atoms sorted by ion (ExtractRelevantCoeffs, PDBReaderLib.cpp:1443-1509), stably:
     // a counting sort over the ion index; then each box set sorted by shape
     // (SortSolventBoxEntry, PDBAmplitude.cpp:161-188)
+    // and, within an ion, by cell of the mesh builder
+    MeshHost mh(d, atoms_on, sets);
     std::vector<int> order(d->natoms);
-    {
+    if (!atoms_on || !mh.ok) {
         std::vector<int> start(d->nion + 1, 0);
         for (int a = 0; a < d->natoms; a++) start[d->ion[a] + 1]++;
         for (int i = 0; i < d->nion; i++) start[i + 1] += start[i];
         for (int a = 0; a < d->natoms; a++) order[start[d->ion[a]]++] = a;
+    } else {
+        mh.sort_atoms(d, order);
     }
     std::vector<int> border[2];
     for (int si = 0; si < 2; si++) {
@@ -508,8 +664,21 @@ Structure::Structure(const dplus_pdb_desc *d, hipStream_t s) {
     const size_t ot = o64 + al(at64.size() * sizeof(double4));
     const size_t od = ot + al(tiles.size() * sizeof(int4));
     const size_t oc = od + al(bdims.size() * sizeof(int4));
-    const size_t total = oc + bcon.size() * sizeof(double);
+    // and the mesh builder's [classes | cells | box pieces | edges]
+    const size_t of = al(oc + bcon.size() * sizeof(double));
+    const size_t os = al(of + mh.fion.size() * sizeof(int));
+    const size_t op = al(os + mh.start.size() * sizeof(int));
+    const size_t ol = al(op + mh.pieces.size() * sizeof(double4));
+    const size_t total = mh.ok ? ol + mh.lens.size() * sizeof(double4) : of;
     std::vector<char> host(total, 0);
+    if (mh.ok) {
+        memcpy(host.data() + of, mh.fion.data(), mh.fion.size() * sizeof(int));
+        memcpy(host.data() + os, mh.start.data(), mh.start.size() * sizeof(int));
+        if (!mh.pieces.empty()) {
+            memcpy(host.data() + op, mh.pieces.data(), mh.pieces.size() * sizeof(double4));
+            memcpy(host.data() + ol, mh.lens.data(), mh.lens.size() * sizeof(double4));
+        }
+    }
     memcpy(host.data(), at32.data(), at32.size() * sizeof(float4));
     memcpy(host.data() + o64, at64.data(), at64.size() * sizeof(double4));
     memcpy(host.data() + ot, tiles.data(), tiles.size() * sizeof(int4));
@@ -522,6 +691,13 @@ Structure::Structure(const dplus_pdb_desc *d, hipStream_t s) {
     dtiles = (const int4 *)(base + ot);
     ddims = (const int4 *)(base + od);
     dcon = (const double *)(base + oc);
+    if (mh.ok) {
+        mesh = mh.sources(atoms_on ? d->natoms : 0);
+        mesh.fion = (const int *)(base + of);
+        mesh.cells = (const int *)(base + os);
+        mesh.pieces = (const double4 *)(base + op);
+        mesh.lens = (const double4 *)(base + ol);
+    }
     check_hip(hipStreamSynchronize(s), "structure upload");
 }
 
@@ -558,7 +734,36 @@ BuildShape Structure::shape_for(const Grid &g, bool use_table) const {
     return sh;
 }
 
-BuildJob Structure::prepare(Grid &g, int slices, Pending &P, hipStream_t s) const {
+// The mesh builder where it is the faster one, within kMeshRoom bytes of workspace or what
+// the direct builder's slice partials may take.
+size_t direct_build_bytes(int N) { return (size_t)kMaxSlices * 12 * pair_units(half_base(N + 1)) * sizeof(double); }
+
+static bool mesh_route_of(const MeshSources &S, long long nsources, int N, double step, bool fp64, int nion, MeshPlan &P,
+                          MeshSizes &Z) {
+    return mesh_plan(S, N, step, fp64, nion, std::max(kMeshRoom, direct_build_bytes(N)), P, Z) &&
+           mesh_pays(P, Z, N, (double)nsources, fp64);
+}
+
+bool Structure::mesh_route(const Grid &g, MeshPlan &P, MeshSizes &Z) const {
+    return mesh_route_of(mesh, nsources, g.N, g.step, g.fp64(), desc.nion, P, Z);
+}
+
+size_t mesh_build_bytes(const dplus_pdb_desc *d, int grid_size, double qmax, bool fp64) {
+    const bool atoms_on = (d->flags & (DPLUS_CALC_ATOMIC_FORMFACTORS | DPLUS_CALC_DUMMY_SOLVENT)) && d->natoms > 0;
+    const BoxSet sets[2] = {{d->box_contrast != 0.0 ? d->nbox : 0, d->box_dims, d->box_com, d->box_contrast},
+                            {d->excl_contrast != 0.0 ? d->nexcl : 0, d->excl_dims, d->excl_com, d->excl_contrast}};
+    if (grid_size % 2) grid_size++;
+    const int N = actual_size(grid_size);
+    const MeshHost mh(d, atoms_on, sets, true);
+    MeshPlan P;
+    MeshSizes Z;
+    return mesh_route_of(mh.sources(atoms_on ? d->natoms : 0), (atoms_on ? d->natoms : 0) + (long long)sets[0].n + sets[1].n,
+                         N, qmax / (double)(grid_size / 2), fp64, d->nion, P, Z)
+               ? Z.bytes
+               : 0;
+}
+
+BuildJob Structure::prepare(Grid &g, int slices, Pending &P, hipStream_t s, bool direct) const {
     std::vector<double> ff;
     form_factor_table(&desc, ion_counts, g.N, g.step, ff);
     // origin: sum of f~(0) over atoms + each box set's contrast * total volume
@@ -566,6 +771,36 @@ BuildJob Structure::prepare(Grid &g, int slices, Pending &P, hipStream_t s) cons
     if (atoms_on)
         for (int i = 0; i < desc.nion; i++) P.origin += ion_counts[i] * ff[i];
     if (boxes_on) P.origin += box_origin;
+    MeshJob &M = P.job;
+    P.mesh = !direct && mesh_route(g, M.plan, M.z);
+    if (P.mesh) {
+        std::vector<MeshBand> bands;
+        mesh_bands(M.plan, M.z, g.N, g.fp64(), bands, M.ntiles);
+        // one upload: [form factors | tables | bands]
+        const size_t nf = ff.size();
+        ff.resize(nf + M.z.tab);
+        mesh_tables(M.plan, g.fp64(), ff.data() + nf);
+        const size_t bytes = ff.size() * sizeof(double);
+        ff.resize(ff.size() + (bands.size() * sizeof(MeshBand) + 7) / 8);
+        memcpy((char *)ff.data() + bytes, bands.data(), bands.size() * sizeof(MeshBand));
+        P.ff.upload(ff.data(), ff.size() * sizeof(double), s);
+        P.part.ensure(M.z.bytes);
+        M.atoms = d64;
+        M.pieces = mesh.pieces;
+        M.lens = mesh.lens;
+        M.natoms = mesh.natoms;
+        M.npieces = mesh.npieces;
+        M.cells = mesh.cells;
+        M.fion = mesh.fion;
+        M.ff = (const double *)P.ff.p;
+        M.tab = M.ff + nf;
+        M.bands = (const MeshBand *)((const char *)P.ff.p + bytes);
+        M.nbands = (int)bands.size();
+        M.work = P.part.p;
+        M.grid = g.dev.p;
+        M.scale = desc.scale;
+        return BuildJob{};
+    }
     // unreduced hardware sin/cos while every phase stays below 128 revolutions
     const double qtop = (double)(g.N + 1) * g.step;
     P.reduce = !g.fp64() && (qtop * rmax / k2Pi >= 128.0 || getenv("DPLUS_REDUCE_PHASE") != nullptr);
@@ -603,6 +838,14 @@ BuildJob Structure::prepare(Grid &g, int slices, Pending &P, hipStream_t s) cons
     return J;
 }
 
+void Structure::launch(Grid &g, BuildJob &J, int wg, const Pending &P, hipStream_t s) const {
+    if (P.mesh)
+        launch_mesh(P.job, g.fp64(), s);
+    else
+        launch_build_batch(P.reduce, wg, &J, 1, s);
+    check_hip(hipGetLastError(), "build launch");
+}
+
 void Structure::enqueue_finish(Grid &g, const Pending &P, hipStream_t s, bool timed) const {
     launch_set_origin(g.fp64(), g.dev.p, P.origin * desc.scale, s);
     check_hip(hipGetLastError(), "set_origin launch");
@@ -618,7 +861,7 @@ void Structure::finish(Grid &g, const Pending &P, bool host_copy, hipStream_t s)
         check_hip(hipStreamSynchronize(s), "pdb build");
 }
 
-void Structure::build(Grid &g, bool host_copy, hipStream_t s, bool use_table) {
+void Structure::build(Grid &g, bool host_copy, hipStream_t s, bool use_table, bool direct) {
     const bool phase64 = getenv("DPLUS_PHASE64") != nullptr;
     // paired builder: every mixed grid (but the FP64-phase diagnostic) and, unless
     // the plain form is selected, every FP64 grid
@@ -627,11 +870,10 @@ void Structure::build(Grid &g, bool host_copy, hipStream_t s, bool use_table) {
         // structure can be built into several grids at once on different streams
         Pending P;
         const BuildShape sh = shape_for(g, use_table);
-        BuildJob J = prepare(g, sh.slices, P, s);
+        BuildJob J = prepare(g, sh.slices, P, s, direct);
         {
             KTimer kt("build", s);
-            launch_build_batch(P.reduce, sh.wg, &J, 1, s);
-            check_hip(hipGetLastError(), "build_atoms launch");
+            launch(g, J, sh.wg, P, s);
         }
         finish(g, P, host_copy, s);
         timing_collect();
@@ -687,7 +929,7 @@ BuildShape Structure::autotune(Grid &g, hipStream_t s, double *best_ms, double *
         for (int wg : {64, 128, 256, 512}) {
             for (int S = 0; S <= smax; S++) {
                 // S = 0: the untimed warm-up of this workgroup size
-                BuildJob J = prepare(g, std::max(S, 1), P, s);
+                BuildJob J = prepare(g, std::max(S, 1), P, s, true);
                 check_hip(hipEventRecord(e0, s), "hipEventRecord");
                 launch_build_batch(P.reduce, wg, &J, 1, s);
                 check_hip(hipGetLastError(), "build_atoms launch");
@@ -705,8 +947,7 @@ BuildShape Structure::autotune(Grid &g, hipStream_t s, double *best_ms, double *
             }
         }
         BuildJob J = prepare(g, best.slices, P, s);
-        launch_build_batch(P.reduce, best.wg, &J, 1, s);
-        check_hip(hipGetLastError(), "build_atoms launch");
+        launch(g, J, best.wg, P, s);
         finish(g, P, false, s);
     } catch (...) {
         (void)hipEventDestroy(e0);
@@ -1647,14 +1888,28 @@ int dplus_structure_build_grids(int n, dplus_structure *const *sh, dplus_grid *c
         }
         Device::get().require();
         const hipStream_t s = Device::get().stream;
-        // mixed grids in grouped launches of up to 16 per phase form; FP64 grids one by one
+        // mixed grids in grouped launches of up to 16 per phase form; FP64 grids and those of the
+        // mesh builder one by one (its workspaces released in stream order as it goes)
         std::vector<int> mixed;
         for (int i = 0; i < n; i++) {
             Grid *g = (Grid *)gh[i];
-            if (g->fp64() || getenv("DPLUS_PHASE64"))
-                ((Structure *)sh[i])->build(*g, host_copy != 0, s);
-            else
+            Structure *st = (Structure *)sh[i];
+            MeshPlan mp;
+            MeshSizes mz;
+            if (g->fp64() || getenv("DPLUS_PHASE64")) {
+                st->build(*g, host_copy != 0, s);
+            } else if (st->mesh_route(*g, mp, mz)) {
+                Structure::Pending P;
+                BuildJob J = st->prepare(*g, 1, P, s);
+                {
+                    KTimer kt("build", s);
+                    st->launch(*g, J, 256, P, s);
+                }
+                st->enqueue_finish(*g, P, s, true);
+                if (host_copy) g->download(s);
+            } else {
                 mixed.push_back(i);
+            }
         }
         std::vector<Structure::Pending> P(mixed.size());
         std::vector<BuildJob> jobs(mixed.size());
@@ -1681,6 +1936,7 @@ int dplus_structure_build_grids(int n, dplus_structure *const *sh, dplus_grid *c
         }
         for (size_t k = 0; k < mixed.size(); k++)
             ((Structure *)sh[mixed[k]])->finish(*(Grid *)gh[mixed[k]], P[k], host_copy != 0, s);
+        check_hip(hipStreamSynchronize(s), "grouped build");
         timing_collect();
     })
 }

@@ -336,6 +336,66 @@ struct BuildBatch {
     int njobs;
     BuildJob job[kMaxBuildJobs];
 };
+// ---- mesh builder (amp_mesh.hip): a grid's amplitudes through a frequency mesh
+constexpr int kMeshFields = 64;    // classes of sources (ions, and one of box pieces)
+constexpr int kMeshCells = 32;     // source cells per axis at most
+constexpr size_t kMeshRoom = (size_t)512 << 20;  // workspace bytes
+constexpr double kMeshPiece = 0.3;  // longest edge of a box piece, nm
+// a structure's sources as the mesh builder reads them: classes 0..nfield-1 (the
+// ions in use, then the box pieces), each sorted by cell
+struct MeshSources {
+    bool ok = false;  // finite coordinates, box pieces of a bounded number
+    int nfield = 0;
+    long long natoms = 0, npieces = 0;
+    double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // extent of the sources, box pieces whole
+    double cell0[3] = {0, 0, 0}, cell_inv = 0.0;
+    int ncell[3] = {1, 1, 1};
+    double piece_half[3] = {0, 0, 0};  // largest half edges of a piece
+    // device: class of each field (ion, or -1: box pieces), first source of every
+    // cell [nfield][cells + 1], box pieces (centre, contrast) and their edges
+    const int *fion = nullptr, *cells = nullptr;
+    const double4 *pieces = nullptr, *lens = nullptr;
+};
+struct MeshAxis {
+    int m, k, n0;  // mesh points; frequencies (n - n0) dk, n < k
+    double h, hinv, x0, dk, dkinv, c, turn, turn_lo;  // mesh point j at c + x0 + j h
+};
+struct MeshPlan {
+    MeshAxis ax[3];
+    int nfield, boxes, nion, shifted, gl, wp_box;
+    int ncell[3];
+    double cell0[3], cell_inv, box_half[3], step;
+    int t_spread, t_sinv, t_interp, t_iinv, t_gl;  // offsets of the tables
+};
+// workspace layout (bytes), classes per pass, slices of a brick's sources, table length
+// (doubles), node spacing in frequency steps, and the kernels' work
+struct MeshSizes {
+    size_t wb, bb, e0, e1, e2, g, b0, b1, bytes;
+    int group, slices, tab;
+    double s, nodes, pairs, dft, tiles;
+};
+struct MeshBand {
+    int shell, j0, rows, cols, tile0;
+};
+struct MeshJob {
+    MeshPlan plan;
+    MeshSizes z;
+    const double4 *atoms, *pieces, *lens;
+    long long natoms, npieces;
+    const int *cells, *fion;
+    const double *ff, *tab;
+    const MeshBand *bands;
+    int nbands, ntiles;
+    void *work, *grid;
+    double scale;
+};
+// the plan of a grid of N shells over `room` bytes of workspace at most; false: not possible
+bool mesh_plan(const MeshSources &S, int N, double step, bool fp64, int nion, size_t room, MeshPlan &P, MeshSizes &Z);
+// whether the mesh builder is the faster one
+bool mesh_pays(const MeshPlan &P, const MeshSizes &Z, int N, double sources, bool fp64);
+void mesh_bands(const MeshPlan &P, const MeshSizes &Z, int N, bool fp64, std::vector<MeshBand> &bands, int &ntiles);
+void mesh_tables(const MeshPlan &P, bool fp64, double *tab);
+void launch_mesh(const MeshJob &J, bool fp64, hipStream_t s);
 // launch shape of the paired builder: workgroup size (64, 128, 256 or 512
 // units) and atom slices (1..kMaxSlices)
 struct BuildShape {
@@ -360,10 +420,12 @@ struct Structure {
     const double4 *d64 = nullptr;
     const int4 *dtiles = nullptr, *ddims = nullptr;
     const double *dcon = nullptr;
+    MeshSources mesh;
     Structure(const dplus_pdb_desc *d, hipStream_t s);
     // use_table: the launch shape from the autotuner's table where it has the grid's
     // class (shapes timed on a device to themselves), else the occupancy model's
-    void build(Grid &g, bool host_copy, hipStream_t s, bool use_table = true);
+    // direct: never through the mesh builder
+    void build(Grid &g, bool host_copy, hipStream_t s, bool use_table = true, bool direct = false);
     // The mixed build in three steps, for callers that launch the builder of
     // several grids together: prepare uploads this grid's form factors and
     // sizes the slice partials (buffers owned by `bufs`, used on stream s) and
@@ -373,8 +435,15 @@ struct Structure {
         DevBuf ff, part;
         double origin = 0.0;
         bool reduce = false;
+        bool mesh = false;  // the grid goes through the mesh builder: launch_mesh(job), no BuildJob
+        MeshJob job{};
     };
-    BuildJob prepare(Grid &g, int slices, Pending &bufs, hipStream_t s) const;
+    // direct: the direct builder whatever mesh_pays says (the autotuner's timing)
+    BuildJob prepare(Grid &g, int slices, Pending &bufs, hipStream_t s, bool direct = false) const;
+    // the builder's kernels of a prepared grid
+    void launch(Grid &g, BuildJob &J, int wg, const Pending &bufs, hipStream_t s) const;
+    // whether the grid goes through the mesh builder, and its plan
+    bool mesh_route(const Grid &g, MeshPlan &P, MeshSizes &Z) const;
     void finish(Grid &g, const Pending &bufs, bool host_copy, hipStream_t s) const;
     // finish's kernels alone (origin, splines): no upload, allocation or
     // synchronisation once g.prepare_splines ran, so they can be captured
@@ -387,6 +456,10 @@ struct Structure {
     BuildShape autotune(Grid &g, hipStream_t s, double *best_ms, double *model_ms);
 };
 
+// workspace bytes of a build: the direct builder's at most, and the mesh builder's (0: the
+// description's grid takes the direct builder)
+size_t direct_build_bytes(int N);
+size_t mesh_build_bytes(const dplus_pdb_desc *d, int grid_size, double qmax, bool fp64);
 std::vector<GroupDev> make_groups(const double *q, int nq, double step);
 // paired builder: work units of a grid with nhalf canonical nodes, the number
 // of atom slices the occupancy model splits a launch of workgroup size wg over

@@ -120,6 +120,7 @@ struct Request {
     bool want_chi = false;
     dplus_oa_params oa{};
     size_t need = 0;
+    bool direct_build = false;  // its budget does not hold the mesh builder's workspace
     // results
     std::vector<double> I;
     double chi2 = 0.0;
@@ -148,8 +149,7 @@ size_t request_bytes(const Request &r) {
         // FP64 partial sums of the paired builder's atom slices (as many as a
         // tuned launch shape may take; FP64 grids too, unless built plainly)
         if (!fp64 || !fp64_plain_builder()) {
-            const long long units = pair_units(half_base(gs / 2 + 4));
-            b += (size_t)kMaxSlices * 12 * units * sizeof(double);
+            b += direct_build_bytes(gs / 2 + 3);
         }
         b += (size_t)(r.desc.natoms + r.desc.nbox + r.desc.nexcl) * 48;
         step = r.qmax / (double)(gs / 2);
@@ -387,7 +387,7 @@ struct Engine {
     // shape table's entries are timed on an otherwise idle device, and on the
     // concurrent request stream they were slower than the model (a 512-request
     // stream 619-637 against 660-672 curves/s).
-    void build(Structure &S, Grid &g, hipStream_t s) {
+    void build(Structure &S, Grid &g, hipStream_t s, bool direct) {
         BuildShape tuned;
         const bool mixed = !g.fp64() && getenv("DPLUS_PHASE64") == nullptr;
         if (mixed && autotune && !shape_lookup(g.N, S.ntiles, &tuned)) {
@@ -398,13 +398,15 @@ struct Engine {
             }
         }
         const double terms = (double)half_base(g.N + 1) * (double)S.nsources;
-        if (!mixed || !batch_builds || terms > batch_terms) {
-            S.build(g, false, s, autotune);
+        MeshPlan mp;
+        MeshSizes mz;
+        if (!mixed || !batch_builds || terms > batch_terms || (!direct && S.mesh_route(g, mp, mz))) {
+            S.build(g, false, s, autotune, direct);
             return;
         }
         Structure::Pending P;
         BuildTicket t;
-        t.job = S.prepare(g, S.shape_for(g, autotune).slices, P, s);
+        t.job = S.prepare(g, S.shape_for(g, autotune).slices, P, s, true);
         t.reduce = P.reduce;
         check_hip(hipEventCreateWithFlags(&t.ready, hipEventDisableTiming), "hipEventCreate");
         if (hipEventCreateWithFlags(&t.done, hipEventDisableTiming) != hipSuccess) {
@@ -551,7 +553,7 @@ struct Engine {
             if (r.has_pdb) {
                 S = structure_for(r, s);
                 G.reset(new Grid(r.grid_size, r.qmax, r.precision));
-                build(*S, *G, s);
+                build(*S, *G, s, r.direct_build);
                 g = G.get();
             }
             const double single[4] = {0, 0, 0, 1}, origin[3] = {0, 0, 0};
@@ -709,7 +711,7 @@ struct Engine {
                 }
                 if (build_in_chain) {
                     sh = S->shape_for(*g, autotune);
-                    J = S->prepare(*g, sh.slices, P, s);
+                    J = S->prepare(*g, sh.slices, P, s, r.direct_build);
                     g->prepare_splines(s);
                 }
             }
@@ -766,13 +768,15 @@ struct Engine {
             // (grid sizes, launch sizes and buffers may differ within a key: an update
             // takes them; rows beyond the one-wave splines add a kernel)
             if (build_in_chain)
-                key += "/b" + std::to_string(sh.wg) + (P.reduce ? "r" : "u") + (g->fp64() ? "d" : "f") +
-                       (g->N > kWaveShellMax ? "L" : "S");
+                key += (P.mesh ? "/m" + std::to_string((P.job.plan.nfield + P.job.z.group - 1) / P.job.z.group) +
+                                     (P.job.npieces > 0 ? "b" : "a")
+                               : "/b" + std::to_string(sh.wg) + (P.reduce ? "r" : "u")) +
+                       (g->fp64() ? "d" : "f") + (g->N > kWaveShellMax ? "L" : "S");
             if (!graph_mode) {
                 if (build_in_chain) {
                     {
                         KTimer kt("build", s);
-                        launch_build_batch(P.reduce, sh.wg, &J, 1, s);
+                        S->launch(*g, J, sh.wg, P, s);
                         check_hip(hipGetLastError(), "build_atoms launch");
                     }
                     S->enqueue_finish(*g, P, s, true);
@@ -800,7 +804,7 @@ struct Engine {
                     }
                 } end_on_throw{s};
                 if (build_in_chain) {
-                    launch_build_batch(P.reduce, sh.wg, &J, 1, s);
+                    S->launch(*g, J, sh.wg, P, s);
                     check_hip(hipGetLastError(), "build_atoms launch");
                     S->enqueue_finish(*g, P, s, false);
                 }
@@ -1036,6 +1040,18 @@ int dplus_engine_submit(dplus_engine *eh, const dplus_request *rq, long long *ti
         }
         r->oa = rq->oa;
         r->need = request_bytes(*r);
+        if (r->has_pdb && (r->precision == DPLUS_PRECISION_FP64 ? !fp64_plain_builder() : true)) {
+            // the mesh builder's workspace where it is the larger one; a budget that holds
+            // the request only without it keeps the direct builder
+            const size_t direct = direct_build_bytes((r->grid_size + r->grid_size % 2) / 2 + 3);
+            const size_t mesh = mesh_build_bytes(&r->desc, r->grid_size, r->qmax, r->precision == DPLUS_PRECISION_FP64);
+            if (mesh > direct) {
+                if (r->need + (mesh - direct) + e->cache_cap + e->arena_cap <= e->budget)
+                    r->need += mesh - direct;
+                else
+                    r->direct_build = true;
+            }
+        }
         if (r->need + e->cache_cap + e->arena_cap > e->budget)
             throw Error(kErrOutOfMemory, "the request needs " + std::to_string(r->need) +
                                              " device bytes, more than the engine's budget of " +
