@@ -369,17 +369,25 @@ __device__ __forceinline__ float wave_total(float v) {
 __device__ __forceinline__ double wave_total(double v) { return wave_sum(v); }
 
 // weights of the 4-point spline (four_point's end derivatives, then the cubic
-// Hermite at t) over values y0..y3: the spline at t is sum_r w[r] y[r]
+// Hermite at t) over values y0..y3, as cubics in t: the spline at t is sum_r w[r] y[r].
+// w[1] = 1 + t (-1/5 + t (-9/5 + t)) closes the sum to 1, so that rounding scales nothing.
 template <typename T>
 __device__ __forceinline__ void spline4_weights(T t, T w[4]) {
-    const T a = (T)(7. / 15.), b = (T)(14. / 15.), c = (T)(4. / 15.), e = (T)(2. / 15.);
-    const T t2 = t * t, t3 = t2 * t;
-    const T h00 = (T)1 - (T)3 * t2 + (T)2 * t3, h01 = (T)3 * t2 - (T)2 * t3, h10 = t - (T)2 * t2 + t3,
-            h11 = t3 - t2;
-    w[0] = h10 * (a - b) + h11 * (c - e);
-    w[1] = h00 + h10 * (c - a) + h11 * (e - b);
-    w[2] = h01 + h10 * (b - e) + h11 * (a - c);
-    w[3] = h10 * (e - c) + h11 * (b - a);
+    w[0] = t * ((T)(-7. / 15.) + t * ((T)(4. / 5.) - (T)(1. / 3.) * t));
+    w[2] = t * ((T)(4. / 5.) + t * ((T)(6. / 5.) - t));
+    w[3] = t * ((T)(-2. / 15.) + t * ((T)(-1. / 5.) + (T)(1. / 3.) * t));
+    w[1] = ((T)1 - w[2]) - (w[0] + w[3]);
+}
+
+// the same for a q, whose weights every direction shares: formed in FP64
+template <typename T>
+__device__ __forceinline__ void q_weights(double t, T w[4]) {
+    double v[4];
+    spline4_weights<double>(t, v);
+    w[0] = (T)v[0];
+    w[2] = (T)v[2];
+    w[3] = (T)v[3];
+    w[1] = ((T)1 - w[2]) - (w[0] + w[3]);
 }
 
 // the four planes' amplitudes (layer - 1 .. layer + 2) of one lookup at (th, ph),
@@ -409,6 +417,279 @@ template <typename T, typename T4>
 __device__ __noinline__ void direct_planes_call(const T4 *__restrict__ g, int layer, double th, double ph,
                                                 cplx<T> *amps) {
     direct_planes<T, T4>(g, layer, th, ph, amps);
+}
+
+// ------------------------------------------------------------------ patch tiles
+// A patch of directions (an equal-area stratum, neighbouring VEGAS bins) touches a small
+// rectangle of each shell's (theta, phi) nodes.  A workgroup copies the rectangle to LDS
+// with coalesced loads, rows and columns wrapped as plane_lookup wraps them, and its
+// directions look up there: 16-byte LDS reads at ~8..20 clocks a wave instead of
+// divergent loads at 64, and one base address for the eight nodes.
+struct Tile {
+    int t0, p0, rows, cols, stride;
+    __device__ int nodes() const { return rows * stride; }
+};
+
+// the rectangle of shell i for theta = pi [ut0, ut1], phi = 2 pi [up0, up1] (1e-6 of a cell
+// of margin for the rounding of the ends)
+__device__ __forceinline__ Tile patch_tile(int shell, double ut0, double ut1, double up0, double up1) {
+    Tile t;
+    const double m = 3.0 * shell, n = 6.0 * shell;
+    t.t0 = (int)floor(ut0 * m - 1e-6) - 1;
+    t.rows = (int)floor(ut1 * m + 1e-6) + 2 - t.t0 + 1;
+    t.p0 = (int)floor(up0 * n - 1e-6);
+    t.cols = (int)floor(up1 * n + 1e-6) + 1 - t.p0 + 1;
+    t.stride = t.cols | 1;  // odd: the rows of one lookup start in different banks
+    return t;
+}
+
+// 256 threads: a wave takes whole rows, or the power of two of them that fits its lanes,
+// so that the column's place is worked out once and a node costs its load and its store
+template <typename T4>
+__device__ __forceinline__ void stage_tile(const T4 *__restrict__ plane, int shell, const Tile &t, T4 *tile) {
+    const int n = 6 * shell, m = 3 * shell;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lw = min(32 - __builtin_clz(t.cols - 1), 6), per = 64 >> lw;
+    for (int c = lane & ((1 << lw) - 1); c < t.cols; c += 64) {
+        int k = t.p0 + c;
+        k += k < 0 ? n : 0;
+        k -= k >= n ? n : 0;
+        const int r0 = w * per + (lane >> lw);
+        if (t.t0 >= 0 && t.t0 + t.rows <= m + 1) {  // no row past a pole
+            const T4 *src = plane + (n * (t.t0 + r0) + k);
+            T4 *dst = tile + r0 * t.stride + c;
+            const int ds = 4 * per * n, dt = 4 * per * t.stride;
+            int r = r0;
+            for (; r + 12 * per < t.rows; r += 16 * per) {  // four loads in flight
+                const T4 a = src[0], b = src[ds], d = src[2 * ds], e = src[3 * ds];
+                dst[0] = a;
+                dst[dt] = b;
+                dst[2 * dt] = d;
+                dst[3 * dt] = e;
+                src += 4 * ds;
+                dst += 4 * dt;
+            }
+            for (; r < t.rows; r += 4 * per) {
+                *dst = *src;
+                src += ds;
+                dst += dt;
+            }
+        } else {
+            const int half = k + m >= n ? k + m - n : k + m;  // past a pole: half a turn away in phi
+#pragma unroll 2
+            for (int r = r0; r < t.rows; r += 4 * per) {
+                int v = t.t0 + r, q = k;
+                if (v < 0 || v > m) {  // the row on the other side
+                    v = v < 0 ? v + m + 1 : v - (m + 1);
+                    q = half;
+                }
+                tile[r * t.stride + c] = plane[n * min(max(v, 0), m) + q];
+            }
+        }
+    }
+}
+
+// cell and fraction of 0 <= x < 2^31 by FP64 additions (the conversions run at a quarter of
+// their rate): x - 1/2 rounds to the cell in the low mantissa bits of x - 1/2 + 1.5 2^52.  At
+// a node the cell may be the lower one, with fraction 1: the same interpolated value.
+__device__ __forceinline__ double cell_of(double x, int &i) {
+    const double magic = 6755399441055744.0, t = (x - 0.5) + magic;
+    i = (int)(unsigned)__double_as_longlong(t);
+    return x - (t - magic);
+}
+
+// plane_lookup on a staged tile, as sums over the nodes with the phi Hermite's and the
+// theta spline's weights
+template <typename T, typename T4>
+__device__ __forceinline__ cplx<T> tile_lookup(const T4 *tile, const Tile &t, int shell, double ut, double up) {
+    int tI, pI;
+    const T s = (T)cell_of(ut * (double)(3 * shell), tI);
+    const T p = (T)cell_of(up * (double)(6 * shell), pI), p2 = p * p, p3 = p2 * p;
+    const T h01 = (T)3 * p2 - (T)2 * p3, h00 = (T)1 - h01, h11 = p3 - p2, h10 = h11 - p2 + p;
+    T w[4];
+    spline4_weights<T>(s, w);
+    const T4 *row = tile + (tI - 1 - t.t0) * t.stride + (pI - t.p0);
+    cplx<T> a = {(T)0, (T)0};
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const T4 A = row[r * t.stride], B = row[r * t.stride + 1];
+        const T x = h00 * A.x + h01 * B.x + h10 * A.z + h11 * B.z;
+        const T y = h00 * A.y + h01 * B.y + h10 * A.w + h11 * B.w;
+        a.x += w[r] * x;
+        a.y += w[r] * y;
+    }
+    return a;
+}
+
+// one plane's lookup from the grid, for what has no tile: the origin (layer 0's plane), the
+// antipode on shell 1 (plane -1), patches larger than the tile
+template <typename T, typename T4>
+__device__ __noinline__ cplx<T> plane_direct(const T4 *__restrict__ g, int lqi, double ut, double up) {
+    if (lqi == 0) {
+        const T4 o = g[0];
+        return {o.x, o.y};
+    }
+    if (lqi < 0) {
+        double nth, nph;
+        antipode(ut * kPi, up * k2Pi, nth, nph);
+        return plane_lookup<T, T4, false>(g + 1, 1, nth * kInvPi, nph * kInv2Pi);
+    }
+    return plane_lookup<T, T4, false>(g + shell_base(lqi), lqi, ut, up);
+}
+
+// the planes' tiles of a patch: lane p of every four works out plane p's (shell0 + p), then
+// each is read as wave-uniform values
+__device__ __forceinline__ Tile tile_of(const Tile &mine, int p) {
+    return {__builtin_amdgcn_readlane(mine.t0, p), __builtin_amdgcn_readlane(mine.p0, p),
+            __builtin_amdgcn_readlane(mine.rows, p), __builtin_amdgcn_readlane(mine.cols, p),
+            __builtin_amdgcn_readlane(mine.stride, p)};
+}
+
+// Sums of M values over groups of L lanes (L >= M, powers of two): at each step a lane
+// passes on half of its values and adds the other lane's of the half it keeps, so M - 1
+// exchanges and log2(L / M) more instead of M log2 L.  Returns the sum of value
+// (lane % L) / (L / M).
+template <int M>
+__device__ __forceinline__ double group_sums(const double (&v)[M], int lane, int L) {
+    if constexpr (M > 1) {
+        const int o = L >> 1;
+        const bool hi = lane & o;
+        double u[M / 2];
+#pragma unroll
+        for (int i = 0; i < M / 2; i++) {
+            const double send = hi ? v[i] : v[i + M / 2], keep = hi ? v[i + M / 2] : v[i];
+            u[i] = keep + __shfl_xor(send, o, 64);
+        }
+        return group_sums<M / 2>(u, lane, o);
+    } else {
+        double t = v[0];
+        for (int o = L >> 1; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+        return t;
+    }
+}
+
+// LDS nodes of one plane's tile: 38 KB, four workgroups per CU
+template <typename T4>
+constexpr int tile_nodes() {
+    return 38 * 1024 / (int)sizeof(T4);
+}
+
+// theta / pi of cos theta = 2 u - 1.  For FP32 lookups 2 asin(sqrt y) / pi, y = 1 - u, by a
+// polynomial of asin(sqrt y) / sqrt y on [0, 1/2] (9e-14) and sqrt by one Newton step on the
+// FP32 root (1e-14): a cell's fraction stays well below FP32's rounding of it.
+template <typename T>
+__device__ __forceinline__ double polar_fraction(double u) {
+    if (sizeof(T) == 8) return acos(2.0 * u - 1.0) * kInvPi;
+    const bool flip = u < 0.5;
+    const double y = fmax(flip ? u : 1.0 - u, 1e-30);
+    const float s0 = __builtin_amdgcn_sqrtf((float)y);
+    double s = (double)s0;
+    s = fma(fma(-s, s, y), (double)(0.5f * __builtin_amdgcn_rcpf(s0)), s);
+    const double c[14] = {0.6366197723674882,   0.10610329546639952, 0.047746473800039865, 0.02842098102029294,
+                          0.019329935850208507, 0.014425052426250716, 0.009232696985335458, 0.02102495864195202,
+                          -0.048506457009034394, 0.18417602577157377, -0.3818597693281228,  0.5575447279642045,
+                          -0.46861904441904245, 0.19281950697472416};
+    double v = c[13];
+#pragma unroll
+    for (int i = 12; i >= 0; i--) v = fma(v, y, c[i]);
+    return flip ? 1.0 - s * v : s * v;
+}
+
+// The MC average of a single leaf over several chunks: a workgroup takes one patch of
+// the stratification (mc_stratify) and 4 D of its chunks, 64 directions each: per plane
+// the patch's tile is staged once and serves 256 D lookups, and the q of the group share
+// the lookups through per-q weights.  The same directions as mc_kernel; the sums over
+// them are grouped by patch instead of by run of 256.  2,000 atoms, grid 100, 10^6
+// directions, 500 q: 1.93 -> 0.94 ms (FP64, 262,144: 0.91 -> 0.45).  mc_kernel waits on 32
+// divergent loads a lookup; here the VALU is full (about 720 instructions per 64
+// directions and group, 150 of them the draw), so fewer instructions are what is left.
+template <typename T, typename T4, int D>
+__global__ __launch_bounds__(256) void mc_patch_kernel(const T4 *const *__restrict__ grids,
+                                                       const RotDev *__restrict__ rots,
+                                                       const GroupDev *__restrict__ groups,
+                                                       const int *__restrict__ active, int mstride,
+                                                       const double *__restrict__ qs, double step, uint64_t seed,
+                                                       long long dir0, int nchunks, int chunk, int nu, int nv, int nset,
+                                                       double *__restrict__ partial) {
+    __shared__ T4 tile[tile_nodes<T4>()];
+    __shared__ T wq[kMaxM][4];
+    __shared__ double red[4][kMaxM];
+    const int gi = blockIdx.y;
+    const GroupDev G = groups[active[gi]];
+    const int patch = blockIdx.x / nset, set = blockIdx.x - patch * nset;
+    const int iu = patch / nv, iv = patch - iu * nv;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int c0 = set * 4 * D + w;  // this wave's chunks: c0, c0 + 4, ...
+    double ut[D], up[D];
+    cplx<T> amp[4][D];
+    const double inu = 1.0 / (double)nu, inv = 1.0 / (double)nv;
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+        const int c = min(c0 + 4 * k, nchunks - 1);  // (a chunk past the last is not summed)
+        const long long d = dir0 + (long long)c * chunk + patch * 64 + lane;
+        double u, v;
+        uniform_pair(seed, (uint32_t)d, (uint32_t)(d >> 32), (uint32_t)G.layer, kStreamMC, u, v);
+        u = ((double)iu + u) * inu;
+        v = ((double)iv + v) * inv;
+        ut[k] = polar_fraction<T>(u);
+        up[k] = (k2Pi * v) * kInv2Pi;
+    }
+    const T4 *g = grids[rots[0].leaf];
+    const Tile mine = patch_tile(max(G.layer - 1 + (lane & 3), 1), polar_fraction<float>((double)(iu + 1) * inu),
+                                 polar_fraction<float>((double)iu * inu), (double)iv * inv, (double)(iv + 1) * inv);
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        const int lqi = G.layer - 1 + p;
+        const Tile t = tile_of(mine, p);
+        if (lqi > 0 && t.nodes() <= tile_nodes<T4>()) {  // uniform over the workgroup
+            if (p > 0) __syncthreads();
+            stage_tile(g + shell_base(lqi), lqi, t, tile);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < D; k++) amp[p][k] = tile_lookup<T, T4>(tile, t, lqi, ut[k], up[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < D; k++) amp[p][k] = plane_direct<T, T4>(g, lqi, ut[k], up[k]);
+        }
+    }
+    const double sc2 = (double)(T)rots[0].scale * (double)(T)rots[0].scale;
+    const double inv_step = 1.0 / step;
+    for (int jb = 0; jb < G.m; jb += kMaxM) {
+        const int m = min(kMaxM, G.m - jb);
+        __syncthreads();
+        if (threadIdx.x < m) {
+            T q4[4];
+            q_weights<T>((qs[G.q0 + jb + threadIdx.x] - G.layer * step) * inv_step, q4);
+#pragma unroll
+            for (int p = 0; p < 4; p++) wq[threadIdx.x][p] = q4[p];
+        }
+        __syncthreads();
+        auto intensity = [&](int j) {
+            const T w0 = wq[j][0], w1 = wq[j][1], w2 = wq[j][2], w3 = wq[j][3];
+            double I = 0.0;
+#pragma unroll
+            for (int k = 0; k < D; k++) {
+                const T ax = w0 * amp[0][k].x + w1 * amp[1][k].x + w2 * amp[2][k].x + w3 * amp[3][k].x;
+                const T ay = w0 * amp[0][k].y + w1 * amp[1][k].y + w2 * amp[2][k].y + w3 * amp[3][k].y;
+                if (c0 + 4 * k < nchunks) I += (double)ax * (double)ax + (double)ay * (double)ay;
+            }
+            return I;
+        };
+        // eight q at a time through the wave's sums
+        for (int j0 = 0; j0 < m; j0 += 8) {
+            double I[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) I[j] = j0 + j < m ? intensity(j0 + j) : 0.0;
+            const double t = group_sums<8>(I, lane, 64);
+            if ((lane & 7) == 0) red[w][j0 + (lane >> 3)] = t;
+        }
+        __syncthreads();
+        if (threadIdx.x < m) {
+            const int j = threadIdx.x;
+            partial[((size_t)gi * gridDim.x + blockIdx.x) * mstride + jb + j] =
+                sc2 * ((red[0][j] + red[1][j]) + (red[2][j] + red[3][j]));
+        }
+    }
 }
 
 constexpr int kZWin = 64;  // nodes of one plane's collapsed row segment (one per lane)
@@ -467,7 +748,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void mc_zcopy_kernel(
     for (int jb = 0; jb < G.m; jb += M) {
         const int m = min(M, G.m - jb);
         const double *q = qs + G.q0 + jb;
-        if (threadIdx.x < m) spline4_weights<T>((T)((q[threadIdx.x] - G.layer * step) * inv_step), wq[threadIdx.x]);
+        if (threadIdx.x < m) q_weights<T>((q[threadIdx.x] - G.layer * step) * inv_step, wq[threadIdx.x]);
         __syncthreads();
         double mine = 0.0;  // lane j < m: the wave's sum over its directions of |A_j|^2
         for (int i = 0; i < 64; i++) {
@@ -833,7 +1114,8 @@ __device__ __forceinline__ double lanes_sum(double v, int L) {
     return v;
 }
 
-template <typename T, typename T4, int kL, bool kSingle, int kP>  // kL: lanes per bin fixed at compile time, or 0 for L
+// kL: lanes per bin fixed at compile time, or 0 for L; kTiled: a single leaf with L >= 8
+template <typename T, typename T4, int kL, bool kSingle, int kP, bool kTiled>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(const T4 *const *__restrict__ grids,
                                                     const RotDev *__restrict__ rots, int nrot,
                                                     const double4 *__restrict__ trans,
@@ -862,13 +1144,14 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(cons
         const int p = pl + L * k;
         double u = 0.5, v = 0.5;
         if (p < ppb) uniform_pair(seed, (uint32_t)(bin * ppb + p), (uint32_t)iter, (uint32_t)G.layer, kStreamVegas, u, v);
-        const double th = acos(1. - 2. * (u * (bt[ti + 1] - bt[ti]) + bt[ti]));
+        u = u * (bt[ti + 1] - bt[ti]) + bt[ti];
         const double ph = (v * (bp[pj + 1] - bp[pj]) + bp[pj]) * 2. * kPi;
-        if (kSingle) {  // the lookup takes the angles themselves
-            qv[k][0] = th;
-            qv[k][1] = ph;
+        if (kSingle) {  // the lookup takes theta / pi and phi / 2 pi (u runs from the other pole than MC's)
+            qv[k][0] = polar_fraction<T>(1. - u);
+            qv[k][1] = ph * kInv2Pi;
             qv[k][2] = 0.0;
         } else {
+            const double th = acos(1. - 2. * u);
             double st, ct, sp, cp;
             sincos(th, &st, &ct);
             sincos(ph, &sp, &cp);
@@ -877,36 +1160,52 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(cons
             qv[k][2] = ct;
         }
     }
-    // single leaf: each point's lookup (the two inner planes and the q-spline slopes)
-    // once, held for every q chunk of the group; points in a rolled loop, one
-    // lookup in flight (unrolled, the points' gathers would be interleaved past
-    // the register budget), their results kept by selection
-    T hold[kP][8];
+    // single leaf: each point's lookup (four planes) once, held for every q chunk of the
+    // group.  A workgroup's bins are neighbours in phi on one theta row of bins (L >= 8), so
+    // where that patch's nodes are fewer than half the points' node reads they are staged
+    // as a tile (grid 250, 98 points a bin: 556 -> 403 us an iteration; FP64, grid 120, 24
+    // points: 143 -> 118; fewer than 8 lanes a bin, or tiles of more nodes, gained nothing);
+    // else the points look up in the grid, in a rolled loop, one lookup in flight
+    // (unrolled, their gathers would be interleaved past the register budget), their
+    // results kept by selection.
+    cplx<T> hold[kP][4];
+    __shared__ T4 tile[kTiled ? tile_nodes<T4>() : 1];
+    __shared__ T wq[kSingle ? kVM : 1][4];
     if (kSingle) {
+        const T4 *grid = grids[rots[0].leaf];
+        const int nb = 256 / L, b0 = blockIdx.x * nb, r0 = b0 / kVB, q0 = b0 % kVB;
+        Tile mine{};
+        if (kTiled)
+            mine = patch_tile(max(G.layer - 1 + (lane & 3), 1), polar_fraction<float>(1. - bt[r0]),
+                              polar_fraction<float>(1. - bt[r0 + 1]), bp[q0], bp[q0 + nb]);
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const int lqi = G.layer - 1 + p;
+            const Tile t = tile_of(mine, p);
+            if (kTiled && lqi > 0 && t.nodes() <= tile_nodes<T4>() && t.nodes() < 4 * ppb * nb) {  // uniform
+                if (p > 0) __syncthreads();
+                stage_tile(grid + shell_base(lqi), lqi, t, tile);
+                __syncthreads();
+#pragma unroll
+                for (int k = 0; k < kP; k++)
+                    if (pl + L * k < ppb) hold[k][p] = tile_lookup<T, T4>(tile, t, lqi, qv[k][0], qv[k][1]);
+            } else {
 #pragma unroll 1
-        for (int k = 0; k < kP; k++) {
-            if (pl + L * k >= ppb) break;
-            double th = qv[0][0], ph = qv[0][1];
+                for (int k = 0; k < kP; k++) {
+                    if (pl + L * k >= ppb) break;
+                    double ut = qv[0][0], up = qv[0][1];
 #pragma unroll
-            for (int kk = 1; kk < kP; kk++)
-                if (kk == k) {
-                    th = qv[kk][0];
-                    ph = qv[kk][1];
-                }
-            cplx<T> amps[4], d1, d2;
-            group_planes<T, T4>(grids[rots[0].leaf], G.layer, th, ph, amps, d1, d2);
+                    for (int kk = 1; kk < kP; kk++)
+                        if (kk == k) {
+                            ut = qv[kk][0];
+                            up = qv[kk][1];
+                        }
+                    const cplx<T> a = plane_direct<T, T4>(grid, lqi, ut, up);
 #pragma unroll
-            for (int kk = 0; kk < kP; kk++)
-                if (kk == k) {
-                    hold[kk][0] = amps[1].x;
-                    hold[kk][1] = amps[1].y;
-                    hold[kk][2] = amps[2].x;
-                    hold[kk][3] = amps[2].y;
-                    hold[kk][4] = d1.x;
-                    hold[kk][5] = d1.y;
-                    hold[kk][6] = d2.x;
-                    hold[kk][7] = d2.y;
+                    for (int kk = 0; kk < kP; kk++)
+                        if (kk == k) hold[kk][p] = a;
                 }
+            }
         }
     }
     for (int jb = 0; jb < G.m; jb += kVM) {
@@ -915,25 +1214,28 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(cons
 #pragma unroll
         for (int j = 0; j < kVM; j++) e[j] = 0.0;
         if (kSingle) {
-            const T sc = (T)rots[0].scale;
-            const double inv_step = 1.0 / step;
+            // the q's weights over the planes, shared by every point
+            const double sc2 = (double)(T)rots[0].scale * (double)(T)rots[0].scale;
+            __syncthreads();
+            if (threadIdx.x < m) {
+                T w4[4];
+                q_weights<T>((qs[G.q0 + jb + threadIdx.x] - G.layer * step) * (1.0 / step), w4);
 #pragma unroll
-            for (int k = 0; k < kP; k++) {
-                if (pl + L * k >= ppb) continue;
-                const cplx<T> p1 = {hold[k][0], hold[k][1]}, p2 = {hold[k][2], hold[k][3]};
-                const cplx<T> d1 = {hold[k][4], hold[k][5]}, d2 = {hold[k][6], hold[k][7]};
+                for (int p = 0; p < 4; p++) wq[threadIdx.x][p] = w4[p];
+            }
+            __syncthreads();
 #pragma unroll
-                for (int j = 0; j < kVM; j++) {
-                    if (j < m) {
-                        const T t = (T)((qs[G.q0 + jb + j] - G.layer * step) * inv_step);
-                        const cplx<T> a = hermite<T>(p1, p2, d1, d2, t);
-                        cplx<T> acc = {(T)0, (T)0};
-                        acc.x += a.x * sc;
-                        acc.y += a.y * sc;
-                        const double I = (double)acc.x * (double)acc.x + (double)acc.y * (double)acc.y;
-                        e[j] += I;
-                        so[k] += I;
-                    }
+            for (int j = 0; j < kVM; j++) {
+                if (j >= m) continue;
+                const T w0 = wq[j][0], w1 = wq[j][1], w2 = wq[j][2], w3 = wq[j][3];
+#pragma unroll
+                for (int k = 0; k < kP; k++) {
+                    if (pl + L * k >= ppb) continue;
+                    const T ax = w0 * hold[k][0].x + w1 * hold[k][1].x + w2 * hold[k][2].x + w3 * hold[k][3].x;
+                    const T ay = w0 * hold[k][0].y + w1 * hold[k][1].y + w2 * hold[k][2].y + w3 * hold[k][3].y;
+                    const double I = sc2 * ((double)ax * (double)ax + (double)ay * (double)ay);
+                    e[j] += I;
+                    so[k] += I;
                 }
             }
         } else {
@@ -955,10 +1257,16 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(cons
                 }
             }
         }
+        if (kTiled || kL == 64) {  // L >= 8
+            const double t = group_sums<kVM>(e, lane, L);
+            const int lj = L / kVM, j = pl / lj;
+            if (pl % lj == 0 && j < m) binsum[((size_t)gi * mstride + jb + j) * (kVB * kVB) + bin] = t;
+        } else {
 #pragma unroll
-        for (int j = 0; j < kVM; j++) {
-            const double t = lanes_sum(e[j], L);
-            if (pl == 0 && j < m) binsum[((size_t)gi * mstride + jb + j) * (kVB * kVB) + bin] = t;
+            for (int j = 0; j < kVM; j++) {
+                const double t = lanes_sum(e[j], L);
+                if (pl == 0 && j < m) binsum[((size_t)gi * mstride + jb + j) * (kVB * kVB) + bin] = t;
+            }
         }
     }
     // variance of vol * S over the bin's points, two-pass (equal to the reference's Welford sum)
@@ -975,49 +1283,48 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(cons
     if (pl == 0) binvar[(size_t)gi * (kVB * kVB) + bin] = sq * ppb;
 }
 
-// damped re-binning weight of axis bin i from the axis's variance marginal
-// (HybridOA.cu:181-263): x = total / (local mean of var), w = ((x-1)/(x ln x))^1.5
-__device__ __forceinline__ double vegas_weight(const double *var, double total, int i) {
-    double x;
-    if (i == 0)
-        x = (var[0] + var[1]) / 2.;
-    else if (i == kVB - 1)
-        x = (var[i] + var[i - 1]) / 2.;
-    else
-        x = (var[i - 1] + var[i] + var[i + 1]) / 3.;
-    x = total / x;
-    x = pow((x - 1.) / (x * log(x)), 1.5);
-    if (x != x) x = 0.;
-    return x;
+// damped re-binning weight (HybridOA.cu:181-263) of x = total / (local mean of the
+// variances): ((x - 1) / (x ln x))^1.5, 0 where that is no number
+__device__ __forceinline__ double vegas_weight(double x) {
+    const double y = (x - 1.) / (x * log(x));
+    const double w = y * sqrt(y);
+    return w != w ? 0. : w;
 }
 
-// serial sweep of the re-binning: new interior boundaries at equal shares of
-// the weights; boundaries the sweep does not reach keep their previous value.
-// w, b and the scratch nb (kVB entries) are LDS arrays: the sweep's chain of
-// dependent steps then waits on LDS, not on global or private memory.
-__device__ void vegas_sweep(const double *w, double *b, double *nb) {
-    double tw = 0.0;
-    for (int i = 0; i < kVB; i++) tw += w[i];
-    for (int i = 0; i < kVB; i++) nb[i] = b[i + 1];
-    double xold, xnew = 0., dw = 0., pts = tw / kVB;
-    int j = 0;
-    for (int i = 0; i < kVB; i++) {
-        dw += w[i];
-        xold = xnew;
-        xnew = b[i + 1];
-        for (; dw > pts; j++) {
-            dw -= pts;
-            if (j < kVB) nb[j] = xnew - dw * (xnew - xold) / w[i];
-        }
+// The re-binning of one axis by a half wave (lane i of 32 holds weight w_i and the bin
+// [b_i, b_i+1]): new interior boundaries at equal shares of the weights.  Boundary j + 1
+// lies in the first bin whose running sum exceeds (j + 1) shares; boundaries that no sum
+// reaches keep their value.  lane i returns boundary i + 1 (of 32; the last stays).
+__device__ __forceinline__ double vegas_rebin(double w, double lo, double hi, int i, double *cum, double *wt, double *edge) {
+    const double first = __shfl(lo, 0, kVB);
+    double c = w;
+#pragma unroll
+    for (int d = 1; d < kVB; d <<= 1) {
+        const double t = __shfl_up(c, d, kVB);
+        if (i >= d) c += t;
     }
-    for (int i = 0; i < kVB - 1; i++) b[1 + i] = nb[i];
+    cum[i] = c;
+    wt[i] = w;
+    edge[i] = hi;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const double want = (cum[kVB - 1] / kVB) * (double)(i + 1);
+    int n = 0;  // bins whose running sum does not exceed the share (the sums do not fall)
+#pragma unroll
+    for (int s = kVB / 2; s > 0; s >>= 1)
+        if (!(cum[n + s - 1] > want)) n += s;
+    if (!(cum[n] > want) || i == kVB - 1) return hi;
+    const double right = edge[n], left = n > 0 ? edge[n - 1] : first;
+    return right - (cum[n] - want) * (right - left) / wt[n];
 }
 
 // one block (1024 threads = the 32x32 bins) per active group: the iteration's
 // integral sum_bins vol * mean_bin(I_j) (wave w takes q = w, w + 16, ...), the
-// theta/phi marginals of the bin variances, re-binning (weights on 64 lanes,
-// then one serial sweep per axis), and the running mean over iterations
-// (HybridVEGASResizeGridKernel; GPUHybridCalc.cu:654-701).
+// theta/phi marginals of the bin variances, re-binning, and the running mean over iterations
+// (HybridVEGASResizeGridKernel; GPUHybridCalc.cu:654-701).  The re-binning runs on one wave,
+// an axis per half wave, by scans and a binary search: 16.5 -> 5.8 us an iteration (its 64
+// serial steps waited on LDS).
 // hist[iter * nq + q] holds the running mean after iteration iter.
 __global__ __launch_bounds__(1024) void vegas_reduce(const GroupDev *__restrict__ groups,
                                                      const int *__restrict__ active, int mstride,
@@ -1030,24 +1337,41 @@ __global__ __launch_bounds__(1024) void vegas_reduce(const GroupDev *__restrict_
     const GroupDev G = groups[g];
     const int bin = threadIdx.x, ti = bin / kVB, pj = bin % kVB;
     double *bt = bounds + (size_t)g * 66, *bp = bt + 33;
-    __shared__ double sv[1024];
+    __shared__ double sv[kVB][kVB + 1];
     __shared__ double svol[1024];
-    __shared__ double marg[2][kVB];
-    __shared__ double wgt[2][kVB];
-    __shared__ double tot[2];
-    __shared__ double sb[2][kVB + 1], snb[2][kVB];
+    __shared__ double cum[2][kVB], wt[2][kVB], edge[2][kVB];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    sv[bin] = binvar[(size_t)gi * 1024 + bin];
+    sv[ti][pj] = binvar[(size_t)gi * 1024 + bin];
     svol[bin] = (bt[ti + 1] - bt[ti]) * (bp[pj + 1] - bp[pj]) / (double)ppb;
-    if (threadIdx.x < 2 * (kVB + 1)) {
-        const int ax = threadIdx.x / (kVB + 1), i = threadIdx.x % (kVB + 1);
-        sb[ax][i] = (ax == 0 ? bt : bp)[i];
+    // wave 0, half wave ax: axis ax, lane i its bin i
+    const int ax = lane / kVB, i = lane % kVB;
+    const double *b = ax == 0 ? bt : bp;
+    double lo = 0.0, hi = 0.0;
+    if (w == 0) {
+        lo = b[i];
+        hi = b[i + 1];
     }
-    __syncthreads();
-    for (int j = w; j < G.m; j += 16) {
+    __syncthreads();  // every boundary is read above before any is rewritten below
+    if (w == 0) {
+        double a = 0.0;
+#pragma unroll 8
+        for (int k = 0; k < kVB; k++) a += ax == 0 ? sv[i][k] : sv[k][i];
+        double total = a;
+#pragma unroll
+        for (int d = kVB / 2; d > 0; d >>= 1) total += __shfl_xor(total, d, kVB);
+        const double before = __shfl_up(a, 1, kVB), after = __shfl_down(a, 1, kVB);
+        const double local = i == 0 ? (a + after) / 2. : i == kVB - 1 ? (a + before) / 2. : (before + a + after) / 3.;
+        const double wgt = total == 0. ? 0. : vegas_weight(total / local);
+        const double nb = vegas_rebin(wgt, lo, hi, i, cum[ax], wt[ax], edge[ax]);
+        if (total != 0.) (ax == 0 ? bt : bp)[i + 1] = nb;
+    }
+    // the integrals: wave w takes q = w - 1, w + 14, ... (wave 0 re-bins meanwhile, and joins
+    // where it is done first)
+    for (int j = w == 0 ? 15 : w - 1; j < G.m; j += 16) {
         const double *bs = binsum + ((size_t)gi * mstride + j) * 1024;
         double c = 0.0;
-        for (int b = lane; b < 1024; b += 64) c += bs[b] * svol[b];
+#pragma unroll
+        for (int k = 0; k < 16; k++) c += bs[lane + 64 * k] * svol[lane + 64 * k];
         c = wave_sum(c);
         if (lane == 0) {
             const int q = G.q0 + j;
@@ -1055,31 +1379,6 @@ __global__ __launch_bounds__(1024) void vegas_reduce(const GroupDev *__restrict_
             if (iter > 0) e = (hist[(size_t)(iter - 1) * nq + q] * (double)iter + e) / (double)(iter + 1);
             hist[(size_t)iter * nq + q] = e;
         }
-    }
-    // every boundary is read above before any is rewritten below
-    if (threadIdx.x < 2 * kVB) {
-        const int ax = threadIdx.x / kVB, i = threadIdx.x % kVB;
-        double a = 0.0;
-        for (int k = 0; k < kVB; k++) a += ax == 0 ? sv[i * kVB + k] : sv[k * kVB + i];
-        marg[ax][i] = a;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        double t = 0.0;
-        for (int i = 0; i < kVB; i++) t += marg[threadIdx.x][i];
-        tot[threadIdx.x] = t;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2 * kVB) {
-        const int ax = threadIdx.x / kVB, i = threadIdx.x % kVB;
-        wgt[ax][i] = tot[ax] == 0. ? 0. : vegas_weight(marg[ax], tot[ax], i);
-    }
-    __syncthreads();
-    if (threadIdx.x < 2 && tot[threadIdx.x] != 0.) vegas_sweep(wgt[threadIdx.x], sb[threadIdx.x], snb[threadIdx.x]);
-    __syncthreads();
-    if (threadIdx.x < 2 * (kVB + 1)) {
-        const int ax = threadIdx.x / (kVB + 1), i = threadIdx.x % (kVB + 1);
-        (ax == 0 ? bt : bp)[i] = sb[ax][i];
     }
 }
 
@@ -1391,6 +1690,25 @@ void launch_mc(bool fp64, bool single, const void *const *grids, const RotDev *r
         mc_reduce<<<nactive, 256, 0, s>>>(groups, active, partial, nblk, mstride, out);
         return;
     }
+    // a single leaf over four chunks or more: by patch (its tile serves every chunk)
+    const long long nchunks = (long long)nblk * 256 / chunk;
+    if (single && nchunks >= 4) {
+        // directions per thread: as many as the chunks fill (a workgroup takes 4 D of them)
+        const int D = nchunks >= 12 ? 4 : nchunks >= 6 ? 2 : 1;
+        const int nset = (int)((nchunks + 4 * D - 1) / (4 * D)), nb = chunk / 64 * nset;  // nb <= nblk
+        const dim3 pg(nb, nactive);
+#define DPLUS_MCP(T, T4, D)                                                                                        \
+    mc_patch_kernel<T, T4, D><<<pg, 256, 0, s>>>((const T4 *const *)grids, rots, groups, active, mstride, qs, step, \
+                                                 seed, dir0, (int)nchunks, chunk, nu, nv, nset, partial)
+        if (fp64) {
+            D == 4 ? (void)DPLUS_MCP(double, double4, 4) : D == 2 ? (void)DPLUS_MCP(double, double4, 2) : (void)DPLUS_MCP(double, double4, 1);
+        } else {
+            D == 4 ? (void)DPLUS_MCP(float, float4, 4) : D == 2 ? (void)DPLUS_MCP(float, float4, 2) : (void)DPLUS_MCP(float, float4, 1);
+        }
+#undef DPLUS_MCP
+        mc_reduce<<<nactive, 256, 0, s>>>(groups, active, partial, nb, mstride, out);
+        return;
+    }
 #define DPLUS_MC(T, T4, S, M)                                                                                      \
     mc_kernel<T, T4, S, M><<<grid, 256, 0, s>>>((const T4 *const *)grids, rots, nrot, trans, groups, active, mstride, \
                                                 qs, step, seed, dir0, nblk, chunk, nu, nv, partial)
@@ -1433,30 +1751,32 @@ void launch_vegas_iter(bool fp64, bool single, const void *const *grids, const R
     int L = 1;
     while (L < ppb && L < 64) L <<= 1;
     dim3 grid(kVB * kVB / (4 * (64 / L)), nactive);
-#define DPLUS_VEGAS(T, T4, KL, S, P)                                                                          \
-    vegas_sample<T, T4, KL, S, P><<<grid, 256, 0, s>>>((const T4 *const *)grids, rots, nrot, trans, groups,      \
-                                                       active, mstride, qs, step, seed, iter, ppb, L, bounds,   \
-                                                       binsum, binvar)
+#define DPLUS_VEGAS(T, T4, KL, S, P, TILED)                                                                   \
+    vegas_sample<T, T4, KL, S, P, TILED><<<grid, 256, 0, s>>>((const T4 *const *)grids, rots, nrot, trans,       \
+                                                              groups, active, mstride, qs, step, seed, iter,    \
+                                                              ppb, L, bounds, binsum, binvar)
     // points per lane: the single-leaf instances are sized to the bin's points
     // (fewer registers), the docked ones take up to kVPts
     const int per_lane = (ppb + L - 1) / L;
-#define DPLUS_VEGAS_P(T, T4, KL)                 \
-    if (!single)                                 \
-        DPLUS_VEGAS(T, T4, KL, false, kVPts);    \
-    else if (per_lane <= 1)                      \
-        DPLUS_VEGAS(T, T4, KL, true, 1);         \
-    else if (per_lane <= 2)                      \
-        DPLUS_VEGAS(T, T4, KL, true, 2);         \
-    else                                         \
-        DPLUS_VEGAS(T, T4, KL, true, kVPts);
-    if (fp64 && L == 64) {
-        DPLUS_VEGAS_P(double, double4, 64)
-    } else if (fp64) {
-        DPLUS_VEGAS_P(double, double4, 0)
-    } else if (L == 64) {
-        DPLUS_VEGAS_P(float, float4, 64)
+#define DPLUS_VEGAS_P(T, T4)                             \
+    if (!single && L == 64)                              \
+        DPLUS_VEGAS(T, T4, 64, false, kVPts, false);     \
+    else if (!single)                                    \
+        DPLUS_VEGAS(T, T4, 0, false, kVPts, false);      \
+    else if (L < 8)                                      \
+        DPLUS_VEGAS(T, T4, 0, true, 1, false);           \
+    else if (L < 64)                                     \
+        DPLUS_VEGAS(T, T4, 0, true, 1, true);            \
+    else if (per_lane <= 1)                              \
+        DPLUS_VEGAS(T, T4, 64, true, 1, true);           \
+    else if (per_lane <= 2)                              \
+        DPLUS_VEGAS(T, T4, 64, true, 2, true);           \
+    else                                                 \
+        DPLUS_VEGAS(T, T4, 64, true, kVPts, true);
+    if (fp64) {
+        DPLUS_VEGAS_P(double, double4)
     } else {
-        DPLUS_VEGAS_P(float, float4, 0)
+        DPLUS_VEGAS_P(float, float4)
     }
 #undef DPLUS_VEGAS_P
 #undef DPLUS_VEGAS
