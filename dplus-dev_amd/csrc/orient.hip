@@ -49,6 +49,116 @@ __device__ __forceinline__ void four_point(const cplx<T> y[4], cplx<T> &d2, cplx
     d3.y = e * (y[1].y - y[0].y) - c * (y[2].y - y[0].y) + b * (y[3].y - y[1].y) - a * (y[3].y - y[2].y);
 }
 
+constexpr double kInvPi = 0.31830988618379067153776752674503;
+constexpr double kInv2Pi = 0.15915494309189533576888376337251;
+
+// theta / pi of cos theta = 2 u - 1.  For FP32 lookups 2 asin(sqrt y) / pi, y = 1 - u, by a
+// polynomial of asin(sqrt y) / sqrt y on [0, 1/2] (9e-14) and sqrt by one Newton step on the
+// FP32 root (1e-14): a cell's fraction stays well below FP32's rounding of it.
+template <typename T>
+__device__ __forceinline__ double polar_fraction(double u) {
+    if (sizeof(T) == 8) return acos(2.0 * u - 1.0) * kInvPi;
+    const bool flip = u < 0.5;
+    const double y = fmax(flip ? u : 1.0 - u, 1e-30);
+    const float s0 = __builtin_amdgcn_sqrtf((float)y);
+    double s = (double)s0;
+    s = fma(fma(-s, s, y), (double)(0.5f * __builtin_amdgcn_rcpf(s0)), s);
+    const double c[14] = {0.6366197723674882,   0.10610329546639952, 0.047746473800039865, 0.02842098102029294,
+                          0.019329935850208507, 0.014425052426250716, 0.009232696985335458, 0.02102495864195202,
+                          -0.048506457009034394, 0.18417602577157377, -0.3818597693281228,  0.5575447279642045,
+                          -0.46861904441904245, 0.19281950697472416};
+    double v = c[13];
+#pragma unroll
+    for (int i = 12; i >= 0; i--) v = fma(v, y, c[i]);
+    return flip ? 1.0 - s * v : s * v;
+}
+
+// phi / 2 pi in [0, 1] of the direction (x, y).  For FP32 lookups atan(t) / 2 pi by a polynomial
+// (3e-14) of t = min / max, the quotient by one Newton step on the FP32 reciprocal.
+template <typename T>
+__device__ __forceinline__ double azimuth_fraction(double y, double x) {
+    if (sizeof(T) == 8) {
+        double ph = atan2(y, x);
+        if (ph < 0.0) ph += k2Pi;
+        return ph * kInv2Pi;
+    }
+    const double ax = fabs(x), ay = fabs(y), mx = fmax(fmax(ax, ay), 1e-30), mn = fmin(ax, ay);
+    double r = (double)__builtin_amdgcn_rcpf((float)mx);
+    r = fma(fma(-mx, r, 1.0), r, r);
+    const double t = mn * r, z = t * t;
+    const double c[15] = {0.15915494309185563,   -0.05305164767892841,  0.03183098720372489,   -0.022736377200679544,
+                          0.017683185381863295,  -0.014461797164107013, 0.012198398114540248,  -0.010409938335242477,
+                          0.008704539505489512,  -0.006766065864383247, 0.004557582911667102,  -0.0024539396615994905,
+                          0.0009607892649646508, -0.0002385112965010332, 2.785172736474061e-05};
+    double v = c[14];
+#pragma unroll
+    for (int i = 13; i >= 0; i--) v = fma(v, z, c[i]);
+    v *= t;
+    v = ay > ax ? 0.25 - v : v;
+    v = x < 0.0 ? 0.5 - v : v;
+    return y < 0.0 ? 1.0 - v : v;
+}
+
+// sin and cos of an angle of FP32 amplitudes' phases: reduced in FP64 to an eighth of a turn
+// and evaluated by polynomials (1e-15 there)
+__device__ __forceinline__ void phase_poly(double angle, double &s, double &c) {
+    const double t = angle * kInv2Pi, k = rint(4.0 * t), r = fma(-0.25, k, t), z = r * r;
+    const double a[7] = {6.283185307179589, -41.34170224040016, 81.60524927661358, -76.70585994242144,
+                         42.05872054224183, -15.096148222634003, 3.8374156880543087};
+    const double b[7] = {1.0000000000000004, -19.73920880217851, 64.93939402246923, -85.45681712812244,
+                         60.24462568572577, -26.424620552027367, 7.818904292222803};
+    double u = a[6], v = b[6];
+#pragma unroll
+    for (int i = 5; i >= 0; i--) {
+        u = fma(u, z, a[i]);
+        v = fma(v, z, b[i]);
+    }
+    u *= r;
+    const int q = (int)(long long)k;
+    s = (q & 1) ? v : u;
+    c = (q & 1) ? u : v;
+    s = (q & 2) ? -s : s;
+    c = ((q + 1) & 2) ? -c : c;
+}
+template <typename T>
+__device__ __forceinline__ void phase_exact(double angle, double &s, double &c) {
+    if (sizeof(T) == 8)
+        sincos(angle, &s, &c);
+    else
+        phase_poly(angle, s, c);
+}
+
+// weights of the 4-point spline (four_point's end derivatives, then the cubic
+// Hermite at t) over values y0..y3, as cubics in t: the spline at t is sum_r w[r] y[r].
+// w[1] = 1 + t (-1/5 + t (-9/5 + t)) closes the sum to 1, so that rounding scales nothing.
+template <typename T>
+__device__ __forceinline__ void spline4_weights(T t, T w[4]) {
+    w[0] = t * ((T)(-7. / 15.) + t * ((T)(4. / 5.) - (T)(1. / 3.) * t));
+    w[2] = t * ((T)(4. / 5.) + t * ((T)(6. / 5.) - t));
+    w[3] = t * ((T)(-2. / 15.) + t * ((T)(-1. / 5.) + (T)(1. / 3.) * t));
+    w[1] = ((T)1 - w[2]) - (w[0] + w[3]);
+}
+
+// the same for a q, whose weights every direction shares: formed in FP64
+template <typename T>
+__device__ __forceinline__ void q_weights(double t, T w[4]) {
+    double v[4];
+    spline4_weights<double>(t, v);
+    w[0] = (T)v[0];
+    w[2] = (T)v[2];
+    w[3] = (T)v[3];
+    w[1] = ((T)1 - w[2]) - (w[0] + w[3]);
+}
+
+// cell and fraction of 0 <= x < 2^31 by FP64 additions (the conversions run at a quarter of
+// their rate): x - 1/2 rounds to the cell in the low mantissa bits of x - 1/2 + 1.5 2^52.  At
+// a node the cell may be the lower one, with fraction 1: the same interpolated value.
+__device__ __forceinline__ double cell_of(double x, int &i) {
+    const double magic = 6755399441055744.0, t = (x - 0.5) + magic;
+    i = (int)(unsigned)__double_as_longlong(t);
+    return x - (t - magic);
+}
+
 // one theta-phi plane (shell >= 1) at theta = ut pi, phi = up 2 pi; kZeroTiny
 // reproduces the CPU variant's snapping of interpolation fractions below 1e-10
 // (Grid.cpp:1242-1245).  The cell and fractions are the reference's
@@ -59,6 +169,43 @@ template <typename T, typename T4, bool kZeroTiny>
 __device__ cplx<T> plane_lookup(const T4 *__restrict__ plane, int shell, double ut, double up) {
     const int phiPoints = 6 * shell, thePoints = 3 * shell;
     const double xt = ut * (double)thePoints, xp = up * (double)phiPoints;
+    if constexpr (sizeof(T) == 4) {
+        // FP32 nodes: the cell by FP64 additions (a node may be its lower cell's upper end) and
+        // the interpolation by weights, half the instructions of the forms below
+        int t0, p0;
+        double ft = cell_of(xt, t0), fp = cell_of(xp, p0);
+        if (t0 < 0) {  // x < 2^-54 may round below the first cell
+            t0 = 0;
+            ft = 0.0;
+        }
+        if (p0 < 0) {
+            p0 = 0;
+            fp = 0.0;
+        }
+        p0 = p0 == phiPoints ? 0 : p0;
+        const int p1 = p0 + 1 == phiPoints ? 0 : p0 + 1;
+        const T p = (T)fp, p2 = p * p, p3 = p2 * p;
+        const T h01 = (T)3 * p2 - (T)2 * p3, h00 = (T)1 - h01, h11 = p3 - p2, h10 = h11 - p2 + p;
+        T w[4];
+        spline4_weights<T>((T)ft, w);
+        cplx<T> a = {(T)0, (T)0};
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            int v = t0 + r - 1, k0 = p0, k1 = p1;  // v in [-1, thePoints + 1]
+            if (v < 0 || v > thePoints) {
+                // past a pole: the row on the other side, half a turn away in phi
+                v = v < 0 ? v + thePoints + 1 : v - (thePoints + 1);
+                k0 += k0 >= thePoints ? -thePoints : thePoints;
+                k1 += k1 >= thePoints ? -thePoints : thePoints;
+            }
+            const T4 A = plane[phiPoints * v + k0], B = plane[phiPoints * v + k1];
+            const T x = h00 * A.x + h01 * B.x + h10 * A.z + h11 * B.z;
+            const T y = h00 * A.y + h01 * B.y + h10 * A.w + h11 * B.w;
+            a.x += w[r] * x;
+            a.y += w[r] * y;
+        }
+        return a;
+    }
     const int tI = (int)xt;
     int pI = (int)xp;
     double tphd = xp - (double)pI;
@@ -93,8 +240,6 @@ __device__ cplx<T> plane_lookup(const T4 *__restrict__ plane, int shell, double 
     return hermite<T>(nn[1], nn[2], d1, d2, tth);
 }
 
-constexpr double kInvPi = 0.31830988618379067153776752674503;
-constexpr double kInv2Pi = 0.15915494309189533576888376337251;
 
 __device__ __forceinline__ void antipode(double th, double ph, double &nth, double &nph) {
     double a = kPi - th, b = ph + kPi;
@@ -126,6 +271,69 @@ __device__ __forceinline__ void group_planes(const T4 *__restrict__ g, int layer
     four_point<T>(amps, d1, d2);
 }
 
+// one plane's lookup out of line, for the rare ones: the origin (layer 0's plane), the antipode
+// on shell 1 (plane -1), directions next to a pole or a row's end, patches larger than a tile
+template <typename T, typename T4>
+__device__ __noinline__ cplx<T> plane_direct(const T4 *__restrict__ g, int lqi, double ut, double up) {
+    if (lqi == 0) {
+        const T4 o = g[0];
+        return {o.x, o.y};
+    }
+    if (lqi < 0) {
+        double nth, nph;
+        antipode(ut * kPi, up * k2Pi, nth, nph);
+        return plane_lookup<T, T4, false>(g + 1, 1, nth * kInvPi, nph * kInv2Pi);
+    }
+    return plane_lookup<T, T4, false>(g + shell_base(lqi), lqi, ut, up);
+}
+
+// the four planes layer - 1 .. layer + 2 at (pi ut, 2 pi up), FP32 nodes.  Where no lane of the
+// wave is next to a pole or at a row's last column (most waves: their directions are
+// neighbours), the eight nodes are four 32-bit offsets from the plane's base, each row's
+// pair one load apart; else plane_lookup's wrapped addresses.
+__device__ __forceinline__ void planes32(const float4 *__restrict__ g, int layer, double ut, double up,
+                                         cplx<float> amps[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int lqi = layer - 1 + i;
+        if (lqi <= 0) {
+            amps[i] = plane_direct<float, float4>(g, lqi, ut, up);
+            continue;
+        }
+        const float4 *plane = g + shell_base(lqi);
+        const int n = 6 * lqi, m = 3 * lqi;
+        int t0, p0;
+        const float t = (float)cell_of(ut * (double)m, t0), p = (float)cell_of(up * (double)n, p0);
+        if (__ballot(t0 < 1 || t0 > m - 2 || p0 < 0 || p0 > n - 2) != 0) {
+            amps[i] = plane_direct<float, float4>(g, lqi, ut, up);
+            continue;
+        }
+        const float p2 = p * p, p3 = p2 * p;
+        const float h01 = 3.f * p2 - 2.f * p3, h00 = 1.f - h01, h11 = p3 - p2, h10 = h11 - p2 + p;
+        float w[4];
+        spline4_weights<float>(t, w);
+        unsigned off = (unsigned)((t0 - 1) * n + p0) * (unsigned)sizeof(float4);
+        const unsigned row = (unsigned)n * (unsigned)sizeof(float4);
+        float4 A[4], B[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++, off += row) {
+            const float4 *q = (const float4 *)((const char *)plane + off);
+            A[r] = q[0];
+            B[r] = q[1];
+        }
+        cplx<float> a = {0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            a.x += w[r] * (h00 * A[r].x + h01 * B[r].x + h10 * A[r].z + h11 * B[r].z);
+            a.y += w[r] * (h00 * A[r].y + h01 * B[r].y + h10 * A[r].w + h11 * B[r].w);
+        }
+        amps[i] = a;
+        // one plane's loads in flight: four planes' would hold 128 registers, and two more waves
+        // per SIMD hide as much
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // R^T q with R = Rx(a) Ry(b) Rz(c): HybridOA.cu:60-63
 __device__ __forceinline__ void rotate_t(const RotDev &r, const double q[3], double o[3]) {
 #pragma unroll
@@ -151,7 +359,12 @@ __device__ __forceinline__ void phase_sincos<double>(double qd, double &s, doubl
 constexpr int kMaxM = 16;  // q-values of one shell group handled per pass (one lookup serves all)
 
 
-// accumulate the docked amplitude along unit direction qv for q-values qs[0..m), m <= M.
+// accumulate the docked amplitude along unit direction qv for q-values qs[0..m), m <= M,
+// (900 copies of two leaves in 120 rotations, 8,192 directions, grid 150: 6.58 -> 5.23 ms with
+// polynomial angles, interpolation weights and the phase sums taken before the amplitudes,
+// which also shortens their rounding: 4.0e-6 -> 7e-7 of I(q); 2,190 VALU instructions a
+// lookup before, at 2 waves per SIMD beside the gathers)
+// whose weights over the four planes are wq (q_weights, in LDS).
 // stepq (equally spaced q, single precision): the translations of a rotation
 // with several step their phases in q, e^{i q_j d} = e^{i q_0 d} (e^{i dq d})^j:
 // two range-reduced sin/cos per translation and one complex rotation per further
@@ -159,53 +372,72 @@ constexpr int kMaxM = 16;  // q-values of one shell group handled per pass (one 
 template <typename T, typename T4, int M = kMaxM>
 __device__ __forceinline__ void docked_amplitude(const T4 *const *__restrict__ grids,
                                                  const RotDev *__restrict__ rots, int nrot,
-                                                 const double4 *__restrict__ trans, int layer,
-                                                 double step, const double qv[3],
-                                                 const double *__restrict__ qs, int m, bool stepq,
+                                                 const double4 *__restrict__ trans, int layer, const double qv[3],
+                                                 const double *__restrict__ qs, const T (*wq)[4], int m, bool stepq,
                                                  cplx<T> acc[M]) {
-    const double inv_step = 1.0 / step;
     const bool rec = sizeof(T) == 4 && stepq && m > 1;
-    const double dq = rec ? (qs[m - 1] - qs[0]) / (double)(m - 1) : 0.0;
+    const double q0t = qs[0] * kInv2Pi, dqt = rec ? (qs[m - 1] - qs[0]) / (double)(m - 1) * kInv2Pi : 0.0;
     for (int r = 0; r < nrot; r++) {
-        const RotDev rd = rots[r];
+        const RotDev &rd = rots[r];
         double rv[3];
         rotate_t(rd, qv, rv);
         if (fabs(rv[2]) > 1.) rv[2] = (rv[2] > 0.) ? 1. : -1.;
-        const double nth = acos(rv[2]);
-        double nph = atan2(rv[1], rv[0]);
-        if (nph < 0.0) nph += k2Pi;
-        cplx<T> amps[4], d1, d2;
-        group_planes<T, T4>(grids[rd.leaf], layer, nth, nph, amps, d1, d2);
+        cplx<T> amps[4];
+        if constexpr (sizeof(T) == 4) {
+            planes32(grids[rd.leaf], layer, polar_fraction<T>(0.5 + 0.5 * rv[2]), azimuth_fraction<T>(rv[1], rv[0]), amps);
+        } else {
+            const double nth = acos(rv[2]);
+            double nph = atan2(rv[1], rv[0]);
+            if (nph < 0.0) nph += k2Pi;
+            cplx<T> d1, d2;
+            group_planes<T, T4>(grids[rd.leaf], layer, nth, nph, amps, d1, d2);
+        }
         const T sc = (T)rd.scale;
-        const bool trivial = (rd.nt == 1) && trans[rd.t0].x == 0.0 && trans[rd.t0].y == 0.0 &&
-                             trans[rd.t0].z == 0.0;
-        if (rec && rd.nt > 1) {
-            cplx<T> a[M];
 #pragma unroll
-            for (int j = 0; j < M; j++) {
-                a[j] = {(T)0, (T)0};
-                if (j < m) {
-                    const T t = (T)((qs[j] - layer * step) * inv_step);
-                    a[j] = hermite<T>(amps[1], amps[2], d1, d2, t);
-                    a[j].x *= sc;
-                    a[j].y *= sc;
-                }
-            }
-            for (int tr = 0; tr < rd.nt; tr++) {
-                const double4 tt = trans[rd.t0 + tr];
+        for (int p = 0; p < 4; p++) {
+            amps[p].x *= sc;
+            amps[p].y *= sc;
+        }
+        // (the weights are read from LDS for every rotation: kept across the loop they would
+        // take 4 M registers)
+        int zero = 0;
+        asm volatile("" : "+v"(zero));
+        auto amplitude = [&](int j) {
+            const T *wj = wq[j + zero];
+            const T w0 = wj[0], w1 = wj[1], w2 = wj[2], w3 = wj[3];
+            return cplx<T>{w0 * amps[0].x + w1 * amps[1].x + w2 * amps[2].x + w3 * amps[3].x,
+                           w0 * amps[0].y + w1 * amps[1].y + w2 * amps[2].y + w3 * amps[3].y};
+        };
+        const int nt = rd.nt, t0 = rd.t0;
+        const bool trivial = nt == 1 && trans[t0].x == 0.0 && trans[t0].y == 0.0 && trans[t0].z == 0.0;
+        if (rec && nt > 1) {
+            // the phases' sums over the translations first, the amplitudes times them once
+            cplx<T> sum[M];
+#pragma unroll
+            for (int j = 0; j < M; j++) sum[j] = {(T)0, (T)0};
+            for (int tr = 0; tr < nt; tr++) {
+                const double4 tt = trans[t0 + tr];
                 const double d = tt.x * qv[0] + tt.y * qv[1] + tt.z * qv[2];
-                T cs, sn, cd, sd;
-                phase_sincos<T>(qs[0] * d, sn, cs);
-                phase_sincos<T>(dq * d, sd, cd);
+                const float f = (float)__builtin_amdgcn_fract(q0t * d), e = (float)__builtin_amdgcn_fract(dqt * d);
+                T cs = __builtin_amdgcn_cosf(f), sn = __builtin_amdgcn_sinf(f);
+                const T cd = __builtin_amdgcn_cosf(e), sd = __builtin_amdgcn_sinf(e);
 #pragma unroll
                 for (int j = 0; j < M; j++) {
                     if (j < m) {
-                        acc[j].x += a[j].x * cs - a[j].y * sn;
-                        acc[j].y += a[j].y * cs + a[j].x * sn;
+                        sum[j].x += cs;
+                        sum[j].y += sn;
                         const T c2 = cs * cd - sn * sd;
                         sn = sn * cd + cs * sd;
                         cs = c2;
                     }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < M; j++) {
+                if (j < m) {
+                    const cplx<T> a = amplitude(j);
+                    acc[j].x += a.x * sum[j].x - a.y * sum[j].y;
+                    acc[j].y += a.y * sum[j].x + a.x * sum[j].y;
                 }
             }
             continue;
@@ -213,46 +445,24 @@ __device__ __forceinline__ void docked_amplitude(const T4 *const *__restrict__ g
 #pragma unroll
         for (int j = 0; j < M; j++) {
             if (j < m) {
-                const T t = (T)((qs[j] - layer * step) * inv_step);
-                cplx<T> a = hermite<T>(amps[1], amps[2], d1, d2, t);
+                const cplx<T> a = amplitude(j);
                 if (trivial) {
-                    acc[j].x += a.x * sc;
-                    acc[j].y += a.y * sc;
+                    acc[j].x += a.x;
+                    acc[j].y += a.y;
                 } else {
                     T sumc = 0, sums = 0;
-                    for (int tr = 0; tr < rd.nt; tr++) {
-                        const double4 tt = trans[rd.t0 + tr];
+                    for (int tr = 0; tr < nt; tr++) {
+                        const double4 tt = trans[t0 + tr];
                         const double qd = qs[j] * (tt.x * qv[0] + tt.y * qv[1] + tt.z * qv[2]);
                         T s, c;
                         phase_sincos<T>(qd, s, c);
                         sumc += c;
                         sums += s;
                     }
-                    acc[j].x += (a.x * sumc - a.y * sums) * sc;
-                    acc[j].y += (a.y * sumc + a.x * sums) * sc;
+                    acc[j].x += a.x * sumc - a.y * sums;
+                    acc[j].y += a.y * sumc + a.x * sums;
                 }
             }
-        }
-    }
-}
-
-// the same for one leaf placed once, unrotated, at the origin: the lookup takes
-// the direction's angles as drawn (no rotation back to angles, no translation
-// phases), a = scale * A(q, theta, phi)
-template <typename T, typename T4, int M = kMaxM>
-__device__ __forceinline__ void single_amplitude(const T4 *__restrict__ grid, T sc, int layer, double step,
-                                                 double th, double ph, const double *__restrict__ qs, int m,
-                                                 cplx<T> acc[M]) {
-    const double inv_step = 1.0 / step;
-    cplx<T> amps[4], d1, d2;
-    group_planes<T, T4>(grid, layer, th, ph, amps, d1, d2);
-#pragma unroll
-    for (int j = 0; j < M; j++) {
-        if (j < m) {
-            const T t = (T)((qs[j] - layer * step) * inv_step);
-            cplx<T> a = hermite<T>(amps[1], amps[2], d1, d2, t);
-            acc[j].x += a.x * sc;
-            acc[j].y += a.y * sc;
         }
     }
 }
@@ -292,6 +502,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 1 : 2) void mc_kernel(const T
         qv[2] = ct;
     }
     __shared__ double red[4][kMaxM];
+    __shared__ T wq[kMaxM][4];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (kSingle) {
         // one lookup per direction serves every q of the group, each q reduced as it is formed
@@ -325,11 +536,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 1 : 2) void mc_kernel(const T
     // docked: M q per pass (8 when no group holds more: fewer accumulators)
     for (int jb = 0; jb < G.m; jb += M) {
         const int m = min(M, G.m - jb);
+        __syncthreads();
+        if (threadIdx.x < m) q_weights<T>((qs[G.q0 + jb + threadIdx.x] - G.layer * step) * (1.0 / step), wq[threadIdx.x]);
+        __syncthreads();
         cplx<T> acc[M];
 #pragma unroll
         for (int j = 0; j < M; j++) acc[j] = {(T)0, (T)0};
-        docked_amplitude<T, T4, M>(grids, rots, nrot, trans, G.layer, step, qv, qs + G.q0 + jb, m, G.uniform != 0,
-                                   acc);
+        docked_amplitude<T, T4, M>(grids, rots, nrot, trans, G.layer, qv, qs + G.q0 + jb, wq, m, G.uniform != 0, acc);
 #pragma unroll
         for (int j = 0; j < M; j++) {
             double I = (double)acc[j].x * (double)acc[j].x + (double)acc[j].y * (double)acc[j].y;
@@ -367,28 +580,6 @@ __device__ __forceinline__ float wave_total(float v) {
            (__int_as_float(__builtin_amdgcn_readlane(b, 32)) + __int_as_float(__builtin_amdgcn_readlane(b, 48)));
 }
 __device__ __forceinline__ double wave_total(double v) { return wave_sum(v); }
-
-// weights of the 4-point spline (four_point's end derivatives, then the cubic
-// Hermite at t) over values y0..y3, as cubics in t: the spline at t is sum_r w[r] y[r].
-// w[1] = 1 + t (-1/5 + t (-9/5 + t)) closes the sum to 1, so that rounding scales nothing.
-template <typename T>
-__device__ __forceinline__ void spline4_weights(T t, T w[4]) {
-    w[0] = t * ((T)(-7. / 15.) + t * ((T)(4. / 5.) - (T)(1. / 3.) * t));
-    w[2] = t * ((T)(4. / 5.) + t * ((T)(6. / 5.) - t));
-    w[3] = t * ((T)(-2. / 15.) + t * ((T)(-1. / 5.) + (T)(1. / 3.) * t));
-    w[1] = ((T)1 - w[2]) - (w[0] + w[3]);
-}
-
-// the same for a q, whose weights every direction shares: formed in FP64
-template <typename T>
-__device__ __forceinline__ void q_weights(double t, T w[4]) {
-    double v[4];
-    spline4_weights<double>(t, v);
-    w[0] = (T)v[0];
-    w[2] = (T)v[2];
-    w[3] = (T)v[3];
-    w[1] = ((T)1 - w[2]) - (w[0] + w[3]);
-}
 
 // the four planes' amplitudes (layer - 1 .. layer + 2) of one lookup at (th, ph),
 // as group_planes takes them, without the q derivatives
@@ -489,15 +680,6 @@ __device__ __forceinline__ void stage_tile(const T4 *__restrict__ plane, int she
     }
 }
 
-// cell and fraction of 0 <= x < 2^31 by FP64 additions (the conversions run at a quarter of
-// their rate): x - 1/2 rounds to the cell in the low mantissa bits of x - 1/2 + 1.5 2^52.  At
-// a node the cell may be the lower one, with fraction 1: the same interpolated value.
-__device__ __forceinline__ double cell_of(double x, int &i) {
-    const double magic = 6755399441055744.0, t = (x - 0.5) + magic;
-    i = (int)(unsigned)__double_as_longlong(t);
-    return x - (t - magic);
-}
-
 // plane_lookup on a staged tile, as sums over the nodes with the phi Hermite's and the
 // theta spline's weights
 template <typename T, typename T4>
@@ -519,22 +701,6 @@ __device__ __forceinline__ cplx<T> tile_lookup(const T4 *tile, const Tile &t, in
         a.y += w[r] * y;
     }
     return a;
-}
-
-// one plane's lookup from the grid, for what has no tile: the origin (layer 0's plane), the
-// antipode on shell 1 (plane -1), patches larger than the tile
-template <typename T, typename T4>
-__device__ __noinline__ cplx<T> plane_direct(const T4 *__restrict__ g, int lqi, double ut, double up) {
-    if (lqi == 0) {
-        const T4 o = g[0];
-        return {o.x, o.y};
-    }
-    if (lqi < 0) {
-        double nth, nph;
-        antipode(ut * kPi, up * k2Pi, nth, nph);
-        return plane_lookup<T, T4, false>(g + 1, 1, nth * kInvPi, nph * kInv2Pi);
-    }
-    return plane_lookup<T, T4, false>(g + shell_base(lqi), lqi, ut, up);
 }
 
 // the planes' tiles of a patch: lane p of every four works out plane p's (shell0 + p), then
@@ -572,27 +738,6 @@ __device__ __forceinline__ double group_sums(const double (&v)[M], int lane, int
 template <typename T4>
 constexpr int tile_nodes() {
     return 38 * 1024 / (int)sizeof(T4);
-}
-
-// theta / pi of cos theta = 2 u - 1.  For FP32 lookups 2 asin(sqrt y) / pi, y = 1 - u, by a
-// polynomial of asin(sqrt y) / sqrt y on [0, 1/2] (9e-14) and sqrt by one Newton step on the
-// FP32 root (1e-14): a cell's fraction stays well below FP32's rounding of it.
-template <typename T>
-__device__ __forceinline__ double polar_fraction(double u) {
-    if (sizeof(T) == 8) return acos(2.0 * u - 1.0) * kInvPi;
-    const bool flip = u < 0.5;
-    const double y = fmax(flip ? u : 1.0 - u, 1e-30);
-    const float s0 = __builtin_amdgcn_sqrtf((float)y);
-    double s = (double)s0;
-    s = fma(fma(-s, s, y), (double)(0.5f * __builtin_amdgcn_rcpf(s0)), s);
-    const double c[14] = {0.6366197723674882,   0.10610329546639952, 0.047746473800039865, 0.02842098102029294,
-                          0.019329935850208507, 0.014425052426250716, 0.009232696985335458, 0.02102495864195202,
-                          -0.048506457009034394, 0.18417602577157377, -0.3818597693281228,  0.5575447279642045,
-                          -0.46861904441904245, 0.19281950697472416};
-    double v = c[13];
-#pragma unroll
-    for (int i = 12; i >= 0; i--) v = fma(v, y, c[i]);
-    return flip ? 1.0 - s * v : s * v;
 }
 
 // The MC average of a single leaf over several chunks: a workgroup takes one patch of
@@ -1170,7 +1315,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(cons
     // results kept by selection.
     cplx<T> hold[kP][4];
     __shared__ T4 tile[kTiled ? tile_nodes<T4>() : 1];
-    __shared__ T wq[kSingle ? kVM : 1][4];
+    __shared__ T wq[kVM][4];
     if (kSingle) {
         const T4 *grid = grids[rots[0].leaf];
         const int nb = 256 / L, b0 = blockIdx.x * nb, r0 = b0 / kVB, q0 = b0 % kVB;
@@ -1213,17 +1358,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(cons
         double e[kVM];
 #pragma unroll
         for (int j = 0; j < kVM; j++) e[j] = 0.0;
+        // the q's weights over the planes, shared by every point
+        __syncthreads();
+        if (threadIdx.x < m) q_weights<T>((qs[G.q0 + jb + threadIdx.x] - G.layer * step) * (1.0 / step), wq[threadIdx.x]);
+        __syncthreads();
         if (kSingle) {
-            // the q's weights over the planes, shared by every point
             const double sc2 = (double)(T)rots[0].scale * (double)(T)rots[0].scale;
-            __syncthreads();
-            if (threadIdx.x < m) {
-                T w4[4];
-                q_weights<T>((qs[G.q0 + jb + threadIdx.x] - G.layer * step) * (1.0 / step), w4);
-#pragma unroll
-                for (int p = 0; p < 4; p++) wq[threadIdx.x][p] = w4[p];
-            }
-            __syncthreads();
 #pragma unroll
             for (int j = 0; j < kVM; j++) {
                 if (j >= m) continue;
@@ -1245,7 +1385,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void vegas_sample(cons
                 cplx<T> acc[kVM];
 #pragma unroll
                 for (int j = 0; j < kVM; j++) acc[j] = {(T)0, (T)0};
-                docked_amplitude<T, T4, kVM>(grids, rots, nrot, trans, G.layer, step, qv[k], qs + G.q0 + jb, m,
+                docked_amplitude<T, T4, kVM>(grids, rots, nrot, trans, G.layer, qv[k], qs + G.q0 + jb, wq, m,
                                              G.uniform != 0, acc);
 #pragma unroll
                 for (int j = 0; j < kVM; j++) {
@@ -1385,8 +1525,8 @@ __global__ __launch_bounds__(1024) void vegas_reduce(const GroupDev *__restrict_
 // ------------------------------------------------------------------ single points
 // GetSphr (Grid.cpp:487-548): the CPU-path lookup used by getAmplitude and GK
 template <typename T, typename T4>
-__device__ __forceinline__ cplx<T> get_sphr(const T4 *__restrict__ g, int N, double step, double rr, double th,
-                            double ph) {
+__device__ __forceinline__ cplx<T> get_sphr(const T4 *__restrict__ g, int N, double step, double rr, double ut,
+                                            double up) {  // theta = pi ut, phi = 2 pi up
     const T4 o = g[0];
     if (rr == 0.0) return {o.x, o.y};
     double frc = rr / step;
@@ -1394,13 +1534,12 @@ __device__ __forceinline__ cplx<T> get_sphr(const T4 *__restrict__ g, int N, dou
     const int fInd = (int)frc;
     const double frac = frc - (double)fInd;
     cplx<T> p[4];
-    const double ut = th * kInvPi, up = ph * kInv2Pi;
     p[1] = fInd > 0 ? plane_lookup<T, T4, true>(g + shell_base(fInd), fInd, ut, up) : cplx<T>{o.x, o.y};
     if (frac < 1.e-9) return p[1];
     p[2] = plane_lookup<T, T4, true>(g + shell_base(fInd + 1), fInd + 1, ut, up);
     if (fInd == 0) {
         double nth, nph;
-        antipode(th, ph, nth, nph);
+        antipode(ut * kPi, up * k2Pi, nth, nph);
         p[0] = plane_lookup<T, T4, true>(g + 1, 1, nth * kInvPi, nph * kInv2Pi);
     } else if (fInd == 1) {
         p[0] = {o.x, o.y};
@@ -1420,10 +1559,22 @@ __device__ __forceinline__ cplx<T> get_cart(const T4 *__restrict__ g, int N, dou
     double r = sqrt(x * x + y * y + z * z);
     if (fabs(z) > r) r = fabs(z);
     if (r == 0.0) return get_sphr<T, T4>(g, N, step, 0.0, 0.0, 0.0);
+    if constexpr (sizeof(T) == 4)
+        return get_sphr<T, T4>(g, N, step, r, polar_fraction<T>(0.5 + 0.5 * (z / r)), azimuth_fraction<T>(y, x));
     const double th = acos(z / r);
     double ph = atan2(y, x);
     if (ph < 0.0) ph += k2Pi;
-    return get_sphr<T, T4>(g, N, step, r, th, ph);
+    return get_sphr<T, T4>(g, N, step, r, th * kInvPi, ph * kInv2Pi);
+}
+
+// the same for a point of known norm r > 0 (a rotated node or sample), rinv = 1 / r
+template <typename T, typename T4>
+__device__ __forceinline__ cplx<T> get_turned(const T4 *__restrict__ g, int N, double step, const double v[3], double r,
+                                              double rinv) {
+    if constexpr (sizeof(T) == 4)
+        return get_sphr<T, T4>(g, N, step, r, polar_fraction<T>(0.5 + 0.5 * (v[2] * rinv)),
+                               azimuth_fraction<T>(v[1], v[0]));
+    return get_cart<T, T4>(g, N, step, v[0], v[1], v[2]);
 }
 
 // batch GetSphr at (q, theta, phi) triples
@@ -1433,7 +1584,7 @@ __global__ __launch_bounds__(256) void sphr_batch(const T4 *__restrict__ g, int 
                            const double *__restrict__ ph, double2 *__restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    cplx<T> a = get_sphr<T, T4>(g, N, step, q[i], th[i], ph[i]);
+    cplx<T> a = get_sphr<T, T4>(g, N, step, q[i], th[i] * kInvPi, ph[i] * kInv2Pi);
     out[i] = make_double2((double)a.x, (double)a.y);
 }
 
@@ -1474,17 +1625,19 @@ __device__ double docked_intensity(const T4 *const *__restrict__ grids, const Le
                                    const RotDev *__restrict__ rots, int nrot, const double4 *__restrict__ trans,
                                    const double q[3]) {
     double ax = 0.0, ay = 0.0;
+    const double n = sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]), ninv = 1.0 / n;
     for (int r = 0; r < nrot; r++) {
         const RotDev rd = rots[r];
         double rv[3];
         rotate_t(rd, q, rv);
         const LeafGeo G = geo[rd.leaf];
-        cplx<T> a = get_cart<T, T4>(grids[rd.leaf], G.N, G.step, rv[0], rv[1], rv[2]);
+        const cplx<T> a = n > 0.0 ? get_turned<T, T4>(grids[rd.leaf], G.N, G.step, rv, n, ninv)
+                                  : get_sphr<T, T4>(grids[rd.leaf], G.N, G.step, 0.0, 0.0, 0.0);
         double sc = 0.0, ss = 0.0;
         for (int tr = 0; tr < rd.nt; tr++) {
             const double4 t = trans[rd.t0 + tr];
-            double s, c;
-            sincos(q[0] * t.x + q[1] * t.y + q[2] * t.z, &s, &c);
+            double s = 0.0, c = 1.0;
+            if (t.x != 0.0 || t.y != 0.0 || t.z != 0.0) phase_exact<T>(q[0] * t.x + q[1] * t.y + q[2] * t.z, s, c);
             sc += c;
             ss += s;
         }
@@ -1868,6 +2021,8 @@ __device__ __forceinline__ void node_indices(long long index, int &qi, long long
     pi = rem % (6 * q);
 }
 
+// (13 copies, grid 150: 700 -> 500 us with the polynomial angles and phases of FP32 grids and
+// the node's norm known; VALU-bound at 385 instructions a lookup)
 // ManualSymmetry::calcAmplitude (Symmetries.cpp:697-716) at every node of the
 // output grid (Grid.cpp:760-826 node vectors), sub-amplitudes through GetCart
 // Space-filling lattice sum sum_{n<N} e^{i n d} = e^{i(N-1)d/2} sin(Nd/2)/sin(d/2)
@@ -1920,17 +2075,19 @@ __global__ __launch_bounds__(256) void dock_grid_kernel(const T4 *const *__restr
         q[2] = qI * ct;
     }
     double ax = 0.0, ay = 0.0;
+    const double n = (double)qi * step_out, ninv = 1.0 / n;  // a node's norm, turned or not
     for (int r = 0; r < nrot; r++) {
         const RotDev rd = rots[r];
         double rv[3];
         rotate_t(rd, q, rv);
         const LeafGeo G = geo[rd.leaf];
-        cplx<T> a = get_cart<T, T4>(grids[rd.leaf], G.N, G.step, rv[0], rv[1], rv[2]);
+        const cplx<T> a = n > 0.0 ? get_turned<T, T4>(grids[rd.leaf], G.N, G.step, rv, n, ninv)
+                                  : get_sphr<T, T4>(grids[rd.leaf], G.N, G.step, 0.0, 0.0, 0.0);
         double sc = 0.0, ss = 0.0;
         for (int tr = 0; tr < rd.nt; tr++) {
             const double4 t = trans[rd.t0 + tr];
-            double s, c;
-            sincos(q[0] * t.x + q[1] * t.y + q[2] * t.z, &s, &c);
+            double s = 0.0, c = 1.0;
+            if (t.x != 0.0 || t.y != 0.0 || t.z != 0.0) phase_exact<T>(q[0] * t.x + q[1] * t.y + q[2] * t.z, s, c);
             sc += c;
             ss += s;
         }
