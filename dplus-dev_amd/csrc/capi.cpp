@@ -1033,7 +1033,7 @@ bool z_copies(const RotDev *rots, int nrot, const double4 *tr, std::vector<ZCopy
         if (a >= 2.0 * kPi) a = 0.0;
         for (int t = 0; t < rots[r].nt; t++) {
             const double4 v = tr[rots[r].t0 + t];
-            zc.push_back(ZCopyDev{a, {v.x, v.y, v.z}, rots[r].scale, rots[r].leaf, 0});
+            zc.push_back(ZCopyDev{a, {v.x, v.y, v.z}, rots[r].scale, rots[r].leaf, 0, 0, 0});
         }
     }
     std::stable_sort(zc.begin(), zc.end(), [](const ZCopyDev &x, const ZCopyDev &y) {
@@ -1051,6 +1051,8 @@ bool z_copies(const RotDev *rots, int nrot, const double4 *tr, std::vector<ZCopy
         const double da = zc[last].alpha - zc[c0].alpha;
         if (da > 0.0) lfit = std::min(lfit, std::floor(60.0 * 2.0 * kPi / (6.0 * da)));
     }
+    for (int i = (int)zc.size() - 1; i >= 0; i--)
+        zc[i].run = i + 1 < (int)zc.size() && zc[i + 1].leaf == zc[i].leaf ? zc[i + 1].run : i + 1;
     if (!zc.empty()) zc[0].aux = (int)std::min(lfit, 1e9);
     out.swap(zc);
     return true;

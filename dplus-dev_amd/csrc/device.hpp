@@ -176,6 +176,7 @@ struct ZCopyDev {
     double t[3];
     double scale;
     int leaf, aux;
+    int run, pad;  // one past the last record of the same leaf
 };
 
 // the copies of rotation records that all turn about z alone, one per

@@ -837,6 +837,18 @@ __global__ __launch_bounds__(256) void mc_patch_kernel(const T4 *const *__restri
     }
 }
 
+constexpr int kRowNodes = 2560;
+
+__device__ __forceinline__ int row_nodes(int layer) {  // four rows, each with its first node again at its end
+    int n = 0;
+#pragma unroll
+    for (int p = 0; p < 4; p++) n += 6 * max(layer - 1 + p, 1) + 1;
+    return n;
+}
+__device__ __forceinline__ bool whole_rows(int layer, int nz) {
+    return 2 * nz >= 5 * (layer + 2) && row_nodes(layer) <= kRowNodes;
+}
+
 constexpr int kZWin = 64;  // nodes of one plane's collapsed row segment (one per lane)
 
 // The MC average of a docking whose copies all turn about z (a helix): every
@@ -865,6 +877,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void mc_zcopy_kernel(
     const GroupDev G = groups[active[gi]];
     // split: the collapse instance takes the shell groups whose planes (up to
     // shell layer + 2) fit the window, the direct instance the others
+    // (mc_zrows_kernel takes those with many copies for their rows)
+    if (split && whole_rows(G.layer, nz)) return;
     const bool collapse_group = G.layer + 2 <= zc[0].aux;
     if (kCollapse ? !collapse_group : (split && collapse_group)) return;
     const long long d = dir0 + (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1068,6 +1082,188 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) void mc_zcopy_kernel(
                 red[0][j] + red[1][j] + red[2][j] + red[3][j];
         }
         __syncthreads();
+    }
+}
+
+// group_sums for FP32: the sum over the wave of value lane / (64 / M)
+template <int M>
+__device__ __forceinline__ float wave_sums(const float (&v)[M], int lane, int o = 32) {
+    if constexpr (M > 1) {
+        const bool hi = lane & o;
+        float u[M / 2];
+#pragma unroll
+        for (int i = 0; i < M / 2; i++) {
+            const float send = hi ? v[i] : v[i + M / 2], keep = hi ? v[i + M / 2] : v[i];
+            u[i] = keep + __shfl_xor(send, o, 64);
+        }
+        return wave_sums<M / 2>(u, lane, o >> 1);
+    } else {
+        float t = v[0];
+        for (; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+        return t;
+    }
+}
+
+// The same average where the copies are many for the rows' length: every chunk of 64 copies of
+// mc_zcopy_kernel collapses its own segment, and together they collapse each node several
+// times.  Here a workgroup takes one direction at a time: its 256 threads apply the theta
+// spline to the four planes' whole rows (coalesced, the row numbers and weights
+// wave-uniform) into LDS, then a thread per copy takes two collapsed nodes per plane, the q
+// weights and its translation's phases.  Both halves run without a chain from one chunk to
+// the next.  Two barriers a direction; three workgroups per CU cover them.
+// 1,000 copies, grid 200, 800 q, 65,536 directions: 158.9 -> 79.5 ms, the VALU full (about
+// 460 instructions per 64 copies: 110 for the planes, 210 for eight q and their phases, 70
+// for the rows).
+// Taken where the rows fit (kRowNodes) and copies >= 2.5 shells: the rows cost 4 * 6 shell
+// / 64 collapses of 35 instructions, a chunk of 64 copies 340 here and 684 there, equal
+// near 2.4 copies per shell.
+template <int M>
+__global__ __launch_bounds__(256, M <= 8 ? 3 : 2) void mc_zrows_kernel(
+    const float4 *const *__restrict__ grids, const ZCopyDev *__restrict__ zc, int nz, const GroupDev
+    *__restrict__ groups, const int *__restrict__ active, int mstride, const double *__restrict__ qs, double
+    step, uint64_t seed, long long dir0, int nblk, int chunk, int nu, int nv, double *__restrict__ partial) {
+    const int gi = blockIdx.y;
+    const GroupDev G = groups[active[gi]];
+    if (!whole_rows(G.layer, nz)) return;
+    __shared__ float4 rows[kRowNodes];
+    __shared__ double dirs[5][256];
+    __shared__ float wq[M][4];
+    __shared__ double qt[M];
+    __shared__ float red[4][2 * M];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    {
+        const long long d = dir0 + (long long)blockIdx.x * blockDim.x + threadIdx.x;
+        double u, v;
+        uniform_pair(seed, (uint32_t)d, (uint32_t)(d >> 32), (uint32_t)G.layer, kStreamMC, u, v);
+        mc_stratify(d, chunk, nu, nv, u, v);
+        const double th = acos(2.0 * u - 1.0), ph = k2Pi * v;
+        double st, ct, sp, cp;
+        sincos(th, &st, &ct);
+        sincos(ph, &sp, &cp);
+        dirs[0][threadIdx.x] = th * kInvPi;
+        dirs[1][threadIdx.x] = ph;
+        dirs[2][threadIdx.x] = cp * st;
+        dirs[3][threadIdx.x] = sp * st;
+        dirs[4][threadIdx.x] = ct;
+    }
+    int n[4], base[4];
+    {
+        int b = 0;
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            n[p] = 6 * max(G.layer - 1 + p, 1);
+            base[p] = b;
+            b += n[p] + 1;
+        }
+    }
+    for (int jb = 0; jb < G.m; jb += M) {
+        const int m = min(M, G.m - jb);
+        const double *q = qs + G.q0 + jb;
+        __syncthreads();
+        if (threadIdx.x < M) {
+            if (threadIdx.x < m) q_weights<float>((q[threadIdx.x] - G.layer * step) * (1.0 / step), wq[threadIdx.x]);
+            qt[threadIdx.x] = threadIdx.x < m ? q[threadIdx.x] * kInv2Pi : 0.0;
+        }
+        __syncthreads();
+        double mine = 0.0;  // thread j < m: the sum over the directions of |A_j|^2
+        for (int i = 0; i < 256; i++) {
+            const double phi = dirs[1][i];
+            // lane p of every four: plane p's row and theta weights (the antipode's for plane -1)
+            int t0;
+            float wt[4];
+            {
+                const int p = lane & 3, lqi = G.layer - 1 + p;
+                const double ut = lqi < 0 ? 1.0 - dirs[0][i] : dirs[0][i];
+                spline4_weights<float>((float)cell_of(ut * (double)(3 * max(lqi, 1)), t0), wt);
+                t0 = max(t0, 0);
+            }
+            float acc[2 * M];
+#pragma unroll
+            for (int j = 0; j < 2 * M; j++) acc[j] = 0.f;
+            for (int k0 = 0, k1; k0 < nz; k0 = k1) {
+                k1 = zc[k0].run;
+                const float4 *g0 = grids[zc[k0].leaf];
+                if (k0 > 0) __syncthreads();  // the previous leaf's copies are done with the rows
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const int lqi = G.layer - 1 + p;
+                    if (lqi == 0) continue;
+                    const int half = n[p] >> 1, tp = __builtin_amdgcn_readlane(t0, p);
+                    float wp[4];
+                    const float4 *row[4];
+                    bool past[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        wp[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wt[r]), p));
+                        int v = tp + r - 1;
+                        past[r] = v < 0 || v > half;  // past a pole: the other side's row, half a turn away
+                        if (past[r]) v = v < 0 ? v + half + 1 : v - (half + 1);
+                        row[r] = g0 + shell_base(max(lqi, 1)) + v * n[p];
+                    }
+                    for (int k = threadIdx.x; k < n[p]; k += 256) {
+                        const int kh = k >= half ? k - half : k + half;
+                        float4 a[4];
+#pragma unroll
+                        for (int r = 0; r < 4; r++) a[r] = row[r][past[r] ? kh : k];
+                        float4 c;
+                        c.x = wp[0] * a[0].x + wp[1] * a[1].x + wp[2] * a[2].x + wp[3] * a[3].x;
+                        c.y = wp[0] * a[0].y + wp[1] * a[1].y + wp[2] * a[2].y + wp[3] * a[3].y;
+                        c.z = wp[0] * a[0].z + wp[1] * a[1].z + wp[2] * a[2].z + wp[3] * a[3].z;
+                        c.w = wp[0] * a[0].w + wp[1] * a[1].w + wp[2] * a[2].w + wp[3] * a[3].w;
+                        rows[base[p] + k] = c;
+                        if (k == 0) rows[base[p] + n[p]] = c;
+                    }
+                }
+                __syncthreads();
+                for (int k = k0 + threadIdx.x; k < k1; k += 256) {
+                    const ZCopyDev z = zc[k];
+                    double up = (phi - z.alpha) * kInv2Pi;
+                    up += up < 0.0 ? 1.0 : 0.0;
+                    const float sc = (float)z.scale;
+                    cplx<float> amps[4];
+#pragma unroll
+                    for (int p = 0; p < 4; p++) {
+                        const int lqi = G.layer - 1 + p;
+                        if (lqi == 0) {
+                            const float4 o = g0[0];
+                            amps[p] = {o.x * sc, o.y * sc};
+                            continue;
+                        }
+                        const double u = lqi < 0 ? (up >= 0.5 ? up - 0.5 : up + 0.5) : up;
+                        int c;
+                        const float t = (float)cell_of(u * (double)n[p], c);
+                        c = min(max(c, 0), n[p] - 1);
+                        const float4 A = rows[base[p] + c], B = rows[base[p] + c + 1];
+                        const float t2 = t * t, t3 = t2 * t;
+                        const float h01 = 3.f * t2 - 2.f * t3, h00 = 1.f - h01, h11 = t3 - t2, h10 = h11 - t2 + t;
+                        amps[p] = {sc * (h00 * A.x + h01 * B.x + h10 * A.z + h11 * B.z),
+                                   sc * (h00 * A.y + h01 * B.y + h10 * A.w + h11 * B.w)};
+                    }
+                    const double dot = z.t[0] * dirs[2][i] + z.t[1] * dirs[3][i] + z.t[2] * dirs[4][i];
+#pragma unroll
+                    for (int j = 0; j < M; j++) {
+                        if (j < m) {
+                            const float ax = wq[j][0] * amps[0].x + wq[j][1] * amps[1].x + wq[j][2] * amps[2].x + wq[j][3] * amps[3].x;
+                            const float ay = wq[j][0] * amps[0].y + wq[j][1] * amps[1].y + wq[j][2] * amps[2].y + wq[j][3] * amps[3].y;
+                            const float f = (float)__builtin_amdgcn_fract(qt[j] * dot);
+                            const float s = __builtin_amdgcn_sinf(f), co = __builtin_amdgcn_cosf(f);
+                            acc[j] += ax * co - ay * s;
+                            acc[M + j] += ay * co + ax * s;
+                        }
+                    }
+                }
+            }
+            const float t = wave_sums<2 * M>(acc, lane);
+            if (lane % (64 / (2 * M)) == 0) red[w][lane / (64 / (2 * M))] = t;
+            __syncthreads();
+            if (threadIdx.x < m) {
+                const int j = threadIdx.x;
+                const double ax = ((double)red[0][j] + (double)red[1][j]) + ((double)red[2][j] + (double)red[3][j]);
+                const double ay = ((double)red[0][M + j] + (double)red[1][M + j]) + ((double)red[2][M + j] + (double)red[3][M + j]);
+                mine += ax * ax + ay * ay;
+            }
+        }
+        if (threadIdx.x < m) partial[((size_t)gi * nblk + blockIdx.x) * mstride + jb + threadIdx.x] = mine;
     }
 }
 
@@ -1460,7 +1656,7 @@ __device__ __forceinline__ double vegas_rebin(double w, double lo, double hi, in
 }
 
 // one block (1024 threads = the 32x32 bins) per active group: the iteration's
-// integral sum_bins vol * mean_bin(I_j) (wave w takes q = w, w + 16, ...), the
+// integral sum_bins vol * mean_bin(I_j) (q dealt over waves 1 to 15 first), the
 // theta/phi marginals of the bin variances, re-binning, and the running mean over iterations
 // (HybridVEGASResizeGridKernel; GPUHybridCalc.cu:654-701).  The re-binning runs on one wave,
 // an axis per half wave, by scans and a binary search: 16.5 -> 5.8 us an iteration (its 64
@@ -1505,7 +1701,7 @@ __global__ __launch_bounds__(1024) void vegas_reduce(const GroupDev *__restrict_
         const double nb = vegas_rebin(wgt, lo, hi, i, cum[ax], wt[ax], edge[ax]);
         if (total != 0.) (ax == 0 ? bt : bp)[i + 1] = nb;
     }
-    // the integrals: wave w takes q = w - 1, w + 14, ... (wave 0 re-bins meanwhile, and joins
+    // the integrals: wave w takes q = w - 1, w + 15, ... (wave 0 re-bins meanwhile, and joins
     // where it is done first)
     for (int j = w == 0 ? 15 : w - 1; j < G.m; j += 16) {
         const double *bs = binsum + ((size_t)gi * mstride + j) * 1024;
@@ -1823,8 +2019,8 @@ void launch_mc(bool fp64, bool single, const void *const *grids, const RotDev *r
     mc_strata(chunk, nu, nv);
     if (!single && zc && nz >= kZCopyMin) {
         // 8 q per pass when no shell group holds more (fewer accumulators);
-        // FP32 grids: the collapse instance and the direct one over the same
-        // grid, each block running in one of them
+        // FP32 grids: the whole-row kernel, the collapse instance and the direct one over the
+        // same grid, each block running in one of them
 #define DPLUS_MCZ(T, T4, C, M, SPLIT)                                                                             \
     mc_zcopy_kernel<T, T4, C, M><<<grid, 256, 0, s>>>((const T4 *const *)grids, zc, nz, groups, active, mstride, \
                                                       qs, step, seed, dir0, nblk, chunk, nu, nv, SPLIT, partial)
@@ -1833,9 +2029,13 @@ void launch_mc(bool fp64, bool single, const void *const *grids, const RotDev *r
         } else if (fp64) {
             DPLUS_MCZ(double, double4, false, kMaxM, false);
         } else if (mstride <= 8) {
+            mc_zrows_kernel<8><<<grid, 256, 0, s>>>((const float4 *const *)grids, zc, nz, groups, active, mstride, qs,
+                                                    step, seed, dir0, nblk, chunk, nu, nv, partial);
             DPLUS_MCZ(float, float4, true, 8, true);
             DPLUS_MCZ(float, float4, false, 8, true);
         } else {
+            mc_zrows_kernel<kMaxM><<<grid, 256, 0, s>>>((const float4 *const *)grids, zc, nz, groups, active, mstride,
+                                                        qs, step, seed, dir0, nblk, chunk, nu, nv, partial);
             DPLUS_MCZ(float, float4, true, kMaxM, true);
             DPLUS_MCZ(float, float4, false, kMaxM, true);
         }

@@ -292,6 +292,29 @@ def test_hybrid_docking_mc_matches_oracle(dplus, oracle, small, prec):
     assert np.max(np.abs(mine - ref) / ref) < (FP64_TOL if prec == 0 else MIXED_TOL)
 
 
+@pytest.mark.parametrize("copies,gs,nq", [((33,), 40, 60), ((40,), 40, 500), ((257,), 30, 40), ((90, 31, 200), 30, 300)])
+def test_whole_row_docking_matches_general_kernel(dplus, monkeypatch, copies, gs, nq):
+    """FP32 copies turned about z alone, through the whole-row kernel and, where the copies are
+    fewer than 2.5 per shell, the collapse and direct ones (33 and 40 copies at grid 40: both sides
+    of the line), q = 0 and the first shells (antipode and origin planes) among them, 8 and 16 q
+    a pass, one to three leaves, a last chunk of one copy: against the general kernel.  FP32 sums
+    of up to 321 copies in another order: 6e-8 sqrt(321) of I is 2e-6 where copies cancel least,
+    5e-6 allowed."""
+    import dplus_mi355x.synth as S
+    leaves = []
+    for i, n in enumerate(copies):
+        xyz, ion, coef9, rad = structure(200 + 50 * i, 11 + i)
+        g = gpu_grid(dplus, gs, 4.0, 1, xyz, ion, coef9, rad, host_copy=False)
+        leaves.append((g, *S.rows_to_docking(S.helix_rows(n, 3.0 + i, 0.3, 27.7 + 3 * i), scale=1.0 - 0.2 * i)))
+    q = np.linspace(0.0, 4.0, nq)
+    mine, _ = dplus.orientation_average(dplus.Docking(leaves), q, seed=4, max_dirs=2048, chunk=1024)
+    monkeypatch.setenv("DPLUS_ZCOPY", "0")
+    ref, _ = dplus.orientation_average(dplus.Docking(leaves), q, seed=4, max_dirs=2048, chunk=1024)
+    e = np.max(np.abs(mine - ref) / ref)
+    say(f"  [rows] {copies} copies, grid {gs}, {nq} q: vs general kernel {e:.2e}")
+    assert e < 5e-6
+
+
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("case", ["two_leaves", "sparse", "one_copy_chunk"])
 def test_zcopy_docking_mc_matches_oracle(dplus, oracle, small, prec, case, monkeypatch):
