@@ -210,17 +210,32 @@ struct LeafGeo {
     double step;
 };
 
-// Gauss-Kronrod phi recursion on the device: a node of the phi trees of one
-// batch of theta tasks (roots first, 15 per theta task) and an open phi interval
+// Gauss-Kronrod phi recursion on the device (docked_gk_level): a split interval,
+// holding the first of its halves' sums until the second comes, and an open interval
+constexpr unsigned long long kGkEmpty = 0x7ff8b1a5c0de0001ull;  // a NaN no sum has
 struct GkNode {
-    double value;
-    int parent;  // -1 for a root
-    int child0, child1;
-    int pending;  // children not yet resolved
+    unsigned long long mail;  // bits of the first half's value, kGkEmpty before
+    int parent, root;         // its own split interval (-1 for a root) and phi tree
 };
 struct GkInterval {
     double pmin, pmax;
-    int node, maxd, mind, pad;
+    int parent, root;
+};
+constexpr int kGkLevels = 15;  // most phi levels launched between two looks of the host
+struct GkLevel {
+    int level;    // within the batch: reads counts[level], counts the next level in counts[level + 1]
+    int nroots;   // phi trees
+    int before;   // intervals below the roots up to and including the batch's first level
+    int first;    // the trees' roots (phi in [0, 2 pi]) instead of a list
+    int last;     // depth reached: accept
+    int cap_int, cap_nodes;
+    double eps;
+    const double2 *roots;  // (q sin theta, q cos theta) of each tree
+    const GkInterval *cur;
+    GkInterval *next;
+    GkNode *nodes;
+    int *counts;
+    double *phival;
 };
 
 struct Grid {
@@ -539,7 +554,7 @@ constexpr size_t kGkNodes = (size_t)1 << 23;
 // two interval levels (task + record), the Kronrod/Gauss sums, the node arena,
 // the phi integrals of a theta level and the counters
 inline size_t gk_device_bytes(size_t nq) {
-    return kGkBatch * (2 * (32 + sizeof(GkInterval)) + 16 + 8) + kGkNodes * sizeof(GkNode) + nq * 32 + 8192;
+    return kGkBatch * std::max<size_t>(2 * sizeof(GkInterval) + 24, 48) + kGkNodes / 2 * sizeof(GkNode) + nq * 32 + 8192;
 }
 // space-filling lattice of a docked grid: basis vectors v[3k..3k+2] (nm) and
 // repetitions n[k]; on = 0 for none

@@ -35,10 +35,9 @@ void launch_docked_cart(bool fp64, const void *const *grids, const LeafGeo *geo,
 void launch_docked_gk(bool fp64, const void *const *grids, const LeafGeo *geo, const RotDev *rots, int nrot,
                       const double4 *trans, long long ntasks, const double4 *tasks, const GkNodes *nodes,
                       double *out, hipStream_t s);
-void launch_gk_decide(long long n, const GkInterval *cur, const double *kvgv, double eps, GkNode *nodes, int *cnt,
-                      int cap_int, int cap_nodes, const double4 *task, double4 *next_task, GkInterval *next,
-                      hipStream_t s);
-void launch_gk_tree_sums(GkNode *nodes, int lo, int hi, int nroots, double *phival, hipStream_t s);
+void launch_docked_gk_level(bool fp64, const void *const *grids, const LeafGeo *geo, const RotDev *rots, int nrot,
+                            const double4 *trans, const GkNodes *nodes, const GkLevel &L, long long bound,
+                            hipStream_t s);
 
 // Gauss-Kronrod 15/7 tables (Common/mathfuncs.h:100-125)
 static const double kX[15] = {
@@ -92,7 +91,8 @@ struct ThetaTask {
     long long maxd, mind;
     int node;          // node in the theta tree of q
     double phival[15]; // phi integrals of the 15 theta nodes
-    double qs[15], qc[15];  // q sin(theta_k), q cos(theta_k) of the 15 theta nodes
+    double sn[15];          // sin(theta_k) of the 15 theta nodes (device recursion)
+    double qs[15], qc[15];  // q sin(theta_k), q cos(theta_k)
     int left = 15;
 };
 
@@ -215,18 +215,19 @@ static void theta_nodes(ThetaTask &t, double qv) {
     const double ba2 = (t.tmax - t.tmin) * 0.5, apb2 = (t.tmax + t.tmin) * 0.5;
     for (int k = 0; k < 15; k++) {
         const double th = apb2 + ba2 * kX[k];
-        t.qs[k] = qv * std::sin(th);
+        t.sn[k] = std::sin(th);
+        t.qs[k] = qv * t.sn[k];
         t.qc[k] = qv * std::cos(th);
     }
 }
 
 // Kronrod and Gauss sums of a theta interval over its 15 phi integrals (GaussLegTheta, Amplitude.cpp:1424-1432)
 static void theta_sums(const ThetaTask &T, double &kv, double &gv) {
-    const double ba2 = (T.tmax - T.tmin) * 0.5, apb2 = (T.tmax + T.tmin) * 0.5;
+    const double ba2 = (T.tmax - T.tmin) * 0.5;
     kv = 0.0;
     gv = 0.0;
     for (int i = 0; i < 15; i++) {
-        const double sT = std::sin(apb2 + ba2 * kX[i]);
+        const double sT = T.sn[i];
         kv += T.phival[i] * kW[i] * ba2 * sT;
         if (i % 2 == 1) gv += T.phival[i] * gW[i / 2] * ba2 * sT;
     }
@@ -254,10 +255,11 @@ static long long gk_zero_q(const DockSet &D, int nq, const double *q, double *ou
 
 // The recursion with every phi interval on the device: the host keeps the theta
 // intervals (their nodes' sines and cosines, decisions and tree); each theta
-// level's 15 phi trees per interval are grown level by level on the device
-// (docked_gk_batch evaluates, gk_decide accepts and splits; gk_tree_sums adds
-// each tree's values level by level from the leaves), and their integrals come
-// back once per theta level.  Every sum is the host replay's:
+// level's 15 phi trees per interval are grown and added up level by level on the
+// device (docked_gk_level), and their integrals come back once per theta level.
+// The host launches as many phi levels as the theta level before it needed and
+// one more, then reads the levels' counts and the integrals in one copy; a level
+// that turns out empty costs its launch, 2 us.  Every sum is the host replay's:
 // the same phi intervals, Kronrod/Gauss sums, decisions and left + right tree
 // sums, so results and evaluation counts are equal.  Returns false when a level
 // outgrows the device arenas (the caller then runs the host replay).
@@ -285,76 +287,75 @@ static bool gk_average_device(const DockSet &D, int nq, const double *q, double 
         nodes.kw[i] = kW[i];
     }
     for (int i = 0; i < 7; i++) nodes.gw[i] = gW[i];
-    DevBuf bnodes, btask[2], biv[2], bkv, barena, bphi, bcnt;
+    DevBuf bnodes, biv[2], barena, bio;
     bnodes.upload(&nodes, sizeof nodes, s);
-    for (int b = 0; b < 2; b++) {
-        btask[b].ensure((size_t)cap_int * sizeof(double4));
-        biv[b].ensure((size_t)cap_int * sizeof(GkInterval));
-    }
-    bkv.ensure((size_t)cap_int * 2 * sizeof(double));
-    barena.ensure((size_t)cap_nodes * sizeof(GkNode));
-    bphi.ensure((size_t)cap_int * sizeof(double));
-    bcnt.ensure(4 * sizeof(int));
+    for (int b = 0; b < 2; b++) biv[b].ensure((size_t)cap_int * sizeof(GkInterval));
+    barena.ensure((size_t)cap_nodes / 2 * sizeof(GkNode));
+    // the roots, then the levels' counts, then the integrals: one copy each way
+    constexpr size_t kCounts = (kGkLevels + 1) * sizeof(int);
+    static_assert(kCounts % sizeof(double2) == 0, "roots, counts and integrals share a buffer");
+    bio.ensure((size_t)cap_int * 24 + kCounts);
     // pinned staging, kept by the thread across averages (an engine worker runs many)
-    static thread_local Pinned<int> hcnt;
-    static thread_local Pinned<double> hphi;
-    static thread_local Pinned<double4> hroot_t;
-    static thread_local Pinned<GkInterval> hroot_i;
-    static thread_local Pinned<GkNode> hroot_n;
-    int *cnt = hcnt.get(4);
-    while (!level.empty()) {
+    static thread_local Pinned<char> hio;
+    int depth = 4;  // phi levels of the theta level before (protein curves: 2 to 5)
+    for (long long maxd = max_depth - 1; !level.empty(); maxd--) {
         const size_t T = level.size(), nroots = 15 * T;
         if (nroots > (size_t)cap_int) return false;
-        double4 *rt = hroot_t.get(nroots);
-        GkInterval *ri = hroot_i.get(nroots);
-        GkNode *rn = hroot_n.get(nroots);
+        const size_t off = nroots * sizeof(double2);
+        char *io = hio.get(nroots * 24 + kCounts);
+        double2 *roots = (double2 *)io;
+        int *cnt = (int *)(io + off);
+        double *phi = (double *)(io + off + kCounts);
         for (size_t t = 0; t < T; t++)
-            for (int k = 0; k < 15; k++) {
-                const size_t r = 15 * t + k;
-                const double pmin = 0.0, pmax = k2Pi;
-                rt[r] = make_double4(level[t].qs[k], level[t].qc[k], (pmax + pmin) * 0.5, (pmax - pmin) * 0.5);
-                ri[r] = GkInterval{pmin, pmax, (int)r, (int)level[t].maxd, (int)level[t].mind, 0};
-                rn[r] = GkNode{0.0, -1, -1, -1, 0};
-            }
-        cnt[0] = 0;
-        cnt[1] = (int)nroots;
-        cnt[2] = 0;
-        int cur = 0;
-        check_hip(hipMemcpyAsync(btask[0].p, rt, nroots * sizeof(double4), hipMemcpyHostToDevice, s), "H2D");
-        check_hip(hipMemcpyAsync(biv[0].p, ri, nroots * sizeof(GkInterval), hipMemcpyHostToDevice, s), "H2D");
-        check_hip(hipMemcpyAsync(barena.p, rn, nroots * sizeof(GkNode), hipMemcpyHostToDevice, s), "H2D");
-        check_hip(hipMemcpyAsync(bcnt.p, cnt, 3 * sizeof(int), hipMemcpyHostToDevice, s), "H2D");
+            for (int k = 0; k < 15; k++) roots[15 * t + k] = make_double2(level[t].qs[k], level[t].qc[k]);
+        GkLevel L{};
+        L.nroots = (int)nroots;
+        L.cap_int = cap_int;
+        L.cap_nodes = cap_nodes;
+        L.eps = eps;
+        L.roots = (const double2 *)bio.p;
+        L.nodes = (GkNode *)barena.p;
+        L.counts = (int *)((char *)bio.p + off);
+        L.phival = (double *)((char *)bio.p + off + kCounts);
         long long n = (long long)nroots;
-        std::vector<int> bounds(1, 0);  // node ranges of the levels: roots first
-        bounds.push_back((int)nroots);
+        int levels = 0, cur = 0, batch = std::min(std::max(depth + 1, 2), kGkLevels);
         while (n > 0) {
+            std::fill(cnt, cnt + kGkLevels + 1, 0);
+            cnt[0] = (int)n;
+            if (levels == 0)
+                check_hip(hipMemcpyAsync(bio.p, io, off + kCounts, hipMemcpyHostToDevice, s), "H2D");
+            else
+                check_hip(hipMemcpyAsync(L.counts, cnt, kCounts, hipMemcpyHostToDevice, s), "H2D");
             {
                 KTimer kt("gk", s);
-                launch_docked_gk(D.fp64, (const void *const *)D.grids.p, (const LeafGeo *)D.geos.p,
-                                 (const RotDev *)D.rotb.p, D.nrot, (const double4 *)D.trb.p, n,
-                                 (const double4 *)btask[cur].p, (const GkNodes *)bnodes.p, (double *)bkv.p, s);
-                launch_gk_decide(n, (const GkInterval *)biv[cur].p, (const double *)bkv.p, eps, (GkNode *)barena.p,
-                                 (int *)bcnt.p, cap_int, cap_nodes, (const double4 *)btask[cur].p,
-                                 (double4 *)btask[1 - cur].p, (GkInterval *)biv[1 - cur].p, s);
+                long long bound = n;
+                for (int l = 0; l < batch; l++) {
+                    L.level = l;
+                    L.first = levels + l == 0;
+                    L.last = maxd - (levels + l) < 0;
+                    L.cur = (const GkInterval *)biv[cur].p;
+                    L.next = (GkInterval *)biv[1 - cur].p;
+                    launch_docked_gk_level(D.fp64, (const void *const *)D.grids.p, (const LeafGeo *)D.geos.p,
+                                           (const RotDev *)D.rotb.p, D.nrot, (const double4 *)D.trb.p,
+                                           (const GkNodes *)bnodes.p, L, bound, s);
+                    bound = std::min<long long>(2 * bound, cap_int);
+                    cur = 1 - cur;
+                }
                 check_hip(hipGetLastError(), "gk launch");
             }
-            check_hip(hipMemcpyAsync(cnt, bcnt.p, 3 * sizeof(int), hipMemcpyDeviceToHost, s), "D2H");
-            check_hip(hipStreamSynchronize(s), "gk level");
-            evals += 15 * n;
-            if (cnt[2]) return false;
-            n = cnt[0];
-            bounds.push_back(cnt[1]);
-            cnt[0] = 0;
-            check_hip(hipMemcpyAsync(bcnt.p, cnt, sizeof(int), hipMemcpyHostToDevice, s), "H2D");
-            cur = 1 - cur;
+            check_hip(hipMemcpyAsync(cnt, L.counts, kCounts + nroots * sizeof(double), hipMemcpyDeviceToHost, s),
+                      "D2H");
+            check_hip(hipStreamSynchronize(s), "gk levels");
+            for (int l = 0; l < batch; l++) {
+                evals += 15 * (long long)cnt[l];
+                if (cnt[l] > 0) depth = levels + l + 1;
+                L.before += cnt[l + 1];
+                if (cnt[l + 1] > cap_int || (long long)nroots + L.before > cap_nodes) return false;
+            }
+            n = cnt[batch];
+            levels += batch;
+            batch = 2;
         }
-        // tree sums from the deepest level to the roots
-        for (size_t b = bounds.size() - 1; b-- > 0;)
-            launch_gk_tree_sums((GkNode *)barena.p, bounds[b], bounds[b + 1], (int)nroots, (double *)bphi.p, s);
-        check_hip(hipGetLastError(), "gk tree sums");
-        double *phi = hphi.get(nroots);
-        check_hip(hipMemcpyAsync(phi, bphi.p, nroots * sizeof(double), hipMemcpyDeviceToHost, s), "D2H");
-        check_hip(hipStreamSynchronize(s), "gk phi integrals");
         // theta decisions of this level, in order
         std::vector<ThetaTask> next;
         for (size_t t = 0; t < T; t++) {

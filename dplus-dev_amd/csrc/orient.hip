@@ -1119,9 +1119,10 @@ __device__ __forceinline__ float wave_sums(const float (&v)[M], int lane, int o 
 // near 2.4 copies per shell.
 template <int M>
 __global__ __launch_bounds__(256, M <= 8 ? 3 : 2) void mc_zrows_kernel(
-    const float4 *const *__restrict__ grids, const ZCopyDev *__restrict__ zc, int nz, const GroupDev
-    *__restrict__ groups, const int *__restrict__ active, int mstride, const double *__restrict__ qs, double
-    step, uint64_t seed, long long dir0, int nblk, int chunk, int nu, int nv, double *__restrict__ partial) {
+    const float4 *const *__restrict__ grids, const ZCopyDev *__restrict__ zc, int nz,
+    const GroupDev *__restrict__ groups, const int *__restrict__ active, int mstride,
+    const double *__restrict__ qs, double step, uint64_t seed, long long dir0, int nblk, int chunk, int nu, int nv,
+    double *__restrict__ partial) {
     const int gi = blockIdx.y;
     const GroupDev G = groups[active[gi]];
     if (!whole_rows(G.layer, nz)) return;
@@ -1888,16 +1889,34 @@ __global__ __launch_bounds__(256) void azimuthal_kernel(const T4 *const *__restr
     if (threadIdx.x == 0) out[p] = (red[0] + red[1] + red[2] + red[3]) / (double)nphi;
 }
 
-// Gauss-Kronrod phi intervals: task t = (q sin(theta), q cos(theta), a, b) of
-// one interval; its 15 integrand points are phi = a + b x_k.  A workgroup of
-// 240 threads evaluates the points of 16 tasks, then one thread per task forms
+// Gauss-Kronrod phi intervals.  A workgroup of 240 threads evaluates the 15
+// points phi = a + b x_k of 16 intervals, then one thread per interval forms
 // the Kronrod and Gauss sums
-//   out[2t] = sum_k I_k b kw_k,  out[2t + 1] = sum_{k odd} I_k b gw_{k/2}
+//   kv = sum_k I_k b kw_k,  gv = sum_{k odd} I_k b gw_{k/2}
 // in k order with every product and sum rounded as written (no fused
 // multiply-add), the arithmetic of DomainModel::GaussLegPhi
-// (Amplitude.cpp:1443-1467), so accept/split decisions on the host follow it.
+// (Amplitude.cpp:1443-1467), so that accept/split decisions follow it.
 constexpr int kGkTasksPerBlock = 16;
 
+template <typename T, typename T4>
+__device__ __forceinline__ double gk_point(const T4 *const *__restrict__ grids, const LeafGeo *__restrict__ geo,
+                                           const RotDev *__restrict__ rots, int nrot,
+                                           const double4 *__restrict__ trans, const double4 &tk, double x) {
+    const double xi = fma(tk.w, x, tk.z);  // one rounding, whatever the caller forms a and b from
+    const double q[3] = {tk.x * cos(xi), tk.x * sin(xi), tk.y};
+    return docked_intensity<T, T4>(grids, geo, rots, nrot, trans, q);
+}
+__device__ __forceinline__ void gk_sums(const double *v, double hw, const GkNodes *__restrict__ nodes, double &kv,
+                                        double &gv) {
+    kv = gv = 0.0;
+    for (int k = 0; k < 15; k++) {
+        const double p = __dmul_rn(v[k], hw);
+        kv = __dadd_rn(kv, __dmul_rn(p, nodes->kw[k]));
+        if (k % 2 == 1) gv = __dadd_rn(gv, __dmul_rn(p, nodes->gw[k / 2]));
+    }
+}
+
+// the sums of a list of tasks (q sin(theta), q cos(theta), a, b): out[2t] = kv, out[2t + 1] = gv
 template <typename T, typename T4>
 __global__ __launch_bounds__(15 * kGkTasksPerBlock) void docked_gk_batch(
     const T4 *const *__restrict__ grids, const LeafGeo *__restrict__ geo, const RotDev *__restrict__ rots,
@@ -1907,106 +1926,98 @@ __global__ __launch_bounds__(15 * kGkTasksPerBlock) void docked_gk_batch(
     const long long t0 = (long long)blockIdx.x * kGkTasksPerBlock;
     const long long t = t0 + threadIdx.x / 15;
     double I = 0.0;
-    if (t < ntasks) {
-        const double4 tk = tasks[t];
-        const double xi = tk.z + tk.w * nodes->x[threadIdx.x % 15];
-        const double q[3] = {tk.x * cos(xi), tk.x * sin(xi), tk.y};
-        I = docked_intensity<T, T4>(grids, geo, rots, nrot, trans, q);
-    }
+    if (t < ntasks)
+        I = gk_point<T, T4>(grids, geo, rots, nrot, trans, tasks[t], nodes->x[threadIdx.x % 15]);
     val[threadIdx.x] = I;
     __syncthreads();
     const long long ts = t0 + threadIdx.x;
     if (threadIdx.x < kGkTasksPerBlock && ts < ntasks) {
-        const double hw = tasks[ts].w;
-        const double *v = val + 15 * threadIdx.x;
-        double kv = 0.0, gv = 0.0;
-        for (int k = 0; k < 15; k++) {
-            const double p = __dmul_rn(v[k], hw);
-            kv = __dadd_rn(kv, __dmul_rn(p, nodes->kw[k]));
-            if (k % 2 == 1) gv = __dadd_rn(gv, __dmul_rn(p, nodes->gw[k / 2]));
-        }
+        double kv, gv;
+        gk_sums(val + 15 * threadIdx.x, tasks[ts].w, nodes, kv, gv);
         out[2 * ts] = kv;
         out[2 * ts + 1] = gv;
     }
 }
 
-// Gauss-Kronrod phi recursion, one level per launch: each open interval is
-// accepted (its node takes its Kronrod sum) or split in two at its midpoint
-// (two new nodes and intervals at slots taken from counters, one atomic per
-// wave: cnt[0] next-level intervals, cnt[1] nodes, cnt[2] set on overflow).
-// Nodes are numbered level by level, so after the last level gk_tree_sums
-// walks the node ranges back to the roots: an inner node takes left + right,
-// and the roots' values are the phi integrals.  The accept rule and the
-// midpoint are GaussLegPhi's (Amplitude.cpp:1449-1467).
-__global__ __launch_bounds__(256) void gk_decide(long long n, const GkInterval *__restrict__ cur,
-                                                  const double *__restrict__ kvgv, double eps, GkNode *nodes,
-                                                  int *cnt, int cap_int, int cap_nodes, const double4 *__restrict__ task,
-                                                  double4 *__restrict__ next_task, GkInterval *__restrict__ next) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = t < n;
-    GkInterval I{0.0, 0.0, 0, 0, 0, 0};
-    double kv = 0.0, gv = 0.0;
-    bool accept = false;
-    if (live) {
-        I = cur[t];
-        kv = kvgv[2 * t];
-        gv = kvgv[2 * t + 1];
-        accept = I.mind < 0 && (I.maxd < 0 || fabs(1.0 - (gv / kv)) <= eps || gv == kv);
-    }
-    const bool split = live && !accept;
-    const unsigned long long mask = __ballot(split);
-    const int lane = threadIdx.x & 63;
-    int c = 0, w = 0;
-    if (mask) {
-        const int leader = __ffsll((long long)mask) - 1, nsplit = __popcll(mask);
-        int bc = 0, bw = 0;
-        if (lane == leader) {
-            bc = atomicAdd(&cnt[1], 2 * nsplit);
-            bw = atomicAdd(&cnt[0], 2 * nsplit);
+// One level of the phi recursion in one launch: a workgroup evaluates 16 open
+// intervals, and its first 16 threads accept each or split it at its midpoint
+// (two new intervals, their slots from one atomic per workgroup, and a node).
+// The accept rule and the midpoint are GaussLegPhi's (Amplitude.cpp:1449-1467).
+// An accepted value climbs: the first half of a split leaves its value at the
+// node, the second takes it, adds and goes on to the node above; left + right
+// either way round is the same sum, and a root's value is its phi integral.  So
+// no pass over the trees follows.  The level's length is read from the device
+// (the grid covers at most 16 times 4,096 intervals, larger levels go round), so
+// several levels are launched without the host waiting for each.  With a launch
+// of its own to decide, one more to add up a level and a wait for each count, a
+// level of up to 1,000 intervals took 25 us, of which the evaluation is 9: 501
+// q at tolerance 1e-3 (36 levels of 60 to 30,000 intervals) 2.28 -> 1.32 ms.
+template <typename T, typename T4>
+__global__ __launch_bounds__(15 * kGkTasksPerBlock, 2) void docked_gk_level(
+    const T4 *const *__restrict__ grids, const LeafGeo *__restrict__ geo, const RotDev *__restrict__ rots,
+    int nrot, const double4 *__restrict__ trans, const GkNodes *__restrict__ nodes, GkLevel L) {
+    __shared__ double val[15 * kGkTasksPerBlock];
+    const int n = L.first ? L.nroots : L.counts[L.level];
+    int below = L.before;  // intervals below the roots, this level's among them
+    for (int l = 1; l <= L.level; l++) below += L.counts[l];
+    if (n > L.cap_int || L.nroots + below > L.cap_nodes) return;  // the host sees the same counts
+    for (int t0 = (int)blockIdx.x * kGkTasksPerBlock; t0 < n; t0 += (int)gridDim.x * kGkTasksPerBlock) {
+        auto interval = [&](int t) {
+            return L.first ? GkInterval{0.0, k2Pi, -1, t} : L.cur[t];
+        };
+        const int t = t0 + (int)threadIdx.x / 15;
+        double I = 0.0;
+        if (t < n) {
+            const GkInterval iv = interval(t);
+            const double2 r = L.roots[iv.root];
+            const double4 tk = make_double4(r.x, r.y, __dmul_rn(__dadd_rn(iv.pmax, iv.pmin), 0.5),
+                                            __dmul_rn(__dsub_rn(iv.pmax, iv.pmin), 0.5));
+            I = gk_point<T, T4>(grids, geo, rots, nrot, trans, tk, nodes->x[threadIdx.x % 15]);
         }
-        bc = __shfl(bc, leader, 64);
-        bw = __shfl(bw, leader, 64);
-        const int rank = __popcll(mask & ((1ull << lane) - 1ull));
-        c = bc + 2 * rank;
-        w = bw + 2 * rank;
+        val[threadIdx.x] = I;
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            const int lane = threadIdx.x, ts = t0 + lane;
+            const bool live = lane < kGkTasksPerBlock && ts < n;
+            GkInterval iv{0.0, 0.0, -1, 0};
+            double kv = 0.0;
+            bool accept = false;
+            if (live) {
+                double gv;
+                iv = interval(ts);
+                gk_sums(val + 15 * lane, __dmul_rn(__dsub_rn(iv.pmax, iv.pmin), 0.5), nodes, kv, gv);
+                accept = L.last || fabs(1.0 - (gv / kv)) <= L.eps || gv == kv;
+            }
+            const bool split = live && !accept;
+            const unsigned long long mask = __ballot(split);
+            int w = 0;
+            if (mask) {
+                if (lane == 0) w = atomicAdd(&L.counts[L.level + 1], 2 * __popcll(mask));
+                w = __shfl(w, 0, 64) + 2 * __popcll(mask & ((1ull << lane) - 1ull));
+            }
+            if (split && w + 2 <= L.cap_int && L.nroots + below + w + 2 <= L.cap_nodes) {
+                const int c = (below + w) / 2;
+                const double mid = (iv.pmax + iv.pmin) * 0.5;
+                L.nodes[c] = GkNode{kGkEmpty, iv.parent, iv.root};
+                L.next[w] = GkInterval{iv.pmin, mid, c, iv.root};
+                L.next[w + 1] = GkInterval{mid, iv.pmax, c, iv.root};
+            }
+            if (live && accept) {
+                double v = kv;
+                int p = iv.parent;
+                while (p >= 0) {
+                    unsigned long long mine = (unsigned long long)__double_as_longlong(v);
+                    if (mine == kGkEmpty) mine = 0x7ff8000000000000ull;
+                    const unsigned long long other = atomicExch(&L.nodes[p].mail, mine);
+                    if (other == kGkEmpty) break;
+                    v = __dadd_rn(v, __longlong_as_double((long long)other));
+                    p = L.nodes[p].parent;
+                }
+                if (p < 0) L.phival[iv.root] = v;
+            }
+        }
+        __syncthreads();
     }
-    if (live && accept) nodes[I.node].value = kv;
-    if (!split) return;
-    if (c + 2 > cap_nodes || w + 2 > cap_int) {
-        atomicExch(&cnt[2], 1);
-        return;
-    }
-    nodes[c] = GkNode{0.0, I.node, -1, -1, 0};
-    nodes[c + 1] = GkNode{0.0, I.node, -1, -1, 0};
-    nodes[I.node].child0 = c;
-    nodes[I.node].child1 = c + 1;
-    const double4 tk = task[t];
-    const double mid = (I.pmax + I.pmin) * 0.5;
-    next[w] = GkInterval{I.pmin, mid, c, I.maxd - 1, I.mind - 1, 0};
-    next[w + 1] = GkInterval{mid, I.pmax, c + 1, I.maxd - 1, I.mind - 1, 0};
-    next_task[w] = make_double4(tk.x, tk.y, (mid + I.pmin) * 0.5, (mid - I.pmin) * 0.5);
-    next_task[w + 1] = make_double4(tk.x, tk.y, (I.pmax + mid) * 0.5, (I.pmax - mid) * 0.5);
-}
-
-// nodes [lo, hi) of one level: a split node takes left + right (its children,
-// in the next range, are final); a root writes its value to phival
-__global__ __launch_bounds__(256) void gk_tree_sums(GkNode *nodes, int lo, int hi, int nroots, double *phival) {
-    const int v = lo + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (v >= hi) return;
-    GkNode &N = nodes[v];
-    if (N.child0 >= 0) N.value = nodes[N.child0].value + nodes[N.child1].value;
-    if (v < nroots) phival[v] = N.value;
-}
-
-void launch_gk_decide(long long n, const GkInterval *cur, const double *kvgv, double eps, GkNode *nodes, int *cnt,
-                      int cap_int, int cap_nodes, const double4 *task, double4 *next_task, GkInterval *next,
-                      hipStream_t s) {
-    gk_decide<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, cur, kvgv, eps, nodes, cnt, cap_int, cap_nodes, task,
-                                                           next_task, next);
-}
-
-void launch_gk_tree_sums(GkNode *nodes, int lo, int hi, int nroots, double *phival, hipStream_t s) {
-    if (hi > lo) gk_tree_sums<<<(unsigned)((hi - lo + 255) / 256), 256, 0, s>>>(nodes, lo, hi, nroots, phival);
 }
 
 // ------------------------------------------------------------------ launchers
@@ -2174,6 +2185,20 @@ void launch_docked_gk(bool fp64, const void *const *grids, const LeafGeo *geo, c
     else
         docked_gk_batch<float, float4><<<nb, bs, 0, s>>>((const float4 *const *)grids, geo, rots, nrot, trans,
                                                           ntasks, tasks, nodes, out);
+}
+
+// one level of at most bound open intervals
+void launch_docked_gk_level(bool fp64, const void *const *grids, const LeafGeo *geo, const RotDev *rots, int nrot,
+                            const double4 *trans, const GkNodes *nodes, const GkLevel &L, long long bound,
+                            hipStream_t s) {
+    const unsigned nb = (unsigned)std::min<long long>((bound + kGkTasksPerBlock - 1) / kGkTasksPerBlock, 4096);
+    const int bs = 15 * kGkTasksPerBlock;
+    if (fp64)
+        docked_gk_level<double, double4><<<nb, bs, 0, s>>>((const double4 *const *)grids, geo, rots, nrot, trans,
+                                                            nodes, L);
+    else
+        docked_gk_level<float, float4><<<nb, bs, 0, s>>>((const float4 *const *)grids, geo, rots, nrot, trans,
+                                                          nodes, L);
 }
 
 void launch_azimuthal(bool fp64, const void *const *grids, const LeafGeo *geo, const RotDev *rots, int nrot,
