@@ -265,7 +265,6 @@ static long long gk_zero_q(const DockSet &D, int nq, const double *q, double *ou
 // outgrows the device arenas (the caller then runs the host replay).
 static bool gk_average_device(const DockSet &D, int nq, const double *q, double eps, long long max_depth,
                               double *out, long long &evals, hipStream_t s) {
-    const int cap_int = (int)kGkBatch, cap_nodes = (int)kGkNodes;
     std::vector<Tree> thetaTrees(nq);
     std::vector<ThetaTask> level;
     for (int i = 0; i < nq; i++) {
@@ -289,18 +288,32 @@ static bool gk_average_device(const DockSet &D, int nq, const double *q, double 
     for (int i = 0; i < 7; i++) nodes.gw[i] = gW[i];
     DevBuf bnodes, biv[2], barena, bio;
     bnodes.upload(&nodes, sizeof nodes, s);
-    for (int b = 0; b < 2; b++) biv[b].ensure((size_t)cap_int * sizeof(GkInterval));
-    barena.ensure((size_t)cap_nodes / 2 * sizeof(GkNode));
+    // Room for 65,536 intervals a level (9 MB) first, all of kGkBatch (136 MB) once a
+    // level needs it: taking and giving back 136 MB costs 1 ms a call in the
+    // allocator, and 501 q at tolerance 1e-3 open 30,000.
+    int cap_int = 1 << 16, cap_nodes = 1 << 19;
     // the roots, then the levels' counts, then the integrals: one copy each way
     constexpr size_t kCounts = (kGkLevels + 1) * sizeof(int);
     static_assert(kCounts % sizeof(double2) == 0, "roots, counts and integrals share a buffer");
-    bio.ensure((size_t)cap_int * 24 + kCounts);
+    auto room = [&]() {
+        for (int b = 0; b < 2; b++) biv[b].ensure((size_t)cap_int * sizeof(GkInterval));
+        barena.ensure((size_t)cap_nodes / 2 * sizeof(GkNode));
+        bio.ensure((size_t)cap_int * 24 + kCounts);
+    };
+    auto grow = [&]() {
+        if (cap_int == (int)kGkBatch) return false;
+        cap_int = (int)kGkBatch;
+        cap_nodes = (int)kGkNodes;
+        room();
+        return true;
+    };
+    room();
     // pinned staging, kept by the thread across averages (an engine worker runs many)
     static thread_local Pinned<char> hio;
     int depth = 4;  // phi levels of the theta level before (protein curves: 2 to 5)
     for (long long maxd = max_depth - 1; !level.empty(); maxd--) {
         const size_t T = level.size(), nroots = 15 * T;
-        if (nroots > (size_t)cap_int) return false;
+        if (nroots > (size_t)cap_int && (nroots > kGkBatch || !grow())) return false;
         const size_t off = nroots * sizeof(double2);
         char *io = hio.get(nroots * 24 + kCounts);
         double2 *roots = (double2 *)io;
@@ -317,6 +330,8 @@ static bool gk_average_device(const DockSet &D, int nq, const double *q, double 
         L.nodes = (GkNode *)barena.p;
         L.counts = (int *)((char *)bio.p + off);
         L.phival = (double *)((char *)bio.p + off + kCounts);
+        const long long evals0 = evals;
+        bool over = false;
         long long n = (long long)nroots;
         int levels = 0, cur = 0, batch = std::min(std::max(depth + 1, 2), kGkLevels);
         while (n > 0) {
@@ -350,11 +365,18 @@ static bool gk_average_device(const DockSet &D, int nq, const double *q, double 
                 evals += 15 * (long long)cnt[l];
                 if (cnt[l] > 0) depth = levels + l + 1;
                 L.before += cnt[l + 1];
-                if (cnt[l + 1] > cap_int || (long long)nroots + L.before > cap_nodes) return false;
+                over = over || cnt[l + 1] > cap_int || (long long)nroots + L.before > cap_nodes;
             }
+            if (over) break;
             n = cnt[batch];
             levels += batch;
             batch = 2;
+        }
+        if (over) {  // this theta level again, with all the room there is
+            if (!grow()) return false;
+            evals = evals0;
+            maxd++;
+            continue;
         }
         // theta decisions of this level, in order
         std::vector<ThetaTask> next;
