@@ -28,7 +28,6 @@ sys.path.insert(0, os.path.join(ROOT, "dplus-dev_amd"))
 sys.path.insert(0, os.path.join(ROOT, "oracle"))
 
 METRIC = "I(q) curves/s + p50/p99 latency, mixed vs FP64 GPU at ≤1e-4 rel err"
-PEAK_FP32_TFLOPS = 157.3  # MI355X published FP32 vector/matrix peak
 PEAK_HBM_GBPS = 8000.0  # MI355X HBM3E
 
 
@@ -123,7 +122,7 @@ def cpu_baseline(W, g64_data, g64_interp, shells=(8, 16, 24)):
                       f"{total:.0f} s"}
 
 
-def docking_curve(D, S, mb, directions=2_000_000):
+def docking_curve(D, S, directions=2_000_000):
     """The docking workload: a 5,000-atom subunit (2.5 nm sphere) on a grid of 200
     (qmax 6) docked as a 1,000-copy helix (radius 12 nm, rise 0.9 nm, twist 27.7
     deg), 800 q on [0, 6], MC over `directions` directions (chunks of 8,192), one
@@ -172,30 +171,13 @@ def docking_curve(D, S, mb, directions=2_000_000):
     log(f"[docking] mixed vs FP64 {err:.2e}, copy-major vs general kernel {err_general:.2e}; node bytes "
         f"{rate / 1e12:.2f} TB/s copy-major, {rate_general / 1e12:.2f} TB/s general (its gather ceiling "
         f"{ceiling / 1e12:.2f} TB/s)")
-    # counted: the copy-major launch's VALU wave instructions from rocprofv3 --pmc of this
-    # workload at 32,768 directions (profiles/docking_zcopy_valu.json), scaled to the
-    # directions run; their issue time at the microbenchmarked rates (FP32-rate, transcendental,
-    # FP64) over the live kernel time
-    roofline = None
-    vjs = os.path.join(ROOT, "profiles", "docking_zcopy_valu.json")
-    if os.path.exists(vjs):
-        P = json.load(open(vjs))
-        wi = P["wave_instructions"]
-        k = float(out["mixed"][3]) / P["directions"]
-        other = wi["valu"] - wi["valu_trans_f32"] - wi["valu_fp64"]
-        issue_s = k * 64.0 * (other / mb["fma32"] + wi["valu_trans_f32"] / mb["sin32"] + wi["valu_fp64"] / mb["fma64"])
-        t = out["mixed"][2] * 1e-3
-        roofline = {"bound": "valu", "kernel": P["kernel"], "achieved": k * wi["valu"] / t,
-                    "peak": k * wi["valu"] / issue_s, "unit": "VALU wave instructions/s (this kernel's mix)",
-                    "frac": issue_s / t, "valu_per_64_copies": wi["valu"] / (P["units"] / 64.0)}
-        log(f"[docking] copy-major VALU issue {issue_s * 1e3:.0f} ms of {t * 1e3:.0f} ms ({issue_s / t:.2f})")
     return {"workload": "5,000-atom subunit on grid 200 (qmax 6) docked as a 1,000-copy helix (R 12 nm, rise 0.9 nm, "
                         "twist 27.7 deg), 800 q, MC 2e6 directions",
             "value": 1.0 / out["mixed"][1], "unit": "curves/s", "fp64_value": 1.0 / out["fp64"][1],
             "general_kernel_value": 1.0 / out["mixed_general"][1],
             "speedup_vs_fp64": out["fp64"][1] / out["mixed"][1], "max_rel_err_vs_fp64": err,
             "max_rel_err_vs_general_kernel": err_general,
-            "directions": int(out["mixed"][3]), "roofline": roofline,
+            "directions": int(out["mixed"][3]),
             "gather": {"kernel": "mc_kernel<float, float4, false> (the general kernel, DPLUS_ZCOPY=0)",
                        "node_GBps_general": rate_general / 1e9, "node_GBps_copy_major": rate / 1e9,
                        "gather_ceiling_GBps": ceiling / 1e9, "general_frac": rate_general / ceiling,
@@ -607,46 +589,22 @@ def main():
     v_rate = v_lookups * 512 / (ms_vegas / max(args.steps, 1) * 1e-3)
     p_ms, p_lk = D.gather_probe(g32, 1 << 18, 0, ngroups)
     ceiling = p_lk * 512 / (p_ms * 1e-3)
-    oa_roof = {"bound": "gather", "kernel": "vegas_sample<float, float4, true> + vegas_reduce",
+    oa_roof = {"bound": "valu", "kernel": "vegas_sample<float, float4, true> + vegas_reduce",
                "achieved": v_rate / 1e9, "peak": ceiling / 1e9, "unit": "GB/s of nodes", "frac": v_rate / ceiling,
                "lookups_per_curve": v_lookups, "bytes_per_lookup": 512,
-               "ceiling": "dplus_gather_probe: the same lookups' node loads alone at full occupancy"}
+               "ceiling": "dplus_gather_probe: the same lookups' node loads alone, each from memory, at full "
+                          "occupancy; the kernel reads them from LDS tiles, so the fraction may exceed 1"}
     log(f"[bench] VEGAS lookups {v_rate / 1e12:.2f} TB/s of nodes, gather ceiling {ceiling / 1e12:.2f} TB/s "
         f"({v_rate / ceiling:.2f})")
 
-    # ---- roofline of the dominant kernel (the amplitude builder, VALU-bound)
-    N = W["gs"] // 2 + 3
-    nhalf = 3 * (N + 1) ** 2 * N
+    # ---- the amplitude builder against HBM: the bytes it cannot do without (the sources read,
+    # every node's amplitude written) over its launch time; and the direct sum's unit,
+    # 8 flops + 2 transcendentals per (node, source) term, that the frequency mesh replaces
     sources = len(W["xyz"]) + len(W["dims"])
-    terms = float(nhalf) * sources
-    # executed per atom and unit (three phi / phi + pi node pairs 120 degrees apart: six terms):
-    # q_x x + q_y y of two pairs (6 flops), their sin/cos (4 transcendentals), the third pair's
-    # e^{i u2} = conj(e^{i u0} e^{i u1}) (6 flops) and twelve FMAs (24 flops); sin/cos of q_z z
-    # come from LDS, evaluated once per (row, atom) per workgroup, whose units span a few rows
-    # (under 2 % of the work, not counted)
-    flop_eq = 36.0 / 6.0 + (4.0 / 6.0) * w_t
+    nodes = float(O_total_points(W["gs"]))
     t_launch = ms_build / max(nb, 1) * 1e-3
-    model_achieved = terms * flop_eq / t_launch / 1e12
-    # counted: the builder launch's VALU wave instructions from rocprofv3 --pmc of this
-    # workload (profiles/build_atoms_pairs_c2_valu.json), 64 lanes each: FP32 flops
-    # (FMA 2, MUL and ADD 1) plus w_T per transcendental, over the live launch time;
-    # issue_frac = their issue time at the microbenchmarked rates / the launch time
-    counted = None
-    vjs = os.path.join(ROOT, "profiles", "build_atoms_pairs_c2_valu.json")
-    if os.path.exists(vjs):
-        wi = json.load(open(vjs))["wave_instructions"]
-        flops32 = 64.0 * (2.0 * wi["valu_fma_f32"] + wi["valu_mul_f32"] + wi["valu_add_f32"])
-        trans = 64.0 * wi["valu_trans_f32"]
-        issue_s = 64.0 * (wi["valu"] - wi["valu_trans_f32"]) / mb["fma32"] + trans / mb["sin32"]
-        counted = {"flops_fp32": flops32, "transcendentals": trans, "valu_instructions_per_term": 64.0 * wi["valu"] / terms,
-                   "achieved": (flops32 + w_t * trans) / t_launch / 1e12, "issue_frac": issue_s / t_launch}
-    achieved = counted["achieved"] if counted else model_achieved
-    # HBM bytes per builder launch from the two rocprofv3 --pmc passes of this workload
-    # (FETCH_SIZE, WRITE_SIZE, each scaled by a known-size copy), kept in profiles/
-    traffic = None
-    pmc = os.path.join(ROOT, "profiles", "build_atoms_pairs_c2_pmc.json")
-    if os.path.exists(pmc):
-        traffic = json.load(open(pmc)).get("traffic_bytes")
+    traffic = 16.0 * len(W["xyz"]) + 28.0 * len(W["dims"]) + 8.0 * nodes
+    achieved = traffic / t_launch / 1e9
 
     cpu = None
     if not args.no_cpu_baseline:
@@ -654,7 +612,7 @@ def main():
         cpu = cpu_baseline(W, g64.data.copy(), g64.interp.copy())
         log(f"[bench] cpu baseline: {cpu}")
 
-    docking = None if args.no_docking else docking_curve(D, S, mb)
+    docking = None if args.no_docking else docking_curve(D, S)
     plain = plain_curve(D, S)
 
     serving = sessions = None
@@ -693,21 +651,12 @@ def main():
             "max_rel_err_vs_fp64": err_plain},
         "speedup_vs_fp64_plain": None if not lat64p else value * float(np.mean(lat64p)),
         "gauss_kronrod": gk_out,
-        "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_FP32_TFLOPS, "traffic": traffic,
-                     "kernel": f"build_atoms_pairs<false, {shape['wg']}>", "launch_ms": t_launch * 1e3,
-                     "terms_per_launch": terms, "flop_eq_per_term": flop_eq,
-                     "transcendental_weight": w_t,
-                     "achieved_from": "counted VALU instructions (rocprofv3 --pmc)" if counted else "flop model",
-                     "counted": counted, "model_achieved": model_achieved,
-                     # the direct sum's unit: 8 flops + 2 transcendentals per (node, source) term over
-                     # all P nodes (the builder does half the nodes by Friedel symmetry and shares sin/cos
-                     # pairs between the unit's nodes, so this exceeds the peak)
-                     "direct_sum_unit_achieved": float(O_total_points(W["gs"])) * sources * (8.0 + 2.0 * w_t) / t_launch / 1e12,
-                     # the same launch against the HBM roofline: PMC bytes per launch over its time
-                     "hbm": None if traffic is None else {
-                         "achieved": traffic / t_launch / 1e9, "peak": PEAK_HBM_GBPS, "unit": "GB/s",
-                         "frac": traffic / t_launch / 1e9 / PEAK_HBM_GBPS}},
+        "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBPS, "unit": "GB/s",
+                     "frac": achieved / PEAK_HBM_GBPS, "traffic": traffic,
+                     "traffic_from": "algorithmic: sources read once, every node's amplitude written once",
+                     "kernel": "mesh_spread + mesh_dft + mesh_interp", "launch_ms": t_launch * 1e3,
+                     "terms_per_launch": nodes * sources,
+                     "direct_sum_unit_achieved": nodes * sources * (8.0 + 2.0 * w_t) / t_launch / 1e12},
         "oa_roofline": oa_roof,
         "cpu_baseline": cpu,
         "docking": docking,
