@@ -122,6 +122,17 @@ DPLUS_HD void mc_stratify(long long d, int chunk, int nu, int nv, double &u, dou
     v = ((double)(w % nv) + v) / (double)nv;
 }
 
+// How the Monte Carlo average of a single leaf cuts its chunks (mc_patch_kernel): a
+// workgroup takes one patch and 4 D of the nchunks >= 4 chunks, a patch's chunks go over nset
+// workgroups.  D is as many as the chunks fill.  Every workgroup writes one block of the partial
+// sums, whose buffer holds chunk / 256 blocks a chunk: 4 nset <= nchunks for every count (five
+// chunks take D = 2: with D = 1 they would be two sets, 2 chunk / 64 blocks where
+// 5 chunk / 256 fit).
+inline void mc_patch_sets(long long nchunks, int &D, int &nset) {
+    D = nchunks >= 12 ? 4 : nchunks >= 5 ? 2 : 1;
+    nset = (int)((nchunks + 4 * D - 1) / (4 * D));
+}
+
 constexpr uint32_t kStreamMC = 0x4D43u;
 constexpr uint32_t kStreamVegas = 0x5645u;
 constexpr uint32_t kStreamAzimuth = 0x415Au;

@@ -2057,9 +2057,10 @@ void launch_mc(bool fp64, bool single, const void *const *grids, const RotDev *r
     // a single leaf over four chunks or more: by patch (its tile serves every chunk)
     const long long nchunks = (long long)nblk * 256 / chunk;
     if (single && nchunks >= 4) {
-        // directions per thread: as many as the chunks fill (a workgroup takes 4 D of them)
-        const int D = nchunks >= 12 ? 4 : nchunks >= 6 ? 2 : 1;
-        const int nset = (int)((nchunks + 4 * D - 1) / (4 * D)), nb = chunk / 64 * nset;  // nb <= nblk
+        int D, nset;
+        mc_patch_sets(nchunks, D, nset);
+        const int nb = chunk / 64 * nset;
+        if (nb > nblk) throw Error(kErrGeneral, "more workgroups than blocks of partial sums");
         const dim3 pg(nb, nactive);
 #define DPLUS_MCP(T, T4, D)                                                                                        \
     mc_patch_kernel<T, T4, D><<<pg, 256, 0, s>>>((const T4 *const *)grids, rots, groups, active, mstride, qs, step, \

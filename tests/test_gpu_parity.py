@@ -217,6 +217,21 @@ def test_mc_matches_oracle(dplus, oracle, small, prec):
     assert np.max(np.abs(mine - ref) / ref) < (FP64_TOL * 1e-3 if prec == 0 else MIXED_TOL)
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("chunks", [4, 5, 6, 7, 9, 12, 17])
+def test_mc_patch_sets_match_oracle(dplus, oracle, small, prec, chunks):
+    """A single leaf's chunks by patch: one, two and four directions a thread, sets that the chunks
+    fill and sets they do not, the last chunk of a set alone."""
+    say(f"[case] MC by patch, {chunks} chunks, precision={prec}")
+    s = small
+    g = gpu_grid(dplus, s["gs"], s["qmax"], prec, s["xyz"], s["ion"], s["coef9"], s["rad"])
+    q = np.linspace(0, s["qmax"], 61)
+    mine, st = dplus.orientation_average(dplus.Docking.single(g), q, seed=9, max_dirs=chunks * 512, chunk=512)
+    assert st.dirs_used == chunks * 512
+    ref, _ = oracle.mc_oa(oracle.Docked.single(s["gs"], s["qmax"], s["data"], s["co"]), q, 9, chunks * 512, 512)
+    assert np.max(np.abs(mine - ref) / ref) < (FP64_TOL * 1e-3 if prec == 0 else MIXED_TOL)
+
+
 def test_mc_convergence_path_matches_oracle(dplus, oracle, small):
     say("[case] MC with convergence")
     s = small

@@ -72,6 +72,33 @@ def test_engine_same_alone_and_in_the_mix(dplus):
             assert r1["chi2_on_device"] == 1
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+def test_engine_mc_of_five_chunks_with_chi2_matches_oracle(dplus, oracle, prec):
+    """40,000 directions in chunks of 8,192: five chunks of a single leaf, whose partial sums lie
+    before the curve and the measured data in a slot's arena."""
+    from dplus_mi355x.serving import Engine
+    say(f"[case] engine: five chunks with chi^2, precision={prec}")
+    pdb = make_pdb(300, 6, 1.2)
+    gs, qmax = 20, 4.0
+    q = np.linspace(0.05, qmax, 40)
+    ions = oracle.Ions(pdb["coef9"], pdb["rad"], np.bincount(pdb["ion"], minlength=len(pdb["coef9"])), 333.0, 1.0,
+                       oracle.CALC_ATOMIC_FORMFACTORS | oracle.CALC_DUMMY_SOLVENT)
+    data = oracle.grid_fill_pdb(gs, qmax, pdb["xyz"], pdb["ion"], ions)
+    ref, used = oracle.mc_oa(oracle.Docked.single(gs, qmax, data, oracle.grid_splines(gs, data)), q, 3, 40000, 8192)
+    assert used == 40960
+    y, sigma = 1.1 * ref, 0.1 * ref
+    for graphs in (False, True):
+        e = Engine(streams=2, graphs=graphs)
+        tickets = [e.submit(q, pdb=pdb, grid_size=gs, qmax=qmax, precision=prec, seed=3, method=dplus.OA_MC,
+                            max_dirs=40000, chunk=8192, data=y, sigma=sigma, fit_scale=1.0, fit_constant=0.0)
+                   for _ in range(3)]
+        for I, r in [e.wait(t) for t in tickets]:
+            assert r["dirs_used"] == 40960
+            assert np.max(np.abs(I - ref) / ref) < (1e-9 if prec == 0 else 1e-4)
+            assert r["chi2"] == pytest.approx(float(np.sum(((I - y) / sigma) ** 2)), rel=1e-12)
+        e.close()
+
+
 def test_engine_graph_requests_match_eager(dplus):
     from dplus_mi355x.serving import Engine
     say("[case] engine: 10 requests eager vs captured graphs (1 stream twice, then 4 streams)")
