@@ -133,6 +133,26 @@ inline void mc_patch_sets(long long nchunks, int &D, int &nset) {
     nset = (int)((nchunks + 4 * D - 1) / (4 * D));
 }
 
+// ---------------------------------------------------------------------------
+// VEGAS: a new boundary of an axis of kVB bins, at a share of the bins' weights.  w and edge
+// (right ends) are the bins', first the axis's lower end, cum the running sums of w added in
+// bin order: they do not fall, and a bin of weight 0 repeats the sum before it, so the first
+// bin whose sum exceeds the share has a weight.  keep is returned where no sum exceeds it.  The
+// share lies in that bin up to the rounding of the sums, and the boundary is held there.
+// ---------------------------------------------------------------------------
+constexpr int kVB = 32;  // bins per axis (GPUHybridCalc.cu:30-31)
+
+DPLUS_HD double vegas_boundary(const double *w, const double *cum, const double *edge, double first, int share,
+                               double keep) {
+    const double want = (cum[kVB - 1] / kVB) * (double)share;
+    int n = 0;  // bins whose running sum does not exceed the share
+    for (int s = kVB / 2; s > 0; s >>= 1)
+        if (!(cum[n + s - 1] > want)) n += s;
+    if (!(cum[n] > want)) return keep;
+    const double right = edge[n], left = n > 0 ? edge[n - 1] : first;
+    return fmax(right - (cum[n] - want) * (right - left) / w[n], left);
+}
+
 constexpr uint32_t kStreamMC = 0x4D43u;
 constexpr uint32_t kStreamVegas = 0x5645u;
 constexpr uint32_t kStreamAzimuth = 0x415Au;

@@ -1439,8 +1439,6 @@ void launch_chi2_param(const double *I, const double *y, const double *sig, int 
 }
 
 // ------------------------------------------------------------------ VEGAS
-constexpr int kVB = 32;  // bins per axis (GPUHybridCalc.cu:30-31)
-
 constexpr int kVM = 8;         // q-values per pass in the VEGAS kernels
 constexpr int kVPts = 4;       // points per lane and bin: points per bin <= 256
 
@@ -1629,38 +1627,37 @@ __device__ __forceinline__ double vegas_weight(double x) {
 }
 
 // The re-binning of one axis by a half wave (lane i of 32 holds weight w_i and the bin
-// [b_i, b_i+1]): new interior boundaries at equal shares of the weights.  Boundary j + 1
-// lies in the first bin whose running sum exceeds (j + 1) shares; boundaries that no sum
-// reaches keep their value.  lane i returns boundary i + 1 (of 32; the last stays).
+// [b_i, b_i+1]): new interior boundaries at equal shares of the weights (vegas_boundary);
+// boundaries that no sum reaches keep their value.  lane i returns boundary i + 1 (of 32; the
+// last stays).  Every lane adds the weights in bin order, from LDS: a scan across the lanes adds
+// each running sum in another order, and a bin of weight 0 then starts or ends above its
+// neighbour's sum.
 __device__ __forceinline__ double vegas_rebin(double w, double lo, double hi, int i, double *cum, double *wt, double *edge) {
     const double first = __shfl(lo, 0, kVB);
-    double c = w;
-#pragma unroll
-    for (int d = 1; d < kVB; d <<= 1) {
-        const double t = __shfl_up(c, d, kVB);
-        if (i >= d) c += t;
-    }
-    cum[i] = c;
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     wt[i] = w;
     edge[i] = hi;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const double want = (cum[kVB - 1] / kVB) * (double)(i + 1);
-    int n = 0;  // bins whose running sum does not exceed the share (the sums do not fall)
+    wave_sync();
+    double c = 0.0, mine = 0.0;
 #pragma unroll
-    for (int s = kVB / 2; s > 0; s >>= 1)
-        if (!(cum[n + s - 1] > want)) n += s;
-    if (!(cum[n] > want) || i == kVB - 1) return hi;
-    const double right = edge[n], left = n > 0 ? edge[n - 1] : first;
-    return right - (cum[n] - want) * (right - left) / wt[n];
+    for (int k = 0; k < kVB; k++) {
+        c += wt[k];
+        if (k == i) mine = c;
+    }
+    cum[i] = mine;
+    wave_sync();
+    return i == kVB - 1 ? hi : vegas_boundary(wt, cum, edge, first, i + 1, hi);
 }
 
 // one block (1024 threads = the 32x32 bins) per active group: the iteration's
 // integral sum_bins vol * mean_bin(I_j) (q dealt over waves 1 to 15 first), the
 // theta/phi marginals of the bin variances, re-binning, and the running mean over iterations
 // (HybridVEGASResizeGridKernel; GPUHybridCalc.cu:654-701).  The re-binning runs on one wave,
-// an axis per half wave, by scans and a binary search: 16.5 -> 5.8 us an iteration (its 64
+// an axis per half wave, by running sums and a binary search: 16.5 -> 5.8 us an iteration (its 64
 // serial steps waited on LDS).
 // hist[iter * nq + q] holds the running mean after iteration iter.
 __global__ __launch_bounds__(1024) void vegas_reduce(const GroupDev *__restrict__ groups,

@@ -257,6 +257,24 @@ def test_vegas_matches_oracle(dplus, oracle, small, prec):
     assert np.max(np.abs(mine - ref) / ref) < (FP64_TOL if prec == 0 else MIXED_TOL)
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("ppb", [2, 8, 98])
+def test_vegas_of_an_isotropic_structure(dplus, oracle, prec, ppb):
+    """One atom at the origin: the bins' variances are rounding noise, zero in some and equal in
+    others, and every direction has the same intensity whatever the bins become."""
+    say(f"[case] VEGAS of one atom at the origin, {ppb} points a bin, precision={prec}")
+    xyz, ion, coef9, rad = structure(1, 3, radius=0.6)
+    gs, qmax = 24, 5.0
+    g = gpu_grid(dplus, gs, qmax, prec, np.zeros((1, 3)), ion, coef9, rad)
+    ions = oracle_ions(oracle, coef9, rad, ion)
+    data = oracle.grid_fill_pdb(gs, qmax, np.zeros((1, 3)), ion, ions)
+    q = np.linspace(0.02, qmax, 45)
+    ref, _ = oracle.mc_oa(oracle.Docked.single(gs, qmax, data, oracle.grid_splines(gs, data)), q, 1, 256, 256)
+    mine, _ = dplus.orientation_average(dplus.Docking.single(g), q, method=dplus.OA_VEGAS, seed=4,
+                                        vegas_iterations=8, vegas_points_per_bin=ppb)
+    assert np.max(np.abs(mine - ref) / ref) < (FP64_TOL if prec == 0 else MIXED_TOL)
+
+
 def test_gk_matches_oracle(dplus, oracle, small):
     say("[case] Gauss-Kronrod")
     s = small

@@ -12,6 +12,13 @@ SOURCE = r"""
 #include "common.hpp"
 using namespace dplus;
 extern "C" void patch_sets(long long nchunks, int *D, int *nset) { mc_patch_sets(nchunks, *D, *nset); }
+extern "C" void rebin(const double *w, const double *b, double *out) {  // vegas_rebin's sums, one axis
+    double cum[kVB], c = 0.0;
+    for (int i = 0; i < kVB; i++) cum[i] = c += w[i];
+    out[0] = b[0];
+    for (int i = 0; i < kVB; i++)
+        out[i + 1] = i == kVB - 1 ? b[i + 1] : vegas_boundary(w, cum, b + 1, b[0], i + 1, b[i + 1]);
+}
 """
 
 
@@ -36,3 +43,60 @@ def test_mc_patch_sets_fit_the_partial_sums(rules):
         assert D.value in (1, 2, 4) and (nset.value - 1) * per < n <= nset.value * per
         for chunk in (256, 512, 768, 8192):
             assert chunk // 64 * nset.value <= n * chunk // 256, (n, chunk)
+
+
+def _rebin(rules, w, b):
+    out = np.empty(33)
+    p = ctypes.POINTER(ctypes.c_double)
+    w, b = np.ascontiguousarray(w, float), np.ascontiguousarray(b, float)
+    rules.rebin(w.ctypes.data_as(p), b.ctypes.data_as(p), out.ctypes.data_as(p))
+    return out
+
+
+def _sweep(w, b):
+    """The serial sweep over the bins: a boundary wherever the running weight passes a share."""
+    new, j, dw, x, pts = b.copy(), 0, 0.0, b[0], w.sum() / 32
+    for i in range(32):
+        dw += w[i]
+        old, x = x, b[i + 1]
+        while dw > pts:
+            dw -= pts
+            if j < 31:
+                new[j + 1] = x - dw * (x - old) / w[i]
+            j += 1
+    return new
+
+
+def test_vegas_boundaries_of_general_weights_are_the_sweeps(rules):
+    rng = np.random.default_rng(3)
+    for _ in range(1000):
+        b = np.concatenate([[0.0], np.sort(rng.random(31)), [1.0]])
+        w = rng.random(32) ** rng.uniform(0.2, 4.0)
+        # a sum's rounding (32 terms: 2^-48 of the total) moves a boundary by that over the weight's density
+        tol = 2.0 ** -48 * w.sum() / w.min() + 1e-15
+        assert np.max(np.abs(_rebin(rules, w, b) - _sweep(w, b))) < tol
+
+
+def test_vegas_boundaries_with_zero_and_equal_weights(rules):
+    """Zero weights beside equal ones, where shares meet running sums exactly up to rounding: every
+    boundary is finite, in order, and lies in a bin of nonzero weight that holds its share."""
+    rng = np.random.default_rng(4)
+    cases = [np.zeros(32), np.eye(32)[0], np.eye(32)[31], np.eye(32)[17] * 1e-300, np.ones(32) * 0.1]
+    cases += [np.where(rng.random(32) < rng.random(), rng.random(), 0.0) for _ in range(4000)]
+    cases += [np.where(rng.random(32) < rng.random(), rng.random(32), 0.0) for _ in range(1000)]
+    for w in cases:
+        b = np.concatenate([[0.0], np.sort(rng.random(31)), [1.0]])
+        out = _rebin(rules, w, b)
+        assert np.isfinite(out).all() and out[0] == 0.0 and out[32] == 1.0
+        if not w.any():
+            assert np.array_equal(out, b)
+            continue
+        c = np.concatenate([[0.0], np.cumsum(w)])
+        eps = 2.0 ** -48 * c[32]
+        # the shares that a sum exceeds come first; boundaries past the last keep their value
+        taken = [i for i in range(1, 32) if c[32] > (c[32] / 32) * i]
+        assert (np.diff(out[[0] + taken]) >= 0).all()
+        for i in taken:
+            share = (c[32] / 32) * i
+            assert any(w[n] > 0 and b[n] <= out[i] <= b[n + 1] and c[n] - eps <= share <= c[n + 1] + eps
+                       for n in range(32))
