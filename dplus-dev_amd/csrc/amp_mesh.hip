@@ -830,7 +830,9 @@ bool mesh_plan(const MeshSources &S, int N, double step, bool fp64, int nion, si
         A.dk = kPi / (sigma * X);
         A.dkinv = 1.0 / A.dk;
         A.dk = 1.0 / A.dkinv;
-        const int reach = (int)std::ceil(Q / A.dk + 0.5 * WI) + 1;
+        const double steps = std::ceil(Q / A.dk + 0.5 * WI) + 1.0;
+        if (!(steps > 0.0 && steps < 65536.0)) return false;  // (also extents that are no sizes of a structure)
+        const int reach = (int)steps;
         const double K = reach * A.dk;
         A.h = kPi / (sigma * K) * (1.0 - 1e-9);
         A.hinv = 1.0 / A.h;

@@ -1,5 +1,5 @@
-"""Rules that size launches and place boundaries, from the headers the kernels include, compiled for
-the CPU."""
+"""Rules that size launches and place boundaries, from the headers the kernels include and the
+library's host code, compiled for the CPU."""
 import ctypes
 import os
 import subprocess
@@ -8,8 +8,10 @@ import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "dplus-dev_amd")
+LIB = os.path.join(PKG, "dplus_mi355x")
 SOURCE = r"""
-#include "common.hpp"
+#include "device.hpp"
 using namespace dplus;
 extern "C" void patch_sets(long long nchunks, int *D, int *nset) { mc_patch_sets(nchunks, *D, *nset); }
 extern "C" void rebin(const double *w, const double *b, double *out) {  // vegas_rebin's sums, one axis
@@ -18,6 +20,30 @@ extern "C" void rebin(const double *w, const double *b, double *out) {  // vegas
     out[0] = b[0];
     for (int i = 0; i < kVB; i++)
         out[i + 1] = i == kVB - 1 ? b[i + 1] : vegas_boundary(w, cum, b + 1, b[0], i + 1, b[i + 1]);
+}
+// the mesh builder's plan of one class of n sources in [lo, hi]: 0 refused, else the mesh's sizes
+static bool plan(const double *lo, const double *hi, int N, double step, int fp64, long long n, MeshPlan &P, MeshSizes &Z) {
+    MeshSources S;
+    S.ok = true;
+    S.nfield = 1;
+    S.natoms = n;
+    for (int a = 0; a < 3; a++) {
+        S.lo[a] = S.cell0[a] = lo[a];
+        S.hi[a] = hi[a];
+    }
+    S.cell_inv = 1.0;
+    return mesh_plan(S, N, step, fp64 != 0, 1, kMeshRoom, P, Z);
+}
+extern "C" int mesh_sizes(const double *lo, const double *hi, int N, double step, int fp64, int *m, int *k, long long *bytes) {
+    MeshPlan P;
+    MeshSizes Z;
+    if (!plan(lo, hi, N, step, fp64, 1000, P, Z)) return 0;
+    for (int a = 0; a < 3; a++) {
+        m[a] = P.ax[a].m;
+        k[a] = P.ax[a].k;
+    }
+    *bytes = (long long)Z.bytes;
+    return 1;
 }
 """
 
@@ -29,7 +55,8 @@ def rules(tmp_path_factory):
     with open(src, "w") as f:
         f.write(SOURCE)
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
-                    "-I" + os.path.join(ROOT, "dplus-dev_amd", "csrc"), src, "-o", out], check=True)
+                    "-I" + os.path.join(PKG, "csrc"), "-I" + os.path.join(ROOT, "include"), src, "-L" + LIB,
+                    "-ldplus_mi355x", "-Wl,-rpath," + LIB, "-o", out], check=True)
     return ctypes.CDLL(out)
 
 
@@ -100,3 +127,22 @@ def test_vegas_boundaries_with_zero_and_equal_weights(rules):
             share = (c[32] / 32) * i
             assert any(w[n] > 0 and b[n] <= out[i] <= b[n + 1] and c[n] - eps <= share <= c[n + 1] + eps
                        for n in range(32))
+
+
+@pytest.mark.parametrize("fp64", [0, 1])
+def test_mesh_plan_refuses_extents_it_has_no_sizes_for(rules, fp64):
+    """One long axis or three, from a protein to beyond any structure, and steps that are no
+    numbers: a plan has positive sizes within the workspace, or is refused."""
+    arr = lambda v: (ctypes.c_double * 3)(*v)
+    m, k, nb = (ctypes.c_int * 3)(), (ctypes.c_int * 3)(), ctypes.c_longlong()
+    for X in (0.0, 1.0, 50.0, 1e3, 1e6, 1e8, 1e9, 1e12, 1e200):
+        for axes in ((0,), (1,), (2,), (0, 1, 2)):
+            for step in (0.05, 1.0, 1e9, float("inf"), float("nan")):
+                half = [X if a in axes else 1.0 for a in range(3)]
+                ok = rules.mesh_sizes(arr([-x for x in half]), arr(half), 53, ctypes.c_double(step), fp64, m, k,
+                                      ctypes.byref(nb))
+                if not ok:
+                    assert X > 5.0 or step > 1.0 or step != step
+                    continue
+                assert all(0 < v < 4096 + 32 for v in m) and all(0 < v < 2 * 65536 + 2 for v in k)
+                assert 0 < nb.value <= 512 << 20
