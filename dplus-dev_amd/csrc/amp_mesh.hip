@@ -785,9 +785,12 @@ namespace {
 constexpr int kSpreadMixed = 10, kInterpMixed = 8, kSpread64 = 16, kInterp64 = 16;
 constexpr double kSigmaMixed = 2.0, kSigma64 = 2.5;
 // interpolation patches: rows at most, and the sides down the rows and along them in
-// frequency steps (mesh_lds bounds the (x, y) planes they need)
+// frequency steps (mesh_lds bounds the (x, y) planes they need, kPatchZ the z points)
 constexpr int kRowsMixed = 16, kRows64 = 12, kThreadsMixed = 256, kThreads64 = 512;
 constexpr double kDownMixed = 6.0, kAlongMixed = 10.0, kDown64 = 3.0, kAlong64 = 6.0;
+// (a column's z points are rounded up to the 8 or 4 that mesh_interp loads at a time)
+static_assert((int)kDownMixed + 1 + kInterpMixed + 7 <= kPatchZ && (int)kDown64 + 1 + kInterp64 + 3 <= kPatchZ,
+              "the rows' z windows fit wzt");
 
 int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
@@ -918,14 +921,16 @@ bool mesh_plan(const MeshSources &S, int N, double step, bool fp64, int nion, si
     return true;
 }
 
-// LDS of the interpolation: a patch's nodes span at most (down + along) / sqrt 2 steps
-// in x and in y, or `along` where the patch is a polar cap's sector
-static size_t mesh_lds(const MeshSizes &Z, bool fp64) {
+// LDS of the interpolation's (x, y) planes.  A patch's rows span at most (rows - 1) s steps of
+// q sin(theta) and its widest row an arc of at most `along` steps, so two of its nodes are at
+// most hypot of the two apart in any direction of the plane (the chord between radii a and b at
+// an angle d is (a - b)^2 + 4 a b sin^2(d / 2) squared), and their windows' first points one
+// more than the whole steps of that.
+size_t mesh_lds(const MeshSizes &Z, bool fp64) {
     const int W = fp64 ? kInterp64 : kInterpMixed, most = fp64 ? kRows64 : kRowsMixed;
     const double down = fp64 ? kDown64 : kDownMixed, along = fp64 ? kAlong64 : kAlongMixed;
     const int rows = (int)std::min((double)most, std::floor(down / Z.s) + 1.0);
-    const double side = std::max(along, ((rows - 1) * Z.s + along) / std::sqrt(2.0));
-    const int n = (int)std::floor(side) + 2 + W;
+    const int n = (int)std::floor(std::hypot((rows - 1) * Z.s, along)) + 2 + W;
     return (size_t)rows * n * (n | 1) * (fp64 ? 16 : 8);
 }
 

@@ -410,6 +410,7 @@ bool mesh_plan(const MeshSources &S, int N, double step, bool fp64, int nion, si
 // whether the mesh builder is the faster one
 bool mesh_pays(const MeshPlan &P, const MeshSizes &Z, int N, double sources, bool fp64);
 void mesh_bands(const MeshPlan &P, const MeshSizes &Z, int N, bool fp64, std::vector<MeshBand> &bands, int &ntiles);
+size_t mesh_lds(const MeshSizes &Z, bool fp64);  // bytes of the interpolation's planes
 void mesh_tables(const MeshPlan &P, bool fp64, double *tab);
 void launch_mesh(const MeshJob &J, bool fp64, hipStream_t s);
 // launch shape of the paired builder: workgroup size (64, 128, 256 or 512

@@ -45,6 +45,45 @@ extern "C" int mesh_sizes(const double *lo, const double *hi, int N, double step
     *bytes = (long long)Z.bytes;
     return 1;
 }
+// the most that a patch's planes and z windows need, over every patch of the grid, against what
+// the launch gives them; 0: refused
+extern "C" int mesh_patches(const double *lo, const double *hi, int N, double step, int fp64, long long *need, long long *have, int *zmost) {
+    MeshPlan P;
+    MeshSizes Z;
+    if (!plan(lo, hi, N, step, fp64, 1000, P, Z)) return 0;
+    std::vector<MeshBand> bands;
+    int ntiles;
+    mesh_bands(P, Z, N, fp64 != 0, bands, ntiles);
+    const int W = fp64 ? 16 : 8;
+    *need = 0;
+    *zmost = 0;
+    *have = (long long)mesh_lds(Z, fp64 != 0);
+    for (const MeshBand &B : bands) {
+        const int n6 = 6 * B.shell, half = 3 * B.shell;
+        const double q = B.shell * step;
+        auto place = [](double r, double inv) { return (int)ceil(r * inv); };
+        for (int k0 = 0; k0 < n6; k0 += B.cols) {
+            int x0 = 1 << 30, x1 = -x0, y0 = x0, y1 = x1, z0 = x0, z1 = x1;
+            for (int r = 0; r < B.rows; r++) {
+                const double t = kPi * (B.j0 + r) / half;
+                const int iz = place(q * cos(t), P.ax[2].dkinv);
+                z0 = std::min(z0, iz);
+                z1 = std::max(z1, iz);
+                for (int k = k0; k < std::min(k0 + B.cols, n6); k++) {
+                    const int ix = place(q * sin(t) * cos(k2Pi * k / n6), P.ax[0].dkinv);
+                    const int iy = place(q * sin(t) * sin(k2Pi * k / n6), P.ax[1].dkinv);
+                    x0 = std::min(x0, ix);
+                    x1 = std::max(x1, ix);
+                    y0 = std::min(y0, iy);
+                    y1 = std::max(y1, iy);
+                }
+            }
+            *need = std::max(*need, (long long)B.rows * (y1 - y0 + W) * ((x1 - x0 + W) | 1) * (fp64 ? 16 : 8));
+            *zmost = std::max(*zmost, z1 - z0 + W);
+        }
+    }
+    return 1;
+}
 """
 
 
@@ -146,3 +185,23 @@ def test_mesh_plan_refuses_extents_it_has_no_sizes_for(rules, fp64):
                     continue
                 assert all(0 < v < 4096 + 32 for v in m) and all(0 < v < 2 * 65536 + 2 for v in k)
                 assert 0 < nb.value <= 512 << 20
+
+
+@pytest.mark.parametrize("fp64", [0, 1])
+def test_mesh_patches_fit_their_planes(rules, fp64):
+    """Every patch of the interpolation at node spacings from far below a frequency step to far
+    above, equal and unequal axes: its (x, y) planes fit the launch's LDS (64 KB a workgroup mixed,
+    128 KB FP64) and its z points the rows' windows."""
+    arr = lambda v: (ctypes.c_double * 3)(*v)
+    need, have, z = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_int()
+    tried = 0
+    for N in (4, 13, 28, 53):
+        for half in ((0.3, 0.3, 0.3), (1.0, 0.8, 0.6), (2.0, 2.0, 2.0), (4.0, 1.0, 7.0), (9.0, 6.0, 5.0), (3.0, 30.0, 2.0)):
+            for step in (0.02, 0.05, 0.11, 0.23, 0.6):
+                if not rules.mesh_patches(arr([-h for h in half]), arr(half), N, ctypes.c_double(step), fp64,
+                                          ctypes.byref(need), ctypes.byref(have), ctypes.byref(z)):
+                    continue
+                tried += 1
+                assert 0 < need.value <= have.value <= (128 if fp64 else 64) << 10, (N, half, step)
+                assert (z.value + 7) // 8 * 8 <= 40
+    assert tried > 80
