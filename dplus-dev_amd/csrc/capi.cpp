@@ -735,13 +735,18 @@ BuildShape Structure::shape_for(const Grid &g, bool use_table) const {
 }
 
 // The mesh builder where it is the faster one, within kMeshRoom bytes of workspace or what
-// the direct builder's slice partials may take.
+// the direct builder's slice partials may take.  DPLUS_BUILD_ROUTE in the environment (a
+// diagnostic, as DPLUS_PHASE64 is): "direct" keeps every build direct, "mesh" takes the mesh
+// wherever it has a plan.
 size_t direct_build_bytes(int N) { return (size_t)kMaxSlices * 12 * pair_units(half_base(N + 1)) * sizeof(double); }
 
 static bool mesh_route_of(const MeshSources &S, long long nsources, int N, double step, bool fp64, int nion, MeshPlan &P,
                           MeshSizes &Z) {
-    return mesh_plan(S, N, step, fp64, nion, std::max(kMeshRoom, direct_build_bytes(N)), P, Z) &&
-           mesh_pays(P, Z, N, (double)nsources, fp64);
+    const char *env = getenv("DPLUS_BUILD_ROUTE");
+    const std::string route = env ? env : "";
+    return route != "direct" &&
+           mesh_plan(S, N, step, fp64, nion, std::max(kMeshRoom, direct_build_bytes(N)), P, Z) &&
+           (route == "mesh" || mesh_pays(P, Z, N, (double)nsources, fp64));
 }
 
 bool Structure::mesh_route(const Grid &g, MeshPlan &P, MeshSizes &Z) const {
@@ -1954,6 +1959,18 @@ int dplus_structure_build_shape(dplus_structure *sh, dplus_grid *gh, int *wg, in
         if (wg) *wg = b.wg;
         if (slices) *slices = b.slices;
         if (tuned) *tuned = t ? 1 : 0;
+    })
+}
+
+int dplus_structure_build_route(dplus_structure *sh, dplus_grid *gh, int *mesh) {
+    API_GUARD({
+        const Structure *st = (const Structure *)sh;
+        const Grid *g = (const Grid *)gh;
+        if (!st || !g || !mesh) throw Error(kErrInvalidArgs, "null argument");
+        MeshPlan P;
+        MeshSizes Z;
+        const bool paired = g->fp64() ? !fp64_plain_builder() : getenv("DPLUS_PHASE64") == nullptr;
+        *mesh = paired && st->mesh_route(*g, P, Z) ? 1 : 0;
     })
 }
 

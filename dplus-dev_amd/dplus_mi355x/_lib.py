@@ -128,6 +128,7 @@ SIGNATURES = {
                                                    ctypes.POINTER(ctypes.c_void_p), ctypes.c_int]),
     "dplus_build_shapes_clear": (ctypes.c_int, []),
     "dplus_structure_build_shape": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, _I, _I, _I]),
+    "dplus_structure_build_route": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, _I]),
     "dplus_build_shapes_save": (ctypes.c_int, [_VP, ctypes.POINTER(ctypes.c_longlong)]),
     "dplus_build_shapes_load": (ctypes.c_int, [ctypes.c_char_p]),
     "dplus_timing_enable": (ctypes.c_int, [ctypes.c_int]),

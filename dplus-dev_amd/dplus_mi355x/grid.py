@@ -136,6 +136,12 @@ class Structure:
                                                     ctypes.byref(tu)))
         return {"wg": wg.value, "slices": sl.value, "tuned": bool(tu.value)}
 
+    def build_route(self, grid):
+        """dplus_structure_build_route: "mesh" or "direct"."""
+        m = ctypes.c_int()
+        L.check(L.lib().dplus_structure_build_route(self._h, grid.handle, ctypes.byref(m)))
+        return "mesh" if m.value else "direct"
+
     def autotune(self, grid):
         """dplus_structure_autotune: times every builder launch shape on this grid,
         records the fastest for the grid's class and builds the grid; returns

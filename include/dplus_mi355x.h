@@ -150,6 +150,10 @@ int dplus_structure_autotune(dplus_structure *s, dplus_grid *g, int *wg, int *sl
 /* the launch shape a mixed build of grid g from structure s takes, and whether
  * it comes from the shape table (1) or the occupancy model (0) */
 int dplus_structure_build_shape(dplus_structure *s, dplus_grid *g, int *wg, int *slices, int *tuned);
+/* whether a build of grid g from structure s goes through the frequency mesh (1) or sums every
+ * source at every node (0); DPLUS_BUILD_ROUTE=direct in the environment keeps every build direct,
+ * DPLUS_BUILD_ROUTE=mesh takes the mesh wherever its workspace is within bounds */
+int dplus_structure_build_route(dplus_structure *s, dplus_grid *g, int *mesh);
 int dplus_build_shapes_save(char **text, long long *len);
 int dplus_build_shapes_load(const char *text);
 int dplus_build_shapes_clear(void);

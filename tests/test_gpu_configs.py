@@ -92,7 +92,7 @@ def oracle_ions(O, coef9, rad, ion, sol=333.0):
 # ---------------------------------------------------------------- mesh builder
 def _mesh_case(kind, seed=3):
     """(atoms xyz, elements, layer (dims, com), excluded (dims, com), voxel, grid size, qmax) of shapes
-    that the frequency-mesh builder has to place right; each is large enough to take it."""
+    that the frequency-mesh builder has to place right."""
     rng = np.random.default_rng(seed)
     el4 = np.array(["C", "N", "O", "S"])
     none = (np.zeros((0, 3), np.int32), np.zeros((0, 3)))
@@ -122,8 +122,9 @@ def _mesh_case(kind, seed=3):
 
 
 @pytest.mark.parametrize("kind", ["slab", "apart", "boxes", "boxes alone", "coarse grid", "fine grid", "12 ions"])
-def test_mesh_builder_vs_oracle(dplus, oracle, kind):
-    """Grids built through the frequency mesh against the oracle's direct sums at sampled nodes.
+def test_mesh_builder_vs_oracle(dplus, oracle, kind, monkeypatch):
+    """Grids built through the frequency mesh (also those that the direct builder takes at this size,
+    with few nodes or many box pieces) against the oracle's direct sums at sampled nodes.
     Tolerances of the shell's RMS: the mixed windows' 6e-8 per axis and side, FP32 sums of 72
     terms (1e-7) and the largest of ~2,000 nodes make 2e-6, times 5; FP64 6e-14 times 16."""
     import dplus_mi355x.synth as S
@@ -143,6 +144,8 @@ def test_mesh_builder_vs_oracle(dplus, oracle, kind):
                          excl_contrast=-333.0)
     for prec, tol in ((0, 1e-12), (1, 1e-5)):
         g = dplus.Grid(gs, qmax, prec)
+        monkeypatch.setenv("DPLUS_BUILD_ROUTE", "mesh")
+        assert st.build_route(g) == "mesh"
         st.build(g, host_copy=True)
         vals = grid_values(g, idx)
         e = node_errors(vals, 0.5 * ref, shell_of)

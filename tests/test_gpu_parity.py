@@ -84,7 +84,7 @@ def test_grid_build_edge_sizes(dplus, oracle, gs, natoms):
 
 
 @pytest.mark.parametrize("gs,natoms", [(6, 7), (24, 300), (70, 4000)])
-def test_fp64_paired_builder_matches_plain(dplus, gs, natoms):
+def test_fp64_paired_builder_matches_plain(dplus, gs, natoms, monkeypatch):
     """FP64 grids: the paired builder (the default FP64 form: Friedel halving,
     phi / phi + pi node pairs sharing the sincos of q_x x + q_y y, the row's
     sincos of q_z z through LDS, atom slices) and the plain builder (one node at
@@ -97,7 +97,9 @@ def test_fp64_paired_builder_matches_plain(dplus, gs, natoms):
     st = dplus.Structure(xyz, ion, coef9, rad, sol_ed=333.0, flags=dplus.CALC_ATOMIC_FORMFACTORS, box_dims=ld,
                          box_com=lc, vox_step=0.1, box_contrast=33.3, excl_dims=ed, excl_com=ec,
                          excl_contrast=-333.0)
+    monkeypatch.setenv("DPLUS_BUILD_ROUTE", "direct")
     g1 = dplus.Grid(gs, 5.0, 0)
+    assert st.build_route(g1) == "direct"
     st.build(g1, host_copy=True)
     dplus.set_fp64_builder(True)
     try:
@@ -110,6 +112,42 @@ def test_fp64_paired_builder_matches_plain(dplus, gs, natoms):
     say(f"    {len(ld)} layer and {len(ed)} excluded-volume boxes, shape {shape}; "
         f"nodes {err:.2e}, splines {err_i:.2e}")
     assert err < 1e-13 and err_i < 1e-12
+
+
+@pytest.mark.parametrize("reduce", [False, True])
+def test_large_direct_and_mesh_builds_match_plain(dplus, reduce, monkeypatch):
+    """4,000 atoms with hydration-layer and excluded-volume boxes at grid 70, large enough for the
+    frequency mesh and for several atom slices of the paired builder: FP64 through the mesh and
+    mixed directly (hardware sin/cos, and the reduced phase form) and through the mesh, against the
+    FP64 builder that takes one node at a time."""
+    say(f"[case] large builds, direct and mesh, vs plain, reduced phases {reduce}")
+    gs = 70
+    xyz, ion, coef9, rad = structure(4000, 30 + gs, radius=2.6)
+    ld, lc = dplus.hydration_boxes(xyz, rad[ion], probe=0.14, thickness=0.28, vox=0.1)
+    ed, ec = dplus.excluded_volume_boxes(xyz, rad[ion], probe=0.14, thickness=0.28, vox=0.1)
+    st = dplus.Structure(xyz, ion, coef9, rad, sol_ed=333.0, flags=dplus.CALC_ATOMIC_FORMFACTORS, box_dims=ld,
+                         box_com=lc, vox_step=0.1, box_contrast=33.3, excl_dims=ed, excl_com=ec,
+                         excl_contrast=-333.0)
+    ref = dplus.Grid(gs, 5.0, 0)
+    dplus.set_fp64_builder(True)
+    try:
+        assert st.build_route(ref) == "direct"
+        st.build(ref, host_copy=True)
+    finally:
+        dplus.set_fp64_builder(False)
+    if reduce:
+        monkeypatch.setenv("DPLUS_REDUCE_PHASE", "1")
+    for prec, route, tol in ((0, "mesh", 1e-13), (1, "mesh", 2e-5), (1, "direct", 2e-5)):
+        if route == "direct":
+            monkeypatch.setenv("DPLUS_BUILD_ROUTE", "direct")
+        else:
+            monkeypatch.delenv("DPLUS_BUILD_ROUTE", raising=False)
+        g = dplus.Grid(gs, 5.0, prec)
+        assert st.build_route(g) == route
+        st.build(g, host_copy=True)
+        err = relmax(g.data, ref.data)
+        say(f"    precision {prec}, {route}: shape {st.build_shape(g)}, nodes {err:.2e}")
+        assert err < tol
 
 
 def test_splines_of_uploaded_data(dplus, oracle):
