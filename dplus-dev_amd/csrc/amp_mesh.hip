@@ -293,7 +293,7 @@ __global__ __launch_bounds__(1024) void mesh_spread(MeshPlan P, int f0, int nsli
     for (int a = 0; a < 3; a++) {
         const double reach = (0.5 * WS + 1e-6) * P.ax[a].h + (boxes ? P.box_half[a] : 0.0);
         const double x = P.ax[a].x0 + o[a] * P.ax[a].h;
-        const double l = (x - reach - P.cell0[a]) * P.cell_inv, h = (x + (n[a] - 1) * P.ax[a].h + reach - P.cell0[a]) * P.cell_inv;
+        const double l = (x - reach - P.cell0[a]) * P.cell_inv[a], h = (x + (n[a] - 1) * P.ax[a].h + reach - P.cell0[a]) * P.cell_inv[a];
         lo[a] = (int)fmin(fmax(floor(l), 0.0), (double)P.ncell[a]);
         hi[a] = (int)fmin(fmax(floor(h), -1.0), (double)(P.ncell[a] - 1));
     }
@@ -853,9 +853,9 @@ bool mesh_plan(const MeshSources &S, int N, double step, bool fp64, int nion, si
         points *= A.m;
         P.cell0[a] = S.cell0[a] - A.c;
         P.ncell[a] = S.ncell[a];
+        P.cell_inv[a] = S.cell_inv[a];
         P.box_half[a] = S.piece_half[a];
     }
-    P.cell_inv = S.cell_inv;
     P.wp_box = 0;
     P.gl = 1;
     if (P.boxes) {
@@ -893,8 +893,13 @@ bool mesh_plan(const MeshSources &S, int N, double step, bool fp64, int nion, si
     Z.g = take(nf * fx * fy * fz * (fp64 ? 16 : 8));
     // two buffers used in turn by as many classes at a time as fit `room`
     // (and slices of a brick's sources, two batches or more each on average)
-    double reach = 1.0;  // bricks a source reaches
-    for (int a = 0; a < 3; a++) reach *= (WS + (a == 2 ? 16.0 : 8.0)) / (a == 2 ? 16.0 : 8.0);
+    // bricks that read a source: those its window reaches, and those that only its cell reaches
+    // (cells of kMeshCell are in the fit of mesh_pays; a long axis has larger ones)
+    double reach = 1.0;
+    for (int a = 0; a < 3; a++) {
+        const double brick = a == 2 ? 16.0 : 8.0, cell = std::max(0.0, 1.0 / S.cell_inv[a] - kMeshCell) * P.ax[a].hinv;
+        reach *= std::min((WS + brick + cell) / brick, P.ax[a].m / brick);
+    }
     const double batches = (double)std::max(S.natoms, S.npieces) * reach / (points / 1024.0) / 256.0;
     Z.slices = (int)std::max(1.0, std::min(4.0, batches / 2.0));
     size_t b0, b1 = al(fz * mx * my * 16);

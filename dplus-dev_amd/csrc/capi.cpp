@@ -388,11 +388,12 @@ struct BoxSet {
 };
 
 // Host side of MeshSources: the cell grid over every atom and box piece (cells of
-// 0.4 nm, larger where more than kMeshCells of them would be needed along an axis),
-// the atoms' order by (ion, cell) and the box pieces by cell.
+// kMeshCell nm, larger along an axis where kMeshCells of them do not cover it, and where
+// the table of cells would outgrow the sources), the atoms' order by (ion, cell) and the
+// box pieces by cell.
 struct MeshHost {
     bool ok = false;
-    double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, cell0[3] = {0, 0, 0}, cell_inv = 0.0, half[3] = {0, 0, 0};
+    double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, cell0[3] = {0, 0, 0}, cell_inv[3] = {0, 0, 0}, half[3] = {0, 0, 0};
     int ncell[3] = {1, 1, 1}, cells = 1;
     std::vector<double4> pieces, lens;
     long long npieces = 0;
@@ -401,8 +402,15 @@ struct MeshHost {
     int cell(const double *p) const {
         int c[3];
         for (int a = 0; a < 3; a++)
-            c[a] = std::min(ncell[a] - 1, std::max(0, (int)((p[a] - cell0[a]) * cell_inv)));
+            c[a] = std::min(ncell[a] - 1, std::max(0, (int)((p[a] - cell0[a]) * cell_inv[a])));
         return (c[0] * ncell[1] + c[1]) * ncell[2] + c[2];
+    }
+
+    // the cuts of a box of edges len along each axis, at most kMeshPiece apart
+    static double cut_box(const double len[3], double cut[3]) {
+        double k = 1.0;
+        for (int a = 0; a < 3; a++) k *= cut[a] = std::max(1.0, std::ceil(len[a] / kMeshPiece - 1e-9));
+        return k;
     }
 
     // measure: extents, classes and the number of pieces alone
@@ -419,81 +427,103 @@ struct MeshHost {
             }
             return std::isfinite(p[0]) && std::isfinite(p[1]) && std::isfinite(p[2]);
         };
-        if (atoms_on)
-            for (int a = 0; a < d->natoms; a++)
-                if (!see(d->xyz + 3 * a)) return;
-        size_t boxes = 0;
-        for (int si = 0; si < 2; si++) boxes += sets[si].n;
-        const size_t most = 4 * boxes + (1u << 20);
+        if (atoms_on) {
+            std::vector<char> used(d->nion, 0);
+            for (int a = 0; a < d->natoms; a++) {
+                if (!see(d->xyz + 3 * a) || d->ion[a] < 0 || d->ion[a] >= d->nion) return;
+                used[d->ion[a]] = 1;
+            }
+            for (int i = 0; i < d->nion; i++)
+                if (used[i]) fion.push_back(i);
+        }
+        // pieces: a piece costs the host about 60 ns and a build about 2 ns, a source 0.7 us
+        // (FP64 4.4) of a direct sum at the largest usual grid; boxes of many more pieces than
+        // this stay whole
+        const size_t boxes = (size_t)sets[0].n + sets[1].n;
+        const size_t most = 64 * boxes + 16 * (size_t)(atoms_on ? d->natoms : 0) + 4096;
         for (int si = 0; si < 2; si++)
             for (int b = 0; b < sets[si].n; b++) {
                 const int *n = sets[si].dims + 3 * b;
                 const double *com = sets[si].com + 3 * b;
                 if (n[0] < 0 || n[1] < 0 || n[2] < 0) return;
                 if (n[0] == 0 || n[1] == 0 || n[2] == 0) continue;  // no volume
-                double cut[3], k = 1.0, len[3];
-                for (int a = 0; a < 3; a++) {
-                    len[a] = n[a] * d->vox_step;
-                    cut[a] = std::max(1.0, std::ceil(len[a] / kMeshPiece - 1e-9));
-                    k *= cut[a];
-                }
+                double cut[3], end[3];
+                const double len[3] = {n[0] * d->vox_step, n[1] * d->vox_step, n[2] * d->vox_step};
+                const double k = cut_box(len, cut);
                 if (!(k + (double)npieces <= (double)most)) return;
                 npieces += (long long)k;
-                for (int a = 0; a < 3; a++) {
-                    len[a] /= cut[a];
-                    half[a] = std::max(half[a], 0.5 * len[a]);
+                for (int a = 0; a < 3; a++) half[a] = std::max(half[a], 0.5 * len[a] / cut[a]);
+                for (int sgn = -1; sgn <= 1; sgn += 2) {  // the outermost pieces' centres
+                    for (int a = 0; a < 3; a++) end[a] = com[a] + sgn * 0.5 * (cut[a] - 1.0) * (len[a] / cut[a]);
+                    if (!see(end)) return;
                 }
-                for (int x = 0; x < (int)cut[0]; x++)
-                    for (int y = 0; y < (int)cut[1]; y++)
-                        for (int z = 0; z < (int)cut[2]; z++) {
-                            const double p[3] = {com[0] + (x - 0.5 * (cut[0] - 1.0)) * len[0],
-                                                 com[1] + (y - 0.5 * (cut[1] - 1.0)) * len[1],
-                                                 com[2] + (z - 0.5 * (cut[2] - 1.0)) * len[2]};
-                            if (!see(p)) return;
-                            if (measure) continue;
-                            pieces.push_back(make_double4(p[0], p[1], p[2], sets[si].contrast));
-                            lens.push_back(make_double4(len[0], len[1], len[2], 0.0));
-                        }
             }
-        if (!(atoms_on && d->natoms > 0) && npieces == 0) return;
-        double size = 0.4;
-        for (int a = 0; a < 3; a++) size = std::max(size, (c_hi[a] - c_lo[a]) / kMeshCells * (1.0 + 1e-9));
-        if (!std::isfinite(size)) return;
-        cell_inv = 1.0 / size;
+        if (npieces > 0) fion.push_back(-1);
+        if (fion.empty() || fion.size() > (size_t)kMeshFields) return;
+        double size[3];
+        for (int a = 0; a < 3; a++) {
+            size[a] = std::max(kMeshCell, (c_hi[a] - c_lo[a]) / kMeshCells * (1.0 + 1e-9));
+            if (!std::isfinite(size[a])) return;
+        }
+        const double room = 2.0 * ((double)(atoms_on ? d->natoms : 0) + (double)npieces) + 8192.0;
+        for (;;) {
+            cells = 1;
+            for (int a = 0; a < 3; a++) {
+                cell_inv[a] = 1.0 / size[a];
+                ncell[a] = std::min(kMeshCells, (int)((c_hi[a] - c_lo[a]) * cell_inv[a]) + 1);
+                cells *= ncell[a];
+            }
+            if (cells == 1 || (double)fion.size() * (cells + 1.0) <= room) break;
+            for (int a = 0; a < 3; a++) size[a] *= 1.26;
+        }
         for (int a = 0; a < 3; a++) {
             cell0[a] = c_lo[a];
-            ncell[a] = std::min(kMeshCells, (int)((c_hi[a] - c_lo[a]) * cell_inv) + 1);
             lo[a] = c_lo[a] - half[a];
             hi[a] = c_hi[a] + half[a];
         }
-        cells = ncell[0] * ncell[1] * ncell[2];
-        if (atoms_on) {
-            std::vector<char> used(d->nion, 0);
-            for (int a = 0; a < d->natoms; a++) {
-                if (d->ion[a] < 0 || d->ion[a] >= d->nion) return;
-                used[d->ion[a]] = 1;
-            }
-            for (int i = 0; i < d->nion; i++)
-                if (used[i]) fion.push_back(i);
-        }
-        if (npieces > 0) fion.push_back(-1);
         ok = true;
         if (measure) return;
         start.assign(fion.size() * (cells + 1), 0);
-        if (!pieces.empty()) {
-            int *st = &start[(fion.size() - 1) * (cells + 1)];
-            std::vector<int> key(pieces.size());
-            for (size_t i = 0; i < pieces.size(); i++) st[(key[i] = cell(&pieces[i].x)) + 1]++;
-            for (int c = 0; c < cells; c++) st[c + 1] += st[c];
-            std::vector<int> at(st, st + cells);
-            std::vector<double4> p2(pieces.size()), l2(pieces.size());
-            for (size_t i = 0; i < pieces.size(); i++) {
-                const int k = at[key[i]]++;
-                p2[k] = pieces[i];
-                l2[k] = lens[i];
+        if (npieces > 0) cut_pieces(d, sets);
+    }
+
+    // the pieces of every box, sorted by cell
+    void cut_pieces(const dplus_pdb_desc *d, const BoxSet *sets) {
+        std::vector<double4> p1, l1;
+        std::vector<int> key;
+        p1.reserve(npieces);
+        l1.reserve(npieces);
+        key.reserve(npieces);
+        int *st = &start[(fion.size() - 1) * (cells + 1)];
+        for (int si = 0; si < 2; si++)
+            for (int b = 0; b < sets[si].n; b++) {
+                const int *n = sets[si].dims + 3 * b;
+                const double *com = sets[si].com + 3 * b;
+                if (n[0] == 0 || n[1] == 0 || n[2] == 0) continue;
+                double cut[3], len[3] = {n[0] * d->vox_step, n[1] * d->vox_step, n[2] * d->vox_step};
+                cut_box(len, cut);
+                for (int a = 0; a < 3; a++) len[a] /= cut[a];
+                for (int x = 0; x < (int)cut[0]; x++)
+                    for (int y = 0; y < (int)cut[1]; y++)
+                        for (int z = 0; z < (int)cut[2]; z++) {
+                            const double4 p = make_double4(com[0] + (x - 0.5 * (cut[0] - 1.0)) * len[0],
+                                                           com[1] + (y - 0.5 * (cut[1] - 1.0)) * len[1],
+                                                           com[2] + (z - 0.5 * (cut[2] - 1.0)) * len[2],
+                                                           sets[si].contrast);
+                            p1.push_back(p);
+                            l1.push_back(make_double4(len[0], len[1], len[2], 0.0));
+                            key.push_back(cell(&p.x));
+                            st[key.back() + 1]++;
+                        }
             }
-            pieces.swap(p2);
-            lens.swap(l2);
+        for (int c = 0; c < cells; c++) st[c + 1] += st[c];
+        std::vector<int> at(st, st + cells);
+        pieces.resize(p1.size());
+        lens.resize(p1.size());
+        for (size_t i = 0; i < p1.size(); i++) {
+            const int k = at[key[i]]++;
+            pieces[k] = p1[i];
+            lens[k] = l1[i];
         }
     }
 
@@ -508,9 +538,9 @@ struct MeshHost {
             m.hi[a] = hi[a];
             m.cell0[a] = cell0[a];
             m.ncell[a] = ncell[a];
+            m.cell_inv[a] = cell_inv[a];
             m.piece_half[a] = half[a];
         }
-        m.cell_inv = cell_inv;
         return m;
     }
 

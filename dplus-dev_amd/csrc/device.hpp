@@ -355,6 +355,7 @@ struct BuildBatch {
 // ---- mesh builder (amp_mesh.hip): a grid's amplitudes through a frequency mesh
 constexpr int kMeshFields = 64;    // classes of sources (ions, and one of box pieces)
 constexpr int kMeshCells = 32;     // source cells per axis at most
+constexpr double kMeshCell = 0.4;  // edge of a cell, nm, where an axis needs no more than that many
 constexpr size_t kMeshRoom = (size_t)512 << 20;  // workspace bytes
 constexpr double kMeshPiece = 0.3;  // longest edge of a box piece, nm
 // a structure's sources as the mesh builder reads them: classes 0..nfield-1 (the
@@ -364,7 +365,7 @@ struct MeshSources {
     int nfield = 0;
     long long natoms = 0, npieces = 0;
     double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // extent of the sources, box pieces whole
-    double cell0[3] = {0, 0, 0}, cell_inv = 0.0;
+    double cell0[3] = {0, 0, 0}, cell_inv[3] = {0, 0, 0};
     int ncell[3] = {1, 1, 1};
     double piece_half[3] = {0, 0, 0};  // largest half edges of a piece
     // device: class of each field (ion, or -1: box pieces), first source of every
@@ -380,7 +381,7 @@ struct MeshPlan {
     MeshAxis ax[3];
     int nfield, boxes, nion, shifted, gl, wp_box;
     int ncell[3];
-    double cell0[3], cell_inv, box_half[3], step;
+    double cell0[3], cell_inv[3], box_half[3], step;
     int t_spread, t_sinv, t_interp, t_iinv, t_gl;  // offsets of the tables
 };
 // workspace layout (bytes), classes per pass, slices of a brick's sources, table length

@@ -30,8 +30,8 @@ static bool plan(const double *lo, const double *hi, int N, double step, int fp6
     for (int a = 0; a < 3; a++) {
         S.lo[a] = S.cell0[a] = lo[a];
         S.hi[a] = hi[a];
+        S.cell_inv[a] = 1.0 / std::max(kMeshCell, (hi[a] - lo[a]) / kMeshCells);
     }
-    S.cell_inv = 1.0;
     return mesh_plan(S, N, step, fp64 != 0, 1, kMeshRoom, P, Z);
 }
 extern "C" int mesh_sizes(const double *lo, const double *hi, int N, double step, int fp64, int *m, int *k, long long *bytes) {
