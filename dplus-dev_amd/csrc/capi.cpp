@@ -406,6 +406,14 @@ struct MeshHost {
         return (c[0] * ncell[1] + c[1]) * ncell[2] + c[2];
     }
 
+    // device bytes of [classes | cells | box pieces | edges], each 256-byte aligned
+    size_t bytes() const {
+        auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+        if (!ok) return 0;
+        return al(fion.size() * sizeof(int)) + al(fion.size() * (size_t)(cells + 1) * sizeof(int)) +
+               2 * al((size_t)npieces * sizeof(double4));
+    }
+
     // the cuts of a box of edges len along each axis, at most kMeshPiece apart
     static double cut_box(const double len[3], double cut[3]) {
         double k = 1.0;
@@ -567,7 +575,7 @@ struct MeshHost {
 };
 }  // namespace
 
-Structure::Structure(const dplus_pdb_desc *d, hipStream_t s) {
+Structure::Structure(const dplus_pdb_desc *d, hipStream_t s, bool with_mesh) {
     if (d->natoms < 0 || d->nion <= 0 || d->nion > 255) throw Error(kErrInvalidArgs, "bad atom/ion counts");
     if (d->nbox < 0 || (d->nbox > 0 && (!d->box_dims || !d->box_com || !(d->vox_step > 0))))
         throw Error(kErrInvalidArgs, "bad solvent boxes");
@@ -595,6 +603,7 @@ Structure::Structure(const dplus_pdb_desc *d, hipStream_t s) {
     } else {
         mh.sort_atoms(d, order);
     }
+    if (!with_mesh) mh.ok = false;  // (the same order of atoms, so the same bits of a direct build)
     std::vector<int> border[2];
     for (int si = 0; si < 2; si++) {
         const BoxSet &B = sets[si];
@@ -783,13 +792,14 @@ bool Structure::mesh_route(const Grid &g, MeshPlan &P, MeshSizes &Z) const {
     return mesh_route_of(mesh, nsources, g.N, g.step, g.fp64(), desc.nion, P, Z);
 }
 
-size_t mesh_build_bytes(const dplus_pdb_desc *d, int grid_size, double qmax, bool fp64) {
+size_t mesh_build_bytes(const dplus_pdb_desc *d, int grid_size, double qmax, bool fp64, size_t &held) {
     const bool atoms_on = (d->flags & (DPLUS_CALC_ATOMIC_FORMFACTORS | DPLUS_CALC_DUMMY_SOLVENT)) && d->natoms > 0;
     const BoxSet sets[2] = {{d->box_contrast != 0.0 ? d->nbox : 0, d->box_dims, d->box_com, d->box_contrast},
                             {d->excl_contrast != 0.0 ? d->nexcl : 0, d->excl_dims, d->excl_com, d->excl_contrast}};
     if (grid_size % 2) grid_size++;
     const int N = actual_size(grid_size);
     const MeshHost mh(d, atoms_on, sets, true);
+    held = mh.bytes();
     MeshPlan P;
     MeshSizes Z;
     return mesh_route_of(mh.sources(atoms_on ? d->natoms : 0), (atoms_on ? d->natoms : 0) + (long long)sets[0].n + sets[1].n,
@@ -947,7 +957,7 @@ void Structure::build(Grid &g, bool host_copy, hipStream_t s, bool use_table, bo
 // table and builds the grid a last time, so it holds the bits every later
 // build of its class gives (the workgroup size changes no sum; the slice
 // count regroups the FP64 partial sums).
-BuildShape Structure::autotune(Grid &g, hipStream_t s, double *best_ms, double *model_ms) {
+BuildShape Structure::autotune(Grid &g, hipStream_t s, double *best_ms, double *model_ms, bool direct) {
     if (g.fp64()) throw Error(kErrInvalidArgs, "the autotuner serves the mixed-precision builder");
     const long long nunits = pair_units(half_base(g.N + 1));
     BuildShape model;
@@ -981,7 +991,7 @@ BuildShape Structure::autotune(Grid &g, hipStream_t s, double *best_ms, double *
                 }
             }
         }
-        BuildJob J = prepare(g, best.slices, P, s);
+        BuildJob J = prepare(g, best.slices, P, s, direct);
         launch(g, J, best.wg, P, s);
         finish(g, P, false, s);
     } catch (...) {

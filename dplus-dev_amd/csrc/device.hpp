@@ -439,7 +439,8 @@ struct Structure {
     const int4 *dtiles = nullptr, *ddims = nullptr;
     const double *dcon = nullptr;
     MeshSources mesh;
-    Structure(const dplus_pdb_desc *d, hipStream_t s);
+    // with_mesh: with the tables of the mesh builder (without, every build is direct)
+    Structure(const dplus_pdb_desc *d, hipStream_t s, bool with_mesh = true);
     // use_table: the launch shape from the autotuner's table where it has the grid's
     // class (shapes timed on a device to themselves), else the occupancy model's
     // direct: never through the mesh builder
@@ -471,13 +472,14 @@ struct Structure {
     BuildShape shape_for(const Grid &g, bool use_table = true) const;
     // times every launch shape on grid g, records the fastest in the shape
     // table and returns it (ms: its time and the occupancy model's)
-    BuildShape autotune(Grid &g, hipStream_t s, double *best_ms, double *model_ms);
+    // (direct: as build's, of the last build; the timed ones are direct)
+    BuildShape autotune(Grid &g, hipStream_t s, double *best_ms, double *model_ms, bool direct = false);
 };
 
 // workspace bytes of a build: the direct builder's at most, and the mesh builder's (0: the
-// description's grid takes the direct builder)
+// description's grid takes the direct builder); held: what the structure keeps for it
 size_t direct_build_bytes(int N);
-size_t mesh_build_bytes(const dplus_pdb_desc *d, int grid_size, double qmax, bool fp64);
+size_t mesh_build_bytes(const dplus_pdb_desc *d, int grid_size, double qmax, bool fp64, size_t &held);
 std::vector<GroupDev> make_groups(const double *q, int nq, double step);
 // paired builder: work units of a grid with nhalf canonical nodes, the number
 // of atom slices the occupancy model splits a launch of workgroup size wg over

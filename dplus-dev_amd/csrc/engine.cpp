@@ -120,7 +120,7 @@ struct Request {
     bool want_chi = false;
     dplus_oa_params oa{};
     size_t need = 0;
-    bool direct_build = false;  // its budget does not hold the mesh builder's workspace
+    bool direct_build = false;  // its budget does not hold the mesh builder's tables and workspace
     // results
     std::vector<double> I;
     double chi2 = 0.0;
@@ -393,7 +393,7 @@ struct Engine {
         if (mixed && autotune && !shape_lookup(g.N, S.ntiles, &tuned)) {
             std::lock_guard<std::mutex> lk(tune_mu);
             if (!shape_lookup(g.N, S.ntiles, &tuned)) {
-                S.autotune(g, s, nullptr, nullptr);
+                S.autotune(g, s, nullptr, nullptr, direct);
                 return;
             }
         }
@@ -490,12 +490,13 @@ struct Engine {
         }
     }
 
-    // content key of a request's PDB description: every array and scalar
+    // content key of a request's PDB description: every array and scalar, and whether the
+    // structure is to have the mesh builder's tables
     static void structure_key(Request &r) {
         const dplus_pdb_desc &d = r.desc;
         uint64_t key[2] = {0x13198A2E03707344ULL, 0x243F6A8885A308D3ULL};
         const double sc[7] = {d.sol_ed, d.c1, d.scale, d.vox_step, d.box_contrast, (double)d.flags, d.excl_contrast};
-        const long long n[4] = {d.natoms, d.nion, d.nbox, d.nexcl};
+        const long long n[5] = {d.natoms, d.nion, d.nbox, d.nexcl, r.direct_build ? 1 : 0};
         hash_bytes(key, n, sizeof n);
         hash_bytes(key, sc, sizeof sc);
         hash_bytes(key, r.xyz.data(), r.xyz.size() * sizeof(double));
@@ -525,7 +526,7 @@ struct Engine {
                     return c.s;
                 }
         }
-        std::shared_ptr<Structure> S(new Structure(&r.desc, s));
+        std::shared_ptr<Structure> S(new Structure(&r.desc, s, !r.direct_build));
         const size_t bytes = S->blob.n + 4096;
         std::lock_guard<std::mutex> lk(cache_mu);
         cache_misses++;
@@ -703,7 +704,7 @@ struct Engine {
                 } else if (!g->fp64() && autotune && !shape_lookup(g->N, S->ntiles, &tuned)) {
                     std::lock_guard<std::mutex> lk(tune_mu);
                     if (!shape_lookup(g->N, S->ntiles, &tuned))
-                        S->autotune(*g, s, nullptr, nullptr);  // times the shapes and builds g with the best
+                        S->autotune(*g, s, nullptr, nullptr, r.direct_build);  // times the shapes and builds g with the best
                     else
                         build_in_chain = true;
                 } else {
@@ -1040,17 +1041,19 @@ int dplus_engine_submit(dplus_engine *eh, const dplus_request *rq, long long *ti
         }
         r->oa = rq->oa;
         r->need = request_bytes(*r);
-        if (r->has_pdb && (r->precision == DPLUS_PRECISION_FP64 ? !fp64_plain_builder() : true)) {
-            // the mesh builder's workspace where it is the larger one; a budget that holds
-            // the request only without it keeps the direct builder
+        if (r->has_pdb) {
+            // what the structure keeps for the mesh builder, and that builder's workspace where
+            // it is the larger one; a budget that holds the request only without the two keeps
+            // the direct builder and a structure without
+            const bool fp64 = r->precision == DPLUS_PRECISION_FP64;
             const size_t direct = direct_build_bytes((r->grid_size + r->grid_size % 2) / 2 + 3);
-            const size_t mesh = mesh_build_bytes(&r->desc, r->grid_size, r->qmax, r->precision == DPLUS_PRECISION_FP64);
-            if (mesh > direct) {
-                if (r->need + (mesh - direct) + e->cache_cap + e->arena_cap <= e->budget)
-                    r->need += mesh - direct;
-                else
-                    r->direct_build = true;
-            }
+            size_t held = 0;
+            const size_t mesh = mesh_build_bytes(&r->desc, r->grid_size, r->qmax, fp64, held);
+            const size_t more = held + (mesh > direct && !(fp64 && fp64_plain_builder()) ? mesh - direct : 0);
+            if (r->need + more + e->cache_cap + e->arena_cap <= e->budget)
+                r->need += more;
+            else
+                r->direct_build = true;
         }
         if (r->need + e->cache_cap + e->arena_cap > e->budget)
             throw Error(kErrOutOfMemory, "the request needs " + std::to_string(r->need) +

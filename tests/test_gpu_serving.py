@@ -182,6 +182,48 @@ def test_engine_admission_budget_and_resident_grid(dplus):
     assert np.array_equal(Ig, I0)
 
 
+def test_engine_budget_that_admits_only_the_direct_builder(dplus, monkeypatch):
+    """A request whose budget holds the direct builder but neither the frequency mesh's workspace nor
+    the tables its structure keeps: admitted, within the budget, with the bits of a direct build,
+    with and without autotuning, eager and captured."""
+    from dplus_mi355x.serving import Engine
+    say("[case] engine: budget for the direct builder alone")
+    pdb = make_pdb(30000, 9, 6.0)
+    q = np.linspace(0.05, 6.0, 60)
+    kw = dict(pdb=pdb, grid_size=44, qmax=6.5, method=dplus.OA_MC, seed=2, max_dirs=4096, chunk=4096)
+
+    def run(budget=0, **engine):
+        dplus.build_shapes_clear()
+        e = Engine(hbm_budget_bytes=budget, streams=1, **engine)
+        I, r = e.wait(e.submit(q, **kw))
+        st = e.stats()
+        e.close()
+        assert not budget or st["peak_reserved"] <= st["budget"]
+        return I, r["reserved_bytes"]
+
+    try:
+        monkeypatch.setenv("DPLUS_BUILD_ROUTE", "mesh")
+        mesh, need_mesh = run()
+        monkeypatch.setenv("DPLUS_BUILD_ROUTE", "direct")
+        direct, _ = run()
+        assert not np.array_equal(mesh, direct)
+        np.testing.assert_allclose(mesh, direct, rtol=1e-4)
+        monkeypatch.setenv("DPLUS_BUILD_ROUTE", "mesh")
+        for autotune in (False, True):
+            for graphs in (False, True):
+                # the cache and the slots' arenas take 3/16 of a budget
+                I, need = run(budget=int((need_mesh - (4 << 20)) * 16 / 13), autotune=autotune, graphs=graphs)
+                say(f"    autotune {autotune}, graphs {graphs}: reserved {need} of {need_mesh}")
+                assert need < need_mesh
+                if autotune:  # another launch shape may regroup the sums
+                    np.testing.assert_allclose(I, direct, rtol=1e-6)
+                    assert not np.array_equal(I, mesh)
+                else:
+                    assert np.array_equal(I, direct)
+    finally:
+        dplus.build_shapes_clear()
+
+
 def test_fit_session_graph_replays(dplus):
     from dplus_mi355x.serving import FitSession
     import dplus_mi355x.synth as S
