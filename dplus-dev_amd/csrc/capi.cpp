@@ -819,6 +819,13 @@ BuildJob Structure::prepare(Grid &g, int slices, Pending &P, hipStream_t s, bool
     MeshJob &M = P.job;
     P.mesh = !direct && mesh_route(g, M.plan, M.z);
     if (P.mesh) {
+        try {
+            P.part.ensure(M.z.bytes);
+        } catch (const Error &) {  // no room for the workspace: the direct sum takes less
+            P.mesh = false;
+        }
+    }
+    if (P.mesh) {
         std::vector<MeshBand> bands;
         mesh_bands(M.plan, M.z, g.N, g.fp64(), bands, M.ntiles);
         // one upload: [form factors | tables | bands]
@@ -829,7 +836,6 @@ BuildJob Structure::prepare(Grid &g, int slices, Pending &P, hipStream_t s, bool
         ff.resize(ff.size() + (bands.size() * sizeof(MeshBand) + 7) / 8);
         memcpy((char *)ff.data() + bytes, bands.data(), bands.size() * sizeof(MeshBand));
         P.ff.upload(ff.data(), ff.size() * sizeof(double), s);
-        P.part.ensure(M.z.bytes);
         M.atoms = d64;
         M.pieces = mesh.pieces;
         M.lens = mesh.lens;
@@ -1947,10 +1953,11 @@ int dplus_structure_build_grids(int n, dplus_structure *const *sh, dplus_grid *c
                 st->build(*g, host_copy != 0, s);
             } else if (st->mesh_route(*g, mp, mz)) {
                 Structure::Pending P;
-                BuildJob J = st->prepare(*g, 1, P, s);
+                const BuildShape sh = st->shape_for(*g);
+                BuildJob J = st->prepare(*g, sh.slices, P, s);
                 {
                     KTimer kt("build", s);
-                    st->launch(*g, J, 256, P, s);
+                    st->launch(*g, J, sh.wg, P, s);
                 }
                 st->enqueue_finish(*g, P, s, true);
                 if (host_copy) g->download(s);

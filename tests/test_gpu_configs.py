@@ -19,6 +19,7 @@ the q values of a few shell layers of a full-size average exactly.
 Tolerances: FP64 mode 1e-6 relative on I(q) (grid nodes 1e-9 of the shell's RMS
 amplitude); mixed 1e-4 on I(q) (grid nodes 2e-5 of the shell's RMS amplitude).
 """
+import os
 import sys
 import time
 
@@ -154,6 +155,85 @@ def test_mesh_builder_vs_oracle(dplus, oracle, kind, monkeypatch):
         first = g.data.copy()
         st.build(g, host_copy=True)
         assert np.array_equal(first, g.data)
+
+
+ARENA_BUILD = r"""
+#include "device.hpp"
+using namespace dplus;
+// a build whose buffers come from `size` bytes of one allocation: 0, or an error's code
+extern "C" int build_in_arena(void *st, void *gh, size_t size, int *mesh, size_t *mesh_bytes, size_t *used) {
+    const Structure &S = *(const Structure *)st;
+    Grid &g = *(Grid *)gh;
+    hipStream_t s = Device::get().stream;
+    MeshPlan mp;
+    MeshSizes mz;
+    *mesh_bytes = S.mesh_route(g, mp, mz) ? mz.bytes : 0;
+    Arena a;
+    if (hipMalloc((void **)&a.base, size) != hipSuccess) return -1;
+    a.size = size;
+    set_arena(&a);
+    int rc = 0;
+    try {
+        Structure::Pending P;
+        const BuildShape sh = S.shape_for(g);
+        BuildJob J = S.prepare(g, sh.slices, P, s);
+        S.launch(g, J, sh.wg, P, s);
+        S.enqueue_finish(g, P, s, false);
+        check_hip(hipStreamSynchronize(s), "build");
+        *mesh = P.mesh ? 1 : 0;
+        *used = a.used;
+    } catch (const Error &e) {
+        (void)hipStreamSynchronize(s);
+        rc = e.code;
+    }
+    set_arena(nullptr);
+    (void)hipFree(a.base);
+    return rc;
+}
+"""
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_build_without_room_for_the_mesh_is_direct(dplus, prec, tmp_path, monkeypatch):
+    """A build that the mesh would take, where its workspace cannot be had but the direct builder's
+    can: the bits of a direct build.  With room for the workspace, the mesh's."""
+    import ctypes
+    import subprocess
+    import dplus_mi355x.synth as S
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    pkg, lib = os.path.join(root, "dplus-dev_amd"), os.path.join(root, "dplus-dev_amd", "dplus_mi355x")
+    src, out = tmp_path / "arena.cpp", tmp_path / "libarena.so"
+    src.write_text(ARENA_BUILD)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(pkg, "csrc"), "-I" + os.path.join(root, "include"), str(src), "-L" + lib,
+                    "-ldplus_mi355x", "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath," + lib, "-o", str(out)], check=True)
+    fn = ctypes.CDLL(str(out)).build_in_arena
+    xyz, el, _, _, _, gs, qmax = _mesh_case("coarse grid")
+    coef9, rad, ion, _ = S.structure_tables(el)
+    st = dplus.Structure(xyz, ion, coef9, rad, sol_ed=333.0, flags=3)
+    want = {}
+    for route in ("mesh", "direct"):
+        monkeypatch.setenv("DPLUS_BUILD_ROUTE", route)
+        g = dplus.Grid(gs, qmax, prec)
+        st.build(g, host_copy=True)
+        want[route] = g.data.copy()
+    assert not np.array_equal(want["mesh"], want["direct"])
+    monkeypatch.setenv("DPLUS_BUILD_ROUTE", "mesh")
+    mesh, nb, used = ctypes.c_int(), ctypes.c_size_t(), ctypes.c_size_t()
+    for size, route in ((256 << 20, "mesh"), (10 << 20, "direct")):
+        g = dplus.Grid(gs, qmax, prec)
+        rc = fn(st._h, g.handle, ctypes.c_size_t(size), ctypes.byref(mesh),
+                ctypes.byref(nb), ctypes.byref(used))
+        say(f"  [arena] precision {prec}, {size >> 20} MB, workspace {nb.value}: rc {rc}, mesh {mesh.value}, used {used.value}")
+        assert rc == 0 and 10 << 20 < nb.value and used.value <= size
+        assert mesh.value == (route == "mesh")
+        g.download()
+        assert np.array_equal(g.data, want[route])
+    # no room for either: refused as before
+    g = dplus.Grid(gs, qmax, prec)
+    assert fn(st._h, g.handle, ctypes.c_size_t(1 << 20), ctypes.byref(mesh),
+              ctypes.byref(nb), ctypes.byref(used)) == 21
+
 
 
 # ---------------------------------------------------------------- 50,000 atoms + hydration, grid 250
