@@ -1233,7 +1233,7 @@ __global__ __launch_bounds__(256, M <= 8 ? 3 : 2) void mc_zrows_kernel(
                         const double u = lqi < 0 ? (up >= 0.5 ? up - 0.5 : up + 0.5) : up;
                         int c;
                         const float t = (float)cell_of(u * (double)n[p], c);
-                        c = min(max(c, 0), n[p] - 1);
+                        c = c == n[p] ? 0 : c;  // (u rounded up to a whole turn; t is 0 there)
                         const float4 A = rows[base[p] + c], B = rows[base[p] + c + 1];
                         const float t2 = t * t, t3 = t2 * t;
                         const float h01 = 3.f * t2 - 2.f * t3, h00 = 1.f - h01, h11 = t3 - t2, h10 = h11 - t2 + t;
