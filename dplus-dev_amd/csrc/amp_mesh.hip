@@ -33,9 +33,9 @@
 // mixed: 113.2 ms direct -> 1.36 ms (spread 0.59, interpolation 0.38, transforms 0.14,
 // weights 0.07); 200,000 atoms at grid 110, mixed: 14.5 -> 0.9 ms; 5,000 atoms and
 // 22,000 boxes at grid 120, FP64: 20.6 -> 0.9 ms.  Error against direct sums in 64 bits,
-// median over the shells of |dA| / |A| (2-norms): mixed 1.0e-7 .. 1.5e-7 where the direct
-// FP32 builder has 2.8e-7 .. 3.9e-7; FP64 4e-15 where the direct one has 1e-15 .. 3e-15
-// (I(q) of both agree to 4e-15, and are equally far from a 64-bit reference).
+// median over the shells of |dA| / |A| (2-norms, against 80-bit sums; 2,000 to 20,000 atoms, a
+// protein, a cube, a slab, off the origin): mixed 6e-8 .. 1.5e-7 where the direct builder has
+// 1.1e-7 .. 4.3e-7; FP64 1.5e-16 .. 2.6e-15 where the direct one has 2.3e-16 .. 2.5e-15.
 //
 // Everything up to the frequency mesh is FP64.  A mixed grid's nodes are
 // interpolated in FP32 with W = 8 and an FP64 grid's in FP64 with W = 16.
@@ -70,36 +70,35 @@ struct Window {
     double inv[kInvDeg];
 };
 
-double bessel_i0(double x) {
-    double t = 1.0, s = 1.0;
+long double bessel_i0(long double x) {
+    long double t = 1.0L, s = 1.0L;
     for (int k = 1; k < 200; k++) {
-        t *= (x / (2.0 * k)) * (x / (2.0 * k));
+        t *= (x / (2.0L * k)) * (x / (2.0L * k));
         s += t;
-        if (t < 1e-18 * s) break;
+        if (t < 1e-21L * s) break;
     }
     return s;
 }
 
-// Gauss-Legendre nodes and weights on [-1, 1]
-void gauss_legendre(int n, std::vector<double> &x, std::vector<double> &w) {
-    x.assign(n, 0.0);
-    w.assign(n, 0.0);
+// Gauss-Legendre nodes and weights on [-1, 1].  In long double: a weight carries the
+// polynomials' rounding divided by 1 - z^2, 6e-15 of a double one, and every transform 1e-15
+void gauss_legendre(int n, std::vector<long double> &x, std::vector<long double> &w) {
+    x.assign(n, 0.0L);
+    w.assign(n, 0.0L);
     for (int i = 0; i < n; i++) {
-        double z = std::cos(kPi * (i + 0.75) / (n + 0.5)), dp = 1.0;
-        for (int it = 0; it < 100; it++) {
-            double p0 = 1.0, p1 = z;
+        long double z = std::cos(kPi * (i + 0.75) / (n + 0.5)), dp = 1.0L;
+        for (int it = 0; it < 6; it++) {  // (doubles its digits each time, from four)
+            long double p0 = 1.0L, p1 = z;
             for (int k = 2; k <= n; k++) {
-                const double p2 = ((2.0 * k - 1.0) * z * p1 - (k - 1.0) * p0) / k;
+                const long double p2 = ((2.0L * k - 1.0L) * z * p1 - (k - 1.0L) * p0) / k;
                 p0 = p1;
                 p1 = p2;
             }
-            dp = n * (z * p1 - p0) / (z * z - 1.0);
-            const double dz = p1 / dp;
-            z -= dz;
-            if (std::fabs(dz) < 1e-16) break;
+            dp = n * (z * p1 - p0) / (z * z - 1.0L);
+            z -= p1 / dp;
         }
         x[i] = z;
-        w[i] = 2.0 / ((1.0 - z * z) * dp * dp);
+        w[i] = 2.0L / ((1.0L - z * z) * dp * dp);
     }
 }
 
@@ -133,25 +132,32 @@ const Window &window(int W, double sigma) {
     Window &k = tab[W];
     if (k.W) return k;
     const int nc = W + 2;
-    const double beta = 0.985 * (1.0 - 0.5 / sigma) * kPi * W, i0b = bessel_i0(beta);
+    const long double beta = 0.985 * (1.0 - 0.5 / sigma) * kPi * W, i0b = bessel_i0(beta);
     k.coef.assign((size_t)W * nc, 0.0);
-    std::vector<long double> fit(std::max(nc, kInvDeg));
+    std::vector<long double> fit(std::max(nc, kInvDeg)), phi((size_t)W * nc), gx, gw;
+    gauss_legendre(32, gx, gw);
+    long double area = 0.0L;
     for (int l = 0; l < W; l++) {
         power_fit(nc, [&](long double z) {
-            const double t = (double)l - 0.5 * W + 0.5 * ((double)z + 1.0);
-            return (long double)(bessel_i0(beta * std::sqrt(std::max(0.0, 1.0 - 4.0 * t * t / ((double)W * W)))) / i0b);
+            const long double t = l - 0.5L * W + 0.5L * (z + 1.0L);
+            return bessel_i0(beta * sqrtl(std::max(0.0L, 1.0L - 4.0L * t * t / ((long double)W * W)))) / i0b;
         }, fit.data());
-        for (int d = 0; d < nc; d++) k.coef[(size_t)l * nc + d] = (double)fit[d];
+        for (int g = 0; g < 32; g++) {
+            long double v = 0.0L;
+            for (int d = nc - 1; d >= 0; d--) v = v * gx[g] + fit[d];
+            area += 0.5L * gw[g] * v;
+        }
+        for (int d = 0; d < nc; d++) phi[(size_t)l * nc + d] = fit[d];
     }
-    std::vector<double> gx, gw;
-    gauss_legendre(32, gx, gw);
+    // of unit area: 1 / phihat starts at 1, which no rounding of its constant term scales
+    for (size_t i = 0; i < phi.size(); i++) k.coef[i] = (double)(phi[i] / area);
     auto phihat = [&](long double xi) {
         long double s = 0.0L;
         for (int l = 0; l < W; l++)
             for (int g = 0; g < 32; g++) {
                 long double v = 0.0L;
-                for (int d = nc - 1; d >= 0; d--) v = v * (long double)gx[g] + (long double)k.coef[(size_t)l * nc + d];
-                s += 0.5L * (long double)gw[g] * v * cosl(xi * (l - 0.5L * W + 0.5L * ((long double)gx[g] + 1.0L)));
+                for (int d = nc - 1; d >= 0; d--) v = v * gx[g] + (long double)k.coef[(size_t)l * nc + d];
+                s += 0.5L * gw[g] * v * cosl(xi * (l - 0.5L * W + 0.5L * (gx[g] + 1.0L)));
             }
         return s;
     };
@@ -614,13 +620,13 @@ __global__ __launch_bounds__(kThreads, 2) void mesh_interp(MeshPlan P, const Mes
     if (threadIdx.x >= 64 && threadIdx.x < 64 + nrow) {
         const int r = threadIdx.x - 64;
         double s, c;
-        sincos(kPi * (double)(B.j0 + r) / (double)half, &s, &c);
+        sincospi((double)(B.j0 + r) / (double)half, &s, &c);
         rz[r] = q * c;
         rs[r] = q * s;
     }
     for (int e = threadIdx.x; e < ncol; e += kThreads) {
-        double s, c;
-        sincos(k2Pi * (double)(k0 + e) / (double)n6, &s, &c);
+        double s, c;  // (of whole fractions of a half turn: an angle in radians carries two more roundings)
+        sincospi((double)(k0 + e) / (double)half, &s, &c);
         cc[e] = c;
         cn[e] = s;
     }
@@ -974,7 +980,7 @@ void mesh_tables(const MeshPlan &P, bool fp64, double *tab) {
     std::copy(s.inv, s.inv + kInvDeg, tab + P.t_sinv);
     std::copy(i.coef.begin(), i.coef.end(), tab + P.t_interp);
     std::copy(i.inv, i.inv + kInvDeg, tab + P.t_iinv);
-    std::vector<double> x, w;
+    std::vector<long double> x, w;
     gauss_legendre(P.gl, x, w);
     std::copy(x.begin(), x.end(), tab + P.t_gl);
     std::copy(w.begin(), w.end(), tab + P.t_gl + P.gl);

@@ -157,6 +157,53 @@ def test_mesh_builder_vs_oracle(dplus, oracle, kind, monkeypatch):
         assert np.array_equal(first, g.data)
 
 
+@pytest.mark.parametrize("n,gs,qmax,half,shift", [(2000, 100, 5.0, (3.0, 3.0, 3.0), 0.0), (5000, 120, 6.1, (3.5, 2.7, 2.2), 0.0),
+                                                  (2000, 40, 3.0, (1.5, 1.5, 1.5), 0.0),
+                                                  (4000, 90, 4.0, (1.0, 1.0, 1.0), (14.0, 3.0, -2.0))])
+def test_fp64_mesh_is_as_precise_as_direct_sums(dplus, n, gs, qmax, half, shift, monkeypatch):
+    """FP64 grids through the mesh and by direct sums against 80-bit sums at 24 nodes of 17 shells:
+    the median over the shells of |dA| / |A| of the mesh is no larger than the direct builder's (a
+    quarter allowed for the sampled nodes; a table of six digits less would be twice or more)."""
+    import dplus_mi355x.synth as S
+    LD = np.longdouble
+    pi = LD("3.14159265358979323846264338327950288")
+    rng = np.random.default_rng(n + gs)
+    xyz = rng.normal(size=(n, 3))
+    xyz *= np.array(half) * rng.uniform(0, 1, (n, 1)) ** (1 / 3) / np.linalg.norm(xyz, axis=1)[:, None]
+    xyz = xyz + shift
+    coef9, rad, ion, _ = S.structure_tables(np.array(["C"] * n))
+    N = gs // 2 + 3
+    idx, shell, qv = [], [], []
+    for i in sorted(set(range(1, 6)) | set(np.linspace(1, N, 14).astype(int).tolist())):
+        for _ in range(24):
+            j, k = int(rng.integers(0, 3 * i + 1)), int(rng.integers(0, 6 * i))
+            idx.append(1 + 6 * (i - 1) * i * i + j * 6 * i + k)
+            shell.append(i)
+            q, th, ph = LD(i) * LD(qmax) / LD(gs // 2), pi * j / (3 * i), pi * k / (3 * i)
+            qv.append([q * np.sin(th) * np.cos(ph), q * np.sin(th) * np.sin(ph), q * np.cos(th)])
+    shell, qv = np.array(shell), np.array(qv, dtype=LD)
+    ref = np.zeros((len(idx), 2), LD)
+    for c in range(0, n, 500):
+        p = qv @ xyz[c:c + 500].astype(LD).T
+        ref += np.stack([np.cos(p).sum(1), np.sin(p).sum(1)], axis=1)
+    st = dplus.Structure(xyz, ion, coef9, rad, sol_ed=0.0, flags=dplus.CALC_ATOMIC_FORMFACTORS)
+    med = {}
+    for route in ("mesh", "direct"):
+        monkeypatch.setenv("DPLUS_BUILD_ROUTE", route)
+        g = dplus.Grid(gs, qmax, 0)
+        assert st.build_route(g) == route
+        st.build(g, host_copy=True)
+        a = np.stack([g.data[0::2][idx], g.data[1::2][idx]], axis=1).astype(LD)
+        e = []
+        for i in np.unique(shell):
+            m = shell == i
+            f = (a[m] * ref[m]).sum() / (ref[m] ** 2).sum()  # the shell's form factor
+            e.append(float(np.sqrt(((a[m] - f * ref[m]) ** 2).sum() / ((f * ref[m]) ** 2).sum())))
+        med[route] = np.median(e)
+    say(f"  [80-bit] {n} atoms, grid {gs}: mesh {med['mesh']:.2e}, direct {med['direct']:.2e}")
+    assert med["mesh"] <= 1.25 * med["direct"]
+
+
 ARENA_BUILD = r"""
 #include "device.hpp"
 using namespace dplus;
