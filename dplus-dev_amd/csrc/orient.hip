@@ -1220,6 +1220,9 @@ __global__ __launch_bounds__(256, M <= 8 ? 3 : 2) void mc_zrows_kernel(
                     const ZCopyDev z = zc[k];
                     double up = (phi - z.alpha) * kInv2Pi;
                     up += up < 0.0 ? 1.0 : 0.0;
+                    // below a whole turn by less than FP32 sees, so that no cell lies past the row's end
+                    constexpr double kTurn = 1.0 - 1e-11;
+                    up = fmin(up, kTurn);
                     const float sc = (float)z.scale;
                     cplx<float> amps[4];
 #pragma unroll
@@ -1230,10 +1233,9 @@ __global__ __launch_bounds__(256, M <= 8 ? 3 : 2) void mc_zrows_kernel(
                             amps[p] = {o.x * sc, o.y * sc};
                             continue;
                         }
-                        const double u = lqi < 0 ? (up >= 0.5 ? up - 0.5 : up + 0.5) : up;
+                        const double u = lqi < 0 ? (up >= 0.5 ? up - 0.5 : fmin(up + 0.5, kTurn)) : up;
                         int c;
                         const float t = (float)cell_of(u * (double)n[p], c);
-                        c = c == n[p] ? 0 : c;  // (u rounded up to a whole turn; t is 0 there)
                         const float4 A = rows[base[p] + c], B = rows[base[p] + c + 1];
                         const float t2 = t * t, t3 = t2 * t;
                         const float h01 = 3.f * t2 - 2.f * t3, h00 = 1.f - h01, h11 = t3 - t2, h10 = h11 - t2 + t;

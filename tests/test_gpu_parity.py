@@ -234,6 +234,26 @@ def test_interpolate_theta_phi_plane_matches_oracle(dplus, oracle, small, prec):
             g.interpolate_theta_phi_plane(*bad)
 
 
+def test_mixed_plane_lookup_at_the_nodes(dplus, small):
+    """A mixed grid's plane lookup at the nodes' own angles gives the nodes' values, first and last
+    rows and columns and the full turn among them."""
+    say("[case] mixed plane lookup at nodes")
+    s = small
+    g = gpu_grid(dplus, s["gs"], s["qmax"], 1, s["xyz"], s["ion"], s["coef9"], s["rad"])
+    ri, th, ph, want = [], [], [], []
+    data = g.data[0::2] + 1j * g.data[1::2]
+    for i in (1, 2, 3, 7, 11, 15):
+        for j in range(3 * i + 1):
+            for k in range(6 * i + 1):
+                ri.append(i)
+                th.append(np.pi * j / (3 * i))
+                ph.append(2 * np.pi * k / (6 * i))
+                want.append(data[1 + 6 * (i - 1) * i * i + j * 6 * i + k % (6 * i)])
+    a = g.interpolate_theta_phi_plane(np.array(ri), np.array(th), np.array(ph))
+    off = np.array(a) != np.array(want)
+    assert not off.any(), (int(off.sum()), len(want))
+
+
 def test_seeded_intensity_matches_oracle(dplus, oracle, small):
     say("[case] seeded CalculateIntensity")
     s = small
