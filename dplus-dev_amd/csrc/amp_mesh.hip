@@ -34,7 +34,7 @@
 // weights 0.07); 200,000 atoms at grid 110, mixed: 14.5 -> 0.9 ms; 5,000 atoms and
 // 22,000 boxes at grid 120, FP64: 20.6 -> 0.9 ms.  Error against direct sums in 64 bits,
 // median over the shells of |dA| / |A| (2-norms, against 80-bit sums; 2,000 to 20,000 atoms, a
-// protein, a cube, a slab, off the origin): mixed 6e-8 .. 1.5e-7 where the direct builder has
+// protein, a cube, a slab, off the origin): mixed 6e-8 .. 1.6e-7 where the direct builder has
 // 1.1e-7 .. 4.3e-7; FP64 1.5e-16 .. 2.6e-15 where the direct one has 2.3e-16 .. 2.5e-15.
 //
 // Everything up to the frequency mesh is FP64.  A mixed grid's nodes are
@@ -125,9 +125,10 @@ void power_fit(int n, F f, long double *c) {
     for (int i = 0; i < n; i++) c[i] = p[i];
 }
 
-const Window &window(int W, double sigma) {
+// single: coefficients for FP32 evaluation, whose transform is that of the rounded ones
+const Window &window(int W, double sigma, bool single) {
     static std::mutex mu;
-    static Window tab[32];  // one oversampling per width
+    static Window tab[32];  // one oversampling and one precision per width
     std::lock_guard<std::mutex> lk(mu);
     Window &k = tab[W];
     if (k.W) return k;
@@ -150,7 +151,10 @@ const Window &window(int W, double sigma) {
         for (int d = 0; d < nc; d++) phi[(size_t)l * nc + d] = fit[d];
     }
     // of unit area: 1 / phihat starts at 1, which no rounding of its constant term scales
-    for (size_t i = 0; i < phi.size(); i++) k.coef[i] = (double)(phi[i] / area);
+    for (size_t i = 0; i < phi.size(); i++) {
+        k.coef[i] = (double)(phi[i] / area);
+        if (single) k.coef[i] = (double)(float)k.coef[i];
+    }
     auto phihat = [&](long double xi) {
         long double s = 0.0L;
         for (int l = 0; l < W; l++)
@@ -975,7 +979,7 @@ void mesh_bands(const MeshPlan &P, const MeshSizes &Z, int N, bool fp64, std::ve
 
 void mesh_tables(const MeshPlan &P, bool fp64, double *tab) {
     const double sigma = fp64 ? kSigma64 : kSigmaMixed;
-    const Window &s = window(fp64 ? kSpread64 : kSpreadMixed, sigma), &i = window(fp64 ? kInterp64 : kInterpMixed, sigma);
+    const Window &s = window(fp64 ? kSpread64 : kSpreadMixed, sigma, false), &i = window(fp64 ? kInterp64 : kInterpMixed, sigma, !fp64);
     std::copy(s.coef.begin(), s.coef.end(), tab + P.t_spread);
     std::copy(s.inv, s.inv + kInvDeg, tab + P.t_sinv);
     std::copy(i.coef.begin(), i.coef.end(), tab + P.t_interp);
