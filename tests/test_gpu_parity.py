@@ -315,6 +315,36 @@ def test_vegas_matches_oracle(dplus, oracle, small, prec):
     assert np.max(np.abs(mine - ref) / ref) < (FP64_TOL if prec == 0 else MIXED_TOL)
 
 
+@pytest.mark.parametrize("prec,gs,layers", [(0, 130, (57, 66)), (1, 190, (81, 96))])
+def test_vegas_tiles_that_fit_some_planes(dplus, oracle, prec, gs, layers):
+    """VEGAS with 98 points a bin over shells whose polar bins' tiles fit LDS on some of a lookup's
+    four planes and not on others (38 KB of nodes), against the oracle on the grid's own nodes."""
+    say(f"[case] VEGAS over tiles at the limit, grid {gs}, precision={prec}")
+    room = 38 * 1024 // (16 if prec else 32)
+    th = np.arccos(1 - 2 / 32) / np.pi  # the first row of bins, four bins wide in phi
+
+    def nodes(i):
+        rows = int(np.floor(th * 3 * i + 1e-6)) + 2 - (int(np.floor(-1e-6)) - 1) + 1
+        cols = int(np.floor(4 / 32 * 6 * i + 1e-6)) + 1 - int(np.floor(-1e-6)) + 1
+        return rows * (cols | 1)
+    mixed = [l for l in range(*layers) if len({nodes(l - 1 + p) <= room for p in range(4)}) == 2]
+    assert mixed
+    qmax = 5.0
+    xyz, ion, coef9, rad = structure(300, 7)
+    g = gpu_grid(dplus, gs, qmax, prec, xyz, ion, coef9, rad)
+    g.download()
+    step = qmax / (gs // 2)
+    q = np.array([(l + 0.37) * step for l in range(*layers) if (l + 0.37) * step <= qmax])
+    assert any(l * step < v <= (l + 1) * step for l in mixed for v in q)
+    dock = oracle.Docked.single(gs, qmax, g.data, g.interp)
+    mine, _ = dplus.orientation_average(dplus.Docking.single(g), q, method=dplus.OA_VEGAS, seed=4,
+                                        vegas_iterations=3, vegas_points_per_bin=98)
+    ref, _ = oracle.vegas_oa(dock, q, 4, 3, 98)
+    e = np.max(np.abs(mine - ref) / ref)
+    say(f"    layers with both kinds of planes {mixed}: vs oracle {e:.2e}")
+    assert e < (FP64_TOL if prec == 0 else MIXED_TOL)
+
+
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("ppb", [2, 8, 98])
 def test_vegas_of_an_isotropic_structure(dplus, oracle, prec, ppb):
@@ -367,6 +397,32 @@ def test_gk_device_recursion_matches_host_replay(dplus, small, prec, monkeypatch
                 f"{np.max(np.abs(a - b)):.2e}")
             assert sa.evaluations == sb.evaluations
             np.testing.assert_array_equal(a, b)
+
+
+def test_gk_level_past_the_first_room_matches_host_replay(dplus, small, monkeypatch):
+    """A phi level of more than 65,536 open intervals: its theta level starts again with all the
+    device room (four allocations more than a call that stays below), and the intensities and
+    evaluation counts are the host replay's."""
+    say("[case] GK levels past 65,536 intervals")
+    s = small
+    g = gpu_grid(dplus, s["gs"], s["qmax"], 0, s["xyz"], s["ion"], s["coef9"], s["rad"])
+    dock = dplus.Docking.single(g)
+    monkeypatch.delenv("DPLUS_GK_HOST", raising=False)
+
+    def run(nq, eps):
+        q = np.linspace(0.05, 4.5, nq)
+        a0 = dplus.device_info()["device_allocations"]
+        I, st = dplus.orientation_average(dock, q, method=dplus.OA_GK, eps=eps, gk_max_depth=12)
+        return I, st.evaluations, dplus.device_info()["device_allocations"] - a0
+    _, _, base = run(20, 1e-3)
+    a, ea, more = run(600, 1e-6)
+    say(f"    {ea} evaluations, allocations {base} and {more}")
+    assert more == base + 4
+    monkeypatch.setenv("DPLUS_GK_HOST", "1")
+    b, eb, _ = run(600, 1e-6)
+    monkeypatch.delenv("DPLUS_GK_HOST")
+    assert ea == eb
+    np.testing.assert_array_equal(a, b)
 
 
 @pytest.mark.parametrize("prec", [0, 1])

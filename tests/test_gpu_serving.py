@@ -99,6 +99,25 @@ def test_engine_mc_of_five_chunks_with_chi2_matches_oracle(dplus, oracle, prec):
         e.close()
 
 
+def test_engine_graphs_across_chunk_counts(dplus):
+    """One slot's kept graph over single-leaf Monte Carlo requests of one to seventeen chunks, whose
+    kernels differ: every replay gives the eager request's bits."""
+    from dplus_mi355x.serving import Engine
+    say("[case] engine: captured requests across chunk counts")
+    pdb = make_pdb(300, 6, 1.2)
+    q = np.linspace(0.05, 4.0, 40)
+    counts = [1, 5, 12, 4, 2, 17, 5, 3, 9, 12, 1, 6]
+    out = {}
+    for graphs in (False, True):
+        e = Engine(streams=1, graphs=graphs)
+        out[graphs] = [e.wait(e.submit(q, pdb=pdb, grid_size=20, qmax=4.0, precision=dplus.PRECISION_MIXED, seed=3,
+                                       method=dplus.OA_MC, max_dirs=n * 1024, chunk=1024)) for n in counts]
+        e.close()
+    for n, (Ie, re), (Ig, rg) in zip(counts, out[False], out[True]):
+        assert rg["graph"] == 1 and not re["graph"] and rg["dirs_used"] == re["dirs_used"] == n * 1024
+        assert np.array_equal(Ie, Ig), n
+
+
 def test_engine_graph_requests_match_eager(dplus):
     from dplus_mi355x.serving import Engine
     say("[case] engine: 10 requests eager vs captured graphs (1 stream twice, then 4 streams)")
