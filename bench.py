@@ -29,6 +29,11 @@ sys.path.insert(0, os.path.join(ROOT, "oracle"))
 
 METRIC = "I(q) curves/s + p50/p99 latency, mixed vs FP64 GPU at ≤1e-4 rel err"
 PEAK_HBM_GBPS = 8000.0  # MI355X HBM3E
+# vector instructions (64 lanes each) that this workload's kernels issue, counted by rocprofv3
+# (profiles/cases_counters.md): one build through the frequency mesh, one VEGAS iteration;
+# the card issues one every four clocks on each of 1,024 SIMDs
+VALU_PER_BUILD, VALU_PER_VEGAS_ITERATION = 265.2e6, 223.3e6
+PEAK_VALU = 1024 * 2.4e9 / 4
 
 
 def log(*a):
@@ -521,6 +526,8 @@ def main():
     w_t = 2.0 * mb["fma32"] / mb["sin32"]  # flop-equivalents of one v_sin/v_cos
     log(f"[bench] VALU microbenchmark ops/s: {mb}; transcendental weight {w_t:.2f} flop-eq")
 
+    assert st.build_route(g32) == "mesh"
+
     # ---- mixed precision: warmup, then timed steps
     for i in range(args.warmup):
         curve(D, st, g32, W, seed=100 + i)
@@ -583,23 +590,29 @@ def main():
     log(f"[bench] GK (tol 1e-4): mixed {gk['mixed'][1]:.3f} s, fp64 {gk['fp64'][1]:.3f} s per average "
         f"({gk['mixed'][2]} integrand evaluations); max rel I(q) mixed vs fp64 = {gk_err:.2e}")
 
-    # ---- the VEGAS kernels against the gather ceiling of the same lookups on the same grid
+    # ---- the VEGAS kernels against vector issue, and their lookups beside the gather ceiling of the
+    # same lookups read from memory
     ngroups = len(np.unique(np.maximum(np.ceil(W["q"] / g32.step_size) - 1, 0)))
     v_lookups = float(W["iters"]) * 1024 * W["ppb"] * ngroups
     v_rate = v_lookups * 512 / (ms_vegas / max(args.steps, 1) * 1e-3)
     p_ms, p_lk = D.gather_probe(g32, 1 << 18, 0, ngroups)
     ceiling = p_lk * 512 / (p_ms * 1e-3)
+    v_issue = VALU_PER_VEGAS_ITERATION * W["iters"] / (ms_vegas / max(args.steps, 1) * 1e-3)
     oa_roof = {"bound": "valu", "kernel": "vegas_sample<float, float4, true> + vegas_reduce",
-               "achieved": v_rate / 1e9, "peak": ceiling / 1e9, "unit": "GB/s of nodes", "frac": v_rate / ceiling,
-               "lookups_per_curve": v_lookups, "bytes_per_lookup": 512,
-               "ceiling": "dplus_gather_probe: the same lookups' node loads alone, each from memory, at full "
-                          "occupancy; the kernel reads them from LDS tiles, so the fraction may exceed 1"}
-    log(f"[bench] VEGAS lookups {v_rate / 1e12:.2f} TB/s of nodes, gather ceiling {ceiling / 1e12:.2f} TB/s "
-        f"({v_rate / ceiling:.2f})")
+               "achieved": v_issue / 1e9, "peak": PEAK_VALU / 1e9, "unit": "G vector instructions/s",
+               "frac": v_issue / PEAK_VALU, "instructions_per_iteration": VALU_PER_VEGAS_ITERATION,
+               "lookups_per_curve": v_lookups, "bytes_per_lookup": 512, "node_GBps": v_rate / 1e9,
+               "gather_ceiling_GBps": ceiling / 1e9,
+               "gather_ceiling": "dplus_gather_probe: the same lookups' node loads alone, each from memory, at full "
+                                 "occupancy; the kernel reads them from LDS tiles"}
+    log(f"[bench] VEGAS {oa_roof['frac']:.2f} of vector issue; lookups {v_rate / 1e12:.2f} TB/s of nodes beside "
+        f"{ceiling / 1e12:.2f} TB/s from memory")
 
-    # ---- the amplitude builder against HBM: the bytes it cannot do without (the sources read,
-    # every node's amplitude written) over its launch time; and the direct sum's unit,
-    # 8 flops + 2 transcendentals per (node, source) term, that the frequency mesh replaces
+    # ---- the amplitude builder against vector issue, the largest of its bounds: its counted
+    # instructions over its launch time (the fullest brick's chain of batches keeps the spread off
+    # it).  Beside it the bytes it cannot do without (the sources read, every node's amplitude
+    # written) against HBM, and the direct sum's unit, 8 flops + 2 transcendentals per
+    # (node, source) term, that the frequency mesh replaces
     sources = len(W["xyz"]) + len(W["dims"])
     nodes = float(O_total_points(W["gs"]))
     t_launch = ms_build / max(nb, 1) * 1e-3
@@ -651,10 +664,13 @@ def main():
             "max_rel_err_vs_fp64": err_plain},
         "speedup_vs_fp64_plain": None if not lat64p else value * float(np.mean(lat64p)),
         "gauss_kronrod": gk_out,
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBPS, "unit": "GB/s",
-                     "frac": achieved / PEAK_HBM_GBPS, "traffic": traffic,
-                     "traffic_from": "algorithmic: sources read once, every node's amplitude written once",
-                     "kernel": "mesh_spread + mesh_dft + mesh_interp", "launch_ms": t_launch * 1e3,
+        "roofline": {"bound": "valu", "achieved": VALU_PER_BUILD / t_launch / 1e9, "peak": PEAK_VALU / 1e9,
+                     "unit": "G vector instructions/s", "frac": VALU_PER_BUILD / t_launch / PEAK_VALU,
+                     "instructions": VALU_PER_BUILD, "instructions_from": "rocprofv3 SQ_INSTS_VALU of this build",
+                     "hbm": {"achieved_GBps": achieved, "peak_GBps": PEAK_HBM_GBPS, "frac": achieved / PEAK_HBM_GBPS,
+                             "traffic": traffic,
+                             "traffic_from": "algorithmic: sources read once, every node's amplitude written once"},
+                     "kernel": "mesh_weights + mesh_spread + mesh_dft + mesh_interp", "launch_ms": t_launch * 1e3,
                      "terms_per_launch": nodes * sources,
                      "direct_sum_unit_achieved": nodes * sources * (8.0 + 2.0 * w_t) / t_launch / 1e12},
         "oa_roofline": oa_roof,

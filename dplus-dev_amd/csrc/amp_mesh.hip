@@ -30,9 +30,9 @@
 // transform prod_a L_a sinc(q_a L_a / 2) to the window's accuracy.
 //
 // Measured (MI355X, GPU time of a build): 50,000 atoms and 136,000 boxes at grid 250,
-// mixed: 113.2 ms direct -> 1.36 ms (spread 0.59, interpolation 0.38, transforms 0.14,
-// weights 0.07); 200,000 atoms at grid 110, mixed: 14.5 -> 0.9 ms; 5,000 atoms and
-// 22,000 boxes at grid 120, FP64: 20.6 -> 0.9 ms.  Error against direct sums in 64 bits,
+// mixed: 119.7 ms direct -> 1.23 ms (spread 0.62, interpolation 0.34, transforms 0.19,
+// weights 0.07); 200,000 atoms at grid 110, mixed: 13.9 -> 0.78 ms; 5,000 atoms and
+// 22,000 boxes at grid 120, FP64: 19.5 -> 0.81 ms.  Error against direct sums in 64 bits,
 // median over the shells of |dA| / |A| (2-norms, against 80-bit sums; 2,000 to 20,000 atoms, a
 // protein, a cube, a slab, off the origin): mixed 6e-8 .. 1.6e-7 where the direct builder has
 // 1.1e-7 .. 4.3e-7; FP64 1.5e-16 .. 2.6e-15 where the direct one has 2.3e-16 .. 2.5e-15.

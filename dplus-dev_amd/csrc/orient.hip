@@ -362,8 +362,8 @@ constexpr int kMaxM = 16;  // q-values of one shell group handled per pass (one 
 // accumulate the docked amplitude along unit direction qv for q-values qs[0..m), m <= M,
 // (900 copies of two leaves in 120 rotations, 8,192 directions, grid 150: 6.58 -> 5.23 ms with
 // polynomial angles, interpolation weights and the phase sums taken before the amplitudes,
-// which also shortens their rounding: 4.0e-6 -> 7e-7 of I(q); 2,190 VALU instructions a
-// lookup before, at 2 waves per SIMD beside the gathers)
+// which also shortens their rounding: 4.0e-6 -> 7e-7 of I(q); 2,190 -> 1,850 VALU instructions
+// a lookup, issued 0.71 of the clocks at 2 waves per SIMD beside the gathers)
 // whose weights over the four planes are wq (q_weights, in LDS).
 // stepq (equally spaced q, single precision): the translations of a rotation
 // with several step their phases in q, e^{i q_j d} = e^{i q_0 d} (e^{i dq d})^j:
@@ -746,8 +746,9 @@ constexpr int tile_nodes() {
 // the lookups through per-q weights.  The same directions as mc_kernel; the sums over
 // them are grouped by patch instead of by run of 256.  2,000 atoms, grid 100, 10^6
 // directions, 500 q: 1.93 -> 0.94 ms (FP64, 262,144: 0.91 -> 0.45).  mc_kernel waits on 32
-// divergent loads a lookup; here the VALU is full (about 720 instructions per 64
-// directions and group, 150 of them the draw), so fewer instructions are what is left.
+// divergent loads a lookup; here the VALU issues all the time (732 instructions counted per
+// 64 directions and group, LDS reads 0.60 of the clocks), so fewer instructions are what is
+// left.
 template <typename T, typename T4, int D>
 __global__ __launch_bounds__(256) void mc_patch_kernel(const T4 *const *__restrict__ grids,
                                                        const RotDev *__restrict__ rots,
@@ -1111,12 +1112,11 @@ __device__ __forceinline__ float wave_sums(const float (&v)[M], int lane, int o 
 // wave-uniform) into LDS, then a thread per copy takes two collapsed nodes per plane, the q
 // weights and its translation's phases.  Both halves run without a chain from one chunk to
 // the next.  Two barriers a direction; three workgroups per CU cover them.
-// 1,000 copies, grid 200, 800 q, 65,536 directions: 158.9 -> 79.5 ms, the VALU full (about
-// 460 instructions per 64 copies: 110 for the planes, 210 for eight q and their phases, 70
-// for the rows).
+// 1,000 copies, grid 200, 800 q, 65,536 directions: 158.9 -> 78.3 ms; VALU issue 0.86 of the
+// clocks at three waves per SIMD, 381 instructions counted per 64 copies.
 // Taken where the rows fit (kRowNodes) and copies >= 2.5 shells: the rows cost 4 * 6 shell
-// / 64 collapses of 35 instructions, a chunk of 64 copies 340 here and 684 there, equal
-// near 2.4 copies per shell.
+// / 64 collapses of 35 instructions (42 of the 381 here), a chunk of 64 copies 340 beside
+// them and 684 there, equal near 2.4 copies per shell.
 template <int M>
 __global__ __launch_bounds__(256, M <= 8 ? 3 : 2) void mc_zrows_kernel(
     const float4 *const *__restrict__ grids, const ZCopyDev *__restrict__ zc, int nz,
