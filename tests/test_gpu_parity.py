@@ -377,7 +377,7 @@ def test_gk_matches_oracle(dplus, oracle, small):
 @pytest.mark.parametrize("prec", [0, 1])
 def test_gk_device_recursion_matches_host_replay(dplus, small, prec, monkeypatch):
     """The Gauss-Kronrod phi recursion grown on the device (accept / split and the
-    left + right tree sums in gk_decide) against the host replay of the same
+    left + right tree sums in docked_gk_level) against the host replay of the same
     recursion: identical intensities and evaluation counts, on a single grid and
     on a docked 12-copy helix, with depth limits and a q = 0 entry."""
     say(f"[case] GK device recursion vs host replay precision={prec}")
