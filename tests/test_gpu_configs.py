@@ -204,6 +204,32 @@ def test_fp64_mesh_is_as_precise_as_direct_sums(dplus, n, gs, qmax, half, shift,
     assert med["mesh"] <= 1.25 * med["direct"]
 
 
+def test_one_large_box_stays_whole(dplus, oracle, monkeypatch):
+    """A box that would make a million pieces beside 500 atoms: the structure keeps it whole and its
+    grids are direct sums whatever the route asked for; a box of a tenth of its edge goes through the
+    mesh.  FP64 nodes against the oracle, and the mesh's mixed ones (the direct builder's mixed sinc
+    of 45 rad has FP32's error of that angle, which the mesh's bound does not cover)."""
+    import dplus_mi355x.synth as S
+    rng = np.random.default_rng(5)
+    xyz, el = rng.uniform(-1, 1, (500, 3)), np.array(["C", "N", "O", "S"])[rng.integers(0, 4, 500)]
+    coef9, rad, ion, _ = S.structure_tables(el)
+    monkeypatch.setenv("DPLUS_BUILD_ROUTE", "mesh")
+    gs, qmax = 24, 3.0
+    idx, shell_of, qv = sample_nodes(oracle, gs, qmax)
+    atoms = oracle.amp_atoms(xyz, ion, oracle_ions(oracle, coef9, rad, ion), qv)
+    for edge, route in ((300, "direct"), (30, "mesh")):
+        dims, com = np.array([[edge] * 3], np.int32), np.array([[0.1, -0.2, 0.3]])
+        st = dplus.Structure(xyz, ion, coef9, rad, sol_ed=333.0, flags=3, box_dims=dims, box_com=com, vox_step=0.1,
+                             box_contrast=33.3)
+        ref = atoms + oracle.amp_boxes(dims, com, 0.1, 33.3, qv)
+        for prec, tol in ((0, 1e-12), (1, 1e-5)):
+            g = dplus.Grid(gs, qmax, prec)
+            assert st.build_route(g) == route
+            st.build(g, host_copy=True)
+            if prec == 0 or route == "mesh":
+                assert node_errors(grid_values(g, idx), ref, shell_of) < tol
+
+
 ARENA_BUILD = r"""
 #include "device.hpp"
 using namespace dplus;
