@@ -10,8 +10,8 @@ average by VEGAS (10 iterations x 1024 bins x 98 points).
 
 One step = one I(q) curve: amplitude grid of the resident atoms and boxes,
 spline coefficients, VEGAS average, I(q) back on the host.  The mixed-precision
-path is timed for --steps steps; the FP64 path (FP64 phases, sincos,
-accumulation, with the mixed builder's algebra) runs the same requests one at a
+path is timed for --steps steps; the FP64 path (the same algebra with FP64
+grids, lookups and accumulation) runs the same requests one at a
 time for comparison, and the maximum relative I(q) difference between the two is
 reported; the plain FP64 builder (one node at a time) is timed beside it.
 """
@@ -549,8 +549,8 @@ def main():
     log(f"[bench] mixed: {args.steps} curves in {elapsed:.3f} s; build {ms_build / max(nb, 1):.2f} ms/launch, "
         f"splines {ms_spl / max(ns, 1):.2f} ms, vegas {ms_vegas / max(args.steps, 1):.2f} ms/curve")
 
-    # ---- FP64 path on the same request: the paired builder's algebra in double
-    # (like for like), then the plain FP64 builder (one node at a time)
+    # ---- FP64 path on the same request: the same algebra in double (like for like: the
+    # frequency mesh), then the plain FP64 builder (one node at a time)
     lat64 = []
     for i in range(args.fp64_steps):
         t0 = time.perf_counter()
@@ -569,7 +569,7 @@ def main():
         D.set_fp64_builder(False)
     err_plain = float(np.max(np.abs(I64p - I64) / np.abs(I64))) if lat64p else None
     if lat64p:
-        log(f"[bench] fp64 plain builder: {np.mean(lat64p):.3f} s/curve; vs paired FP64 {err_plain:.2e}")
+        log(f"[bench] fp64 plain builder: {np.mean(lat64p):.3f} s/curve; vs FP64 {err_plain:.2e}")
 
     # ---- the same grids averaged by adaptive Gauss-Kronrod (relative tolerance 1e-4, depth 8)
     # (one untimed average first: the first one grows the device memory pool by the GK arenas)
